@@ -57,7 +57,7 @@ STEP_KERNELS = {"ntt_fwd": ("k_ntt_A", "k_ntt_B"), "ntt_inv": ("k_ntt_B", "k_ntt
                 "add": ("k_add",), "perm": ("k_perm",), "copy": ("k_copy",),
                 "rsv": ("k_rs",), "ptacc": ("k_ptacc",), "ntt_fwd_a": ("k_ntt_A",), "ksi": ("k_ksi",),
                 "ntt_inv_b": ("k_ntt_B",), "modup": ("k_modup",), "moddown": ("k_modup",),
-                "ntt_fwd_b": ("k_ntt_B",), "tensor_ib": ("k_tensor_ib",)}
+                "ntt_fwd_b": ("k_ntt_B",), "tensor_ib": ("k_tensor_ib",), "ksdown": ("k_modup",)}
 
 
 def kernel_bytes(name, kind, nkern, total, epilogue):

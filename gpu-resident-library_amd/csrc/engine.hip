@@ -233,6 +233,12 @@ Ctx::Ctx(uint32_t n_, const std::vector<uint64_t>& q, const std::vector<uint64_t
         put(tab, &c.d_tabMD);
         put(tq, &c.d_tqMD);
         put(tqn, &c.d_tqnegMD);
+        // the same times -P^-1: the fused ModDown of a keyswitch
+        std::vector<uint64_t> tabKS((size_t)K * l);
+        for (uint32_t i = 0; i < l; ++i)
+            for (uint32_t k = 0; k < K; ++k)
+                tabKS[(size_t)k * l + i] = host_mulmod(tab[(size_t)k * l + i], mods[i] - c.pinv[i], mods[i]);
+        put(tabKS, &c.d_tabKS);
         // rescale dropping tower l-1: s1 = q_{l-1}^-1 mod q_i, s2 = -s1 mod q_i
         // (s2 = floor(Q' [Q'^-1]_{q_l} / q_l) mod q_i is congruent to -s1, src/params.cpp:50-75)
         if (l >= 2) {
@@ -262,27 +268,26 @@ Ctx::Ctx(uint32_t n_, const std::vector<uint64_t>& q, const std::vector<uint64_t
             put(tabRS, &c.d_tabRS);
             put(tg, (const uint64_t**)&c.d_rstg);
             put(rsw, &c.d_rs_sw);
-            // the surviving towers as the fused ModDown's targets
-            std::vector<uint64_t> rq(l - 1), rqn(l - 1), rtw(l - 1), rred(l - 1), rtwd(l - 1), rqf(2 * (size_t)(l - 1));
-            for (uint32_t i = 0; i + 1 < l; ++i) {
-                rq[i] = mods[i];
-                rqn[i] = host_qneg(mods[i]);
-                rtw[i] = (uint64_t)(uintptr_t)rt[i].fw2;
-                rred[i] = lazy_red_of(mods[i]);
-                rtwd[i] = (uint64_t)(uintptr_t)rt[i].fw2d;
-                const double qd = (double)mods[i], qi = 1.0 / qd;
-                std::memcpy(&rqf[2 * i], &qd, 8);
-                std::memcpy(&rqf[2 * i + 1], &qi, 8);
-            }
-            put(rq, &c.d_rs_tq);
-            put(rqn, &c.d_rs_tqneg);
-            put(rtw, &c.d_rs_ttw);
-            put(rred, &c.d_rs_tred);
-            put(rtwd, &c.d_rs_ttwd);
-            put(rqf, &c.d_rs_tqf);
         }
     }
     put(std::vector<uint64_t>(L + K, 0), &d_zeros);
+    std::vector<uint64_t> mq(L), mqn(L), mtw(L), mred(L), mtwd(L), mqf(2 * (size_t)L);
+    for (uint32_t i = 0; i < L; ++i) {
+        mq[i] = mods[i];
+        mqn[i] = host_qneg(mods[i]);
+        mtw[i] = (uint64_t)(uintptr_t)rt[i].fw2;
+        mred[i] = lazy_red_of(mods[i]);
+        mtwd[i] = (uint64_t)(uintptr_t)rt[i].fw2d;
+        const double qd = (double)mods[i], qi = 1.0 / qd;
+        std::memcpy(&mqf[2 * i], &qd, 8);
+        std::memcpy(&mqf[2 * i + 1], &qi, 8);
+    }
+    put(mq, &d_md_tq);
+    put(mqn, &d_md_tqneg);
+    put(mtw, &d_md_ttw);
+    put(mred, &d_md_tred);
+    put(mtwd, &d_md_ttwd);
+    put(mqf, &d_md_tqf);
     consts.alloc(blob.size() * 8);
     hip_check(hipMemcpy(consts.p, blob.data(), blob.size() * 8, hipMemcpyHostToDevice), "upload constants");
     for (auto& f : fix) *f.dst = consts.as<uint64_t>() + f.off;
@@ -912,6 +917,7 @@ void Plan::run_jobs(size_t i, hipStream_t s, uint32_t which, uint32_t first, uin
         case Step::NTT_IB: launch_ntt(GF_J(NttJob), cnt, geom, false, s, 1); break;
         case Step::MODUP: launch_modup(GF_J(ModupJob), cnt, geom, st.arg, s); break;
         case Step::MODDOWN: launch_moddown(GF_J(ModupJob), cnt, geom, st.arg, s); break;
+        case Step::KSDOWN: launch_modup(GF_J(ModupJob), cnt, geom, st.arg, s); break;
         case Step::NTT_FB: launch_ntt(GF_J(NttJob), cnt, geom, true, s, 2); break;
     }
 #undef GF_J
@@ -973,10 +979,10 @@ void PlanBuilder::keyswitch_core(uint32_t l, const uint64_t* d, const DevKey& ke
         ksi_moddown_src(l, d, key, ws, lazy_rows, p_rowpass);
         return;
     }
-    if (p_rowpass) throw std::runtime_error("gpufhe: the fused ModDown needs the fused inner product");
     modup(l, d, ws, extra0, extra1, dx0, dx1);
     const uint64_t* dig = ws + WsLayout::make(C).dig * C.n;
-    inner_moddown_src(l, key, ws, [&](uint32_t pi, uint32_t i) { return digit_tower(l, d, dig, pi, i); });
+    inner_moddown_src(
+        l, key, ws, [&](uint32_t pi, uint32_t i) { return digit_tower(l, d, dig, pi, i); }, 0, p_rowpass);
 }
 
 bool PlanBuilder::use_ksi(uint32_t l) const {
@@ -990,6 +996,11 @@ bool PlanBuilder::use_modup(uint32_t l) const {
 // P towers
 bool PlanBuilder::use_moddown(uint32_t l) const {
     return C_.moddown_fused && use_modup(l) && C_.K <= MODUP_MAXSRC && l >= 2;
+}
+// the fused ModDown of a keyswitch: the same kernel without the dropped tower
+bool PlanBuilder::use_ks_moddown() const {
+    return C_.fused && C_.moddown_fused && !C_.geom.single && !C_.wide && C_.K <= MODUP_MAXSRC &&
+           C_.n % MODUP_TILE == 0;
 }
 
 // 3b-5. The digits' row pass fused with the inner product over Q_l P
@@ -1139,7 +1150,8 @@ const uint64_t* PlanBuilder::digit_tower(uint32_t l, const uint64_t* d, const ui
 // into the workspace accumulators, 5. their P towers to coefficient form
 // (ModDown's sources).  digit(pi, i) names the digit towers.
 template <class F>
-void PlanBuilder::inner_moddown_src(uint32_t l, const DevKey& key, uint64_t* ws, F digit, uint64_t gk) {
+void PlanBuilder::inner_moddown_src(uint32_t l, const DevKey& key, uint64_t* ws, F digit, uint64_t gk,
+                                    bool p_rowpass) {
     const Ctx& C = C_;
     const uint32_t n = C.n, K = C.K, W = l + K;
     const LevelConst& lv = C.lv[l];
@@ -1170,15 +1182,19 @@ void PlanBuilder::inner_moddown_src(uint32_t l, const DevKey& key, uint64_t* ws,
     for (int c = 0; c < 2; ++c)
         for (uint32_t k = 0; k < K; ++k) {
             const uint32_t r = C.row_p(k);
-            intt_p_.push_back(NttJob{res[c] + (size_t)(l + k) * n, xp + (size_t)(c * K + k) * n, C.rt[r].iv2,
-                                     nullptr, C.mods[r], lv.pd_post[k], lv.pd_postp[k]});
+            (p_rowpass ? intt_pb_ : intt_p_)
+                .push_back(NttJob{res[c] + (size_t)(l + k) * n, xp + (size_t)(c * K + k) * n, C.rt[r].iv2, nullptr,
+                                  C.mods[r], lv.pd_post[k], lv.pd_postp[k]});
         }
 }
 
 void PlanBuilder::keyswitch(uint32_t l, const uint64_t* d, uint64_t* ba0, uint64_t* ba1,
                             const DevKey& key, uint64_t* ws, const uint64_t* t0,
                             const uint64_t* t1) {
-    keyswitch_core(l, d, key, ws, nullptr, nullptr, nullptr, nullptr);
+    // with the fused ModDown the accumulators' Q rows only feed its
+    // epilogue's lazy Shoup products
+    const bool fmd = use_ks_moddown();
+    keyswitch_core(l, d, key, ws, nullptr, nullptr, nullptr, nullptr, fmd ? l : 0, fmd);
     moddown_tail(l, ws, ba0, ba1, t0, t1);
 }
 
@@ -1188,26 +1204,81 @@ void PlanBuilder::moddown_tail(uint32_t l, uint64_t* ws, uint64_t* ba0, uint64_t
                                const uint64_t* t1) {
     const Ctx& C = C_;
     const uint32_t n = C.n, K = C.K;
-    const LevelConst& lv = C.lv[l];
     const WsLayout w = WsLayout::make(C);
     uint64_t* res[2] = {ws + w.res0 * n, ws + w.res1 * n};
     uint64_t* xp = ws + w.xp * n;
     uint64_t* conv = ws + w.x * n;  // the part towers are dead once ModUp has converted them
-    // 6-8. ApproxModDown of both accumulators, fused with r = t + ba (:203-224)
     uint64_t* outs[2] = {ba0, ba1};
     const uint64_t* ts[2] = {t0, t1};
-    for (int c = 0; c < 2; ++c) {
-        uint64_t* cv = conv + (size_t)c * l * n;
-        for (uint32_t j0 = 0; j0 < l; j0 += C.conv_chunk)
-            conv_dn_.push_back(ConvJob{xp + (size_t)c * K * n, cv, lv.d_tabMD, lv.d_tqMD, lv.d_tqnegMD, K, l,
-                                       j0, j0 + C.conv_chunk < l ? j0 + C.conv_chunk : l, C.wide});
-        for (uint32_t i = 0; i < l; ++i) {
-            ntt_conv_.push_back(NttJob{cv + (size_t)i * n, cv + (size_t)i * n, C.rt[i].fw2, nullptr,
-                                       C.mods[i], 0, 0});
-            combine_.push_back(CombineJob{res[c] + (size_t)i * n, cv + (size_t)i * n,
-                                          ts[c] ? ts[c] + (size_t)i * n : nullptr, outs[c] + (size_t)i * n,
-                                          C.mods[i], lv.pinv[i], lv.pinvp[i]});
+    const bool fmd = use_ks_moddown();
+    for (int c = 0; c < 2; ++c)
+        ks_tail(ModdownSrc{l, (uint32_t)c, xp + (size_t)c * K * n, nullptr, nullptr, ts[c], res[c],
+                           conv + (size_t)c * l * n, outs[c], true},
+                fmd);
+}
+
+void PlanBuilder::moddown_sources(ModupJob& J, const LevelConst& lv, const uint64_t* xp) const {
+    const Ctx& C = C_;
+    for (uint32_t k = 0; k < C.K; ++k) {
+        const uint32_t r = C.row_p(k);
+        J.src[k] = xp + (size_t)k * C.n;
+        J.stw[k] = C.rt[r].iv2;
+        J.sq[k] = C.mods[r];
+        J.post[k] = lv.pd_post[k];
+        J.postp[k] = lv.pd_postp[k];
+        if (C.modup_f64 && C.rt[r].iv2d) {
+            J.stwd[k] = C.rt[r].iv2d;
+            J.sqd[k] = (double)C.mods[r];
+            J.sqinv[k] = 1.0 / J.sqd[k];
+            f64_twiddle(lv.pd_post[k], C.mods[r], J.spost[k], J.spostq[k]);
         }
+    }
+    J.sp = C.K;
+    J.tq = C.d_md_tq;
+    J.tqneg = C.d_md_tqneg;
+    J.ttw = C.d_md_ttw;
+    J.tred = C.d_md_tred;
+    J.ttwd = C.modup_f64 ? C.d_md_ttwd : C.d_zeros;
+    J.tqf = C.d_md_tqf;
+}
+
+// The ModDown of one component of a keyswitch with out = t + ba:
+//   out_i = t_i + (res_i - NTT_i(conv_i)) P^-1 = NTT_i(-P^-1 conv_i) + res_i P^-1 + t_i
+// by linearity, so the fused form converts with -P^-1 folded into the
+// constants, leaves each tower's column pass in out, and its row pass adds
+// the other two terms as it stores: the conversion's towers and the combine's
+// operands do not travel through HBM a second time.
+void PlanBuilder::ks_tail(const ModdownSrc& m, bool fused) {
+    const Ctx& C = C_;
+    const uint32_t n = C.n, l = m.l;
+    const LevelConst& lv = C.lv[l];
+    if (fused) {
+        ModupJob J{};
+        moddown_sources(J, lv, m.xp);
+        J.dst = m.out;
+        J.tab = lv.d_tabKS;
+        J.sc = l;
+        ksdown_.push_back(J);
+        ksdown_src_.push_back(m);
+        for (uint32_t i = 0; i < l; ++i) {
+            NttJob T{m.out + (size_t)i * n, m.out + (size_t)i * n, C.rt[i].fw2, nullptr, C.mods[i], 0, 0};
+            T.e0 = m.res + (size_t)i * n;
+            T.c0 = lv.pinv[i];
+            T.c0p = lv.pinvp[i];
+            T.e1 = m.t ? m.t + (size_t)i * n : nullptr;
+            T.e1_plain = 1;
+            ntt_vb_.push_back(T);
+        }
+        return;
+    }
+    for (uint32_t j0 = 0; j0 < l; j0 += C.conv_chunk)
+        conv_dn_.push_back(ConvJob{m.xp, m.vc, lv.d_tabMD, lv.d_tqMD, lv.d_tqnegMD, C.K, l, j0,
+                                   j0 + C.conv_chunk < l ? j0 + C.conv_chunk : l, C.wide});
+    for (uint32_t i = 0; i < l; ++i) {
+        uint64_t* cv = m.vc + (size_t)i * n;
+        ntt_conv_.push_back(NttJob{cv, cv, C.rt[i].fw2, nullptr, C.mods[i], 0, 0});
+        combine_.push_back(CombineJob{m.res + (size_t)i * n, cv, m.t ? m.t + (size_t)i * n : nullptr,
+                                      m.out + (size_t)i * n, C.mods[i], lv.pinv[i], lv.pinvp[i]});
     }
 }
 
@@ -1256,29 +1327,9 @@ void PlanBuilder::rescale_tail(const ModdownSrc& m, bool fused) {
     const LevelConst& lv = C.lv[l];
     if (fused) {
         ModupJob J{};
-        for (uint32_t k = 0; k < K; ++k) {
-            const uint32_t r = C.row_p(k);
-            J.src[k] = m.xp + (size_t)k * n;
-            J.stw[k] = C.rt[r].iv2;
-            J.sq[k] = C.mods[r];
-            J.post[k] = lv.pd_post[k];
-            J.postp[k] = lv.pd_postp[k];
-            if (C.modup_f64 && C.rt[r].iv2d) {
-                J.stwd[k] = C.rt[r].iv2d;
-                J.sqd[k] = (double)C.mods[r];
-                J.sqinv[k] = 1.0 / J.sqd[k];
-                f64_twiddle(lv.pd_post[k], C.mods[r], J.spost[k], J.spostq[k]);
-            }
-        }
+        moddown_sources(J, lv, m.xp);
         J.dst = m.out;   // surviving tower i's column-pass output at out + i n
         J.tab = lv.d_tabRS;
-        J.tq = lv.d_rs_tq;
-        J.tqneg = lv.d_rs_tqneg;
-        J.ttw = lv.d_rs_ttw;
-        J.tred = lv.d_rs_tred;
-        J.ttwd = C.modup_f64 ? lv.d_rs_ttwd : C.d_zeros;
-        J.tqf = lv.d_rs_tqf;
-        J.sp = K;
         J.sc = last;
         J.dt = m.dt;
         J.dr = m.dr;
@@ -1439,7 +1490,8 @@ void PlanBuilder::rotate_hoisted(uint32_t l, uint32_t m, const uint64_t* ks, con
         for (uint32_t i = 0; i < l; ++i) perm_.push_back(PermJob{c0 + (size_t)i * n, a0 + (size_t)i * n, ks[j]});
         // the inner product reads the shared digits through sigma_k: no permuted copies
         inner_moddown_src(
-            l, *keys[j], ws, [&](uint32_t pi, uint32_t i) { return digit_tower(l, c1, dig, pi, i); }, ks[j]);
+            l, *keys[j], ws, [&](uint32_t pi, uint32_t i) { return digit_tower(l, c1, dig, pi, i); }, ks[j],
+            use_ks_moddown());
         moddown_tail(l, ws, o0[j], o1[j], a0, nullptr);
     }
 }
@@ -1473,7 +1525,7 @@ void PlanBuilder::linear_transform(uint32_t l, uint32_t m, const uint64_t* ks, c
             continue;
         }
         uint64_t* ws = ws_rot[j];
-        r0.push_back(ws + w.t0 * n);   // sigma(c0) + ba0 overwrites sigma(c0) element by element
+        r0.push_back(ws + w.dig * n);   // not over sigma(c0) (t0), which the ModDown's last stage adds
         r1.push_back(ws + w.t1 * n);
         rk.push_back(ks[j]);
         rkey.push_back(keys[j]);
@@ -1586,9 +1638,10 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         modup_.clear();
         modup_src_.clear();
     }
-    // likewise a fused ModDown stage: the P towers' whole inverse transforms,
-    // the prologue, the epilogue transforms whole
-    if (!moddown_.empty() && moddown_.size() * (C_.n / MODUP_TILE) < C_.modup_min_wgs) {
+    // likewise the fused ModDown stages: the P towers' whole inverse transforms,
+    // the prologue or conversion, the epilogue transforms (and combines) apart,
+    // over accumulators reduced by the inner product
+    if (moddown_.size() + ksdown_.size() && (moddown_.size() + ksdown_.size()) * (C_.n / MODUP_TILE) < C_.modup_min_wgs) {
         for (NttJob& j : intt_pb_) intt_p_.push_back(j);
         intt_pb_.clear();
         ntt_vb_.clear();
@@ -1596,6 +1649,13 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         std::vector<ModdownSrc> ms;
         ms.swap(moddown_src_);
         for (const ModdownSrc& m : ms) rescale_tail(m, false);
+        if (!ksdown_.empty()) {
+            ksdown_.clear();
+            ms.clear();
+            ms.swap(ksdown_src_);
+            for (const ModdownSrc& m : ms) ks_tail(m, false);
+            for (KsiJob& j : ksi_) j.lazy_out = 0;
+        }
     }
     for (auto* v : {&intt_up_, &intt_upb_, &ntt_dig_, &ntt_diga_, &intt_p_, &intt_pb_, &ntt_conv_, &intt_drop_,
                     &ntt_sw_, &ntt_v_, &ntt_vb_}) {
@@ -1620,7 +1680,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     // pass of its two output rows itself (jobs with at least two transformed
     // parts: two LDS regions to hand the rows over in), and those row-pass
     // jobs leave their stage
-    if (C_.ksi_rowpass && !moddown_.empty() && !intt_pb_.empty()) {
+    if (C_.ksi_rowpass && !intt_pb_.empty()) {
         std::map<const uint64_t*, size_t> by_in;
         for (size_t i = 0; i < intt_pb_.size(); ++i) by_in[intt_pb_[i].in] = i;
         std::vector<char> used(intt_pb_.size(), 0);
@@ -1734,6 +1794,10 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         stage(Step::MODDOWN, moddown_.data() + i, e - i, sizeof(ModupJob));
         P->steps.back().arg = moddown_[i].sp;
         i = e;
+    }
+    if (!ksdown_.empty()) {   // every job has the context's K sources
+        GF_STAGE(KSDOWN, ksdown_);
+        P->steps.back().arg = C_.K;
     }
     GF_STAGE(CONV, conv_dn_);
     GF_STAGE(NTT_F, ntt_conv_);

@@ -88,13 +88,7 @@ struct LevelConst {
     const uint64_t* d_tabRS = nullptr;         // PHatModq * (-P^-1 s1) * R mod q_i, [K][l-1]
     const RsTarget* d_rstg = nullptr;          // [l-1]
     const uint64_t* d_rs_sw = nullptr;         // [2 (l-1)] rs_sw_consts of each surviving tower
-    // the surviving towers as targets of the fused ModDown (ModupJob tables, [l-1])
-    const uint64_t* d_rs_tq = nullptr;
-    const uint64_t* d_rs_tqneg = nullptr;
-    const uint64_t* d_rs_ttw = nullptr;
-    const uint64_t* d_rs_tred = nullptr;
-    const uint64_t* d_rs_ttwd = nullptr;
-    const uint64_t* d_rs_tqf = nullptr;        // [2 (l-1)]
+    const uint64_t* d_tabKS = nullptr;         // PHatModq * (-P^-1) * R mod q_i, [K][l]
 };
 
 // Resident parameter set: Q moduli (L), P moduli (K), part width alpha.
@@ -110,6 +104,14 @@ public:
     std::vector<LevelConst> lv;               // index l = 1..L (0 unused)
     DevBuf consts;                            // all per-level device constants
     const uint64_t* d_zeros = nullptr;        // L + K zero words (a target table with no fp64 target)
+    // the Q towers as targets of the fused ModDown (ModupJob tables, [L];
+    // a level uses a prefix)
+    const uint64_t* d_md_tqneg = nullptr;
+    const uint64_t* d_md_tq = nullptr;
+    const uint64_t* d_md_ttw = nullptr;
+    const uint64_t* d_md_tred = nullptr;
+    const uint64_t* d_md_ttwd = nullptr;
+    const uint64_t* d_md_tqf = nullptr;       // [2 L]
     // EvalMult+Rescale with merged ModDown/rescale, and keyswitches whose
     // digit row pass feeds the key inner product directly (KSI)
     bool fused = true;
@@ -212,8 +214,9 @@ struct Step {
     // NTT_IB: an inverse transform's first (row) pass only; MODUP: the fused
     // ModUp (modup.hpp), arg = the jobs' source count
     // TENSOR_IB: the tensor product fused with the inverse row pass of its t2
+    // KSDOWN: the fused ModDown of keyswitches, arg = the jobs' source count
     enum Kind { NTT_F, NTT_I, TENSOR, CONV, INNER, COMBINE, SWITCH, FUSE, ADD, PERM, COPY, RSV, PTACC,
-                NTT_FA, KSI, NTT_IB, MODUP, MODDOWN, NTT_FB, TENSOR_IB } kind;
+                NTT_FA, KSI, NTT_IB, MODUP, MODDOWN, NTT_FB, TENSOR_IB, KSDOWN } kind;
     size_t off;     // byte offset of the first job in the plan's device buffer
     uint32_t count;
     // KSI: LDS regions (bits 0-7) and waves per workgroup (bits 8-15); the
@@ -326,13 +329,23 @@ private:
         uint32_t l, c;
         const uint64_t *xp, *dt, *dr, *t, *res;
         uint64_t *vc, *out;
+        bool ks = false;   // a keyswitch's ModDown (ks_tail), not a rescale's
     };
     std::vector<ModdownSrc> moddown_src_;   // what each fused ModDown job computes, to run it apart
+    std::vector<ModupJob> ksdown_;          // the fused ModDowns of keyswitches (no dropped tower)
+    std::vector<ModdownSrc> ksdown_src_;
     // the rescale tail of one component of the fused EvalMult+Rescale: the
     // prologue and the epilogue transforms (apart), or the fused ModDown and
     // the epilogue's row pass
     void rescale_tail(const ModdownSrc& m, bool fused);
     bool use_moddown(uint32_t l) const;
+    // the ModDown of one component of a keyswitch, fused with out = t + ba:
+    // conversion, forward transforms and combine (apart), or the fused
+    // ModDown and its row pass with the combine as epilogue
+    void ks_tail(const ModdownSrc& m, bool fused);
+    bool use_ks_moddown() const;
+    // the K P towers as the sources of a fused ModDown job
+    void moddown_sources(ModupJob& J, const LevelConst& lv, const uint64_t* xp) const;
     void evalmult_rescale_fused(uint32_t l, const uint64_t* c0a, const uint64_t* c1a,
                                 const uint64_t* c0b, const uint64_t* c1b, uint64_t* o0, uint64_t* o1,
                                 const DevKey& key, uint64_t* ws);
@@ -356,7 +369,8 @@ private:
                                 uint32_t i) const;
     // gk != 0: the digits are read through the automorphism of index gk
     template <class F>
-    void inner_moddown_src(uint32_t l, const DevKey& key, uint64_t* ws, F digit, uint64_t gk = 0);
+    void inner_moddown_src(uint32_t l, const DevKey& key, uint64_t* ws, F digit, uint64_t gk = 0,
+                           bool p_rowpass = false);
     void moddown_tail(uint32_t l, uint64_t* ws, uint64_t* ba0, uint64_t* ba1, const uint64_t* t0,
                       const uint64_t* t1);
     std::vector<PtAccJob> ptacc_;

@@ -89,6 +89,9 @@ struct NttJob {
     const uint64_t* twd;
     const uint64_t* twrd;
     double fq, fqinv;
+    // forward epilogue: 1: e1 is added as it is (residues in [0, q), or null
+    // for none; c1 unused), out = NTT(in) + e0*c0 + e1
+    uint32_t e1_plain;
 };
 
 // floor(2^64 / q) for the moduli whose forward transforms run without
@@ -424,22 +427,41 @@ GF_HD uint64_t ntt_final(uint64_t v, const NttJob& j) {
 // reduced once (or stored as is for a lazy_out job without epilogue).
 // the epilogue's value for a forward transform's output v and the operands
 // x0 = e0[gi], x1 = e1[gi] (j.e0 set)
-template <bool LZ>
+// EP (ntt_ep_form): 0: both operands times their factors; 1: x1 as it is;
+// 2: no x1
+template <bool LZ, int EP>
 GF_HD uint64_t ntt_ep_value(uint64_t v, const NttJob& j, uint64_t x0, uint64_t x1) {
     if constexpr (LZ) {
         const uint64_t nq = 0 - j.q;
         v += shoup_lazy4(x0, j.c0, j.c0p, nq);
-        v += shoup_lazy4(x1, j.c1, j.c1p, nq);
+        if constexpr (EP == 0) v += shoup_lazy4(x1, j.c1, j.c1p, nq);
+        if constexpr (EP == 1) v += x1;
         return reduce_red(v, j.q, (uint32_t)j.red);
     } else {
         uint64_t r = csub(csub(csub(v, 4 * j.q), 2 * j.q), j.q);
         r = addmod(r, shoup(x0, j.c0, j.c0p, j.q), j.q);
-        return addmod(r, shoup(x1, j.c1, j.c1p, j.q), j.q);
+        if constexpr (EP == 0) r = addmod(r, shoup(x1, j.c1, j.c1p, j.q), j.q);
+        if constexpr (EP == 1) r = addmod(r, x1, j.q);
+        return r;
     }
+}
+// f(integral_constant EP) for the job's epilogue (j.e0 set): uniform per workgroup
+template <class F>
+GF_HD void with_ep(const NttJob& j, F&& f) {
+    if (!j.e1_plain) f(std::integral_constant<int, 0>{});
+    else if (j.e1) f(std::integral_constant<int, 1>{});
+    else f(std::integral_constant<int, 2>{});
 }
 template <bool LZ>
 GF_HD uint64_t ntt_final_ep(uint64_t v, const NttJob& j, uint64_t gi) {
-    if (j.e0) return ntt_ep_value<LZ>(v, j, gat(gcast(j.e0), gi), gat(gcast(j.e1), gi));
+    if (j.e0) {
+        uint64_t r = 0;
+        with_ep(j, [&](auto E) {
+            constexpr int EP = decltype(E)::value;
+            r = ntt_ep_value<LZ, EP>(v, j, gat(gcast(j.e0), gi), EP == 2 ? 0 : gat(gcast(j.e1), gi));
+        });
+        return r;
+    }
     if constexpr (LZ) {
         if (j.lazy_out) return v;
         return reduce_red(v, j.q, (uint32_t)j.red);
@@ -533,7 +555,7 @@ GF_HD void wave_units(uint32_t tid, uint32_t nthr, F f) {
 // words are requested before any is used (per word, the loads would
 // otherwise wait in turn behind the previous word's arithmetic, a memory
 // round trip each; 2 at a time keep the kernel's register count).
-template <uint32_t R, uint32_t WORDS, bool LZ>
+template <uint32_t R, uint32_t WORDS, bool LZ, int EP>
 GF_HD void row_out_ep(const NttJob& j, GF_GLOBAL uint64_t* dst, uint32_t off, const uint64_t* lds, uint32_t tid,
                       uint32_t nthr) {
     const uint32_t W = nthr < 64 ? nthr : 64;
@@ -551,7 +573,7 @@ GF_HD void row_out_ep(const NttJob& j, GF_GLOBAL uint64_t* dst, uint32_t off, co
                 const uint32_t idx = (u0 << R) + (mb + m) * W + lane;
                 if (U % 64 == 0 || idx < WORDS) {
                     x0[m] = gat(e0, off + idx);
-                    x1[m] = gat(e1, off + idx);
+                    x1[m] = EP == 2 ? 0 : gat(e1, off + idx);
                 }
             }
             GF_SCHED_FENCE();
@@ -559,7 +581,7 @@ GF_HD void row_out_ep(const NttJob& j, GF_GLOBAL uint64_t* dst, uint32_t off, co
             for (uint32_t m = 0; m < MB; ++m) {
                 const uint32_t idx = (u0 << R) + (mb + m) * W + lane;
                 if (U % 64 == 0 || idx < WORDS)
-                    gat(dst, off + idx) = ntt_ep_value<LZ>(lds[padded(idx)], j, x0[m], x1[m]);
+                    gat(dst, off + idx) = ntt_ep_value<LZ, EP>(lds[padded(idx)], j, x0[m], x1[m]);
             }
         }
     }
@@ -612,7 +634,9 @@ GF_HD void row_tile(const NttJob& j, const TileDesc& d, const GF_GLOBAL uint64_t
         sync.wave();
         if constexpr (FIN == 2) {
             if (j.e0) {
-                row_out_ep<PL::R, WORDS, LZ>(j, dst, off, lds, tid, nthr);
+                with_ep(j, [&](auto E) {
+                    row_out_ep<PL::R, WORDS, LZ, decltype(E)::value>(j, dst, off, lds, tid, nthr);
+                });
                 return;
             }
         }

@@ -267,8 +267,12 @@ void gf_plan_destroy(gf_plan* p);
 /* ---- plan introspection, for timing one stage on its own stream ----
  * kind: 0 fwd NTT, 1 inverse NTT, 2 tensor, 3 basis conversion, 4 key inner
  * product, 5 ModDown combine, 6 switch modulus, 7 rescale fuse, 8 add,
- * 9 automorphism, 10 copy, 11 dropped-tower build, 12 fused ModDown/rescale
- * prologue.  jobs = towers (or conversion chunks) per launch. */
+ * 9 automorphism, 10 copy, 11 fused ModDown/rescale prologue, 12 plaintext
+ * accumulate, 13 fwd NTT column pass, 14 digit row pass + key inner product,
+ * 15 inverse NTT row pass, 16 fused ModUp, 17 fused ModDown + rescale
+ * prologue, 18 fwd NTT row pass, 19 tensor + inverse row pass, 20 fused
+ * ModDown of a keyswitch.  jobs = towers (or conversion chunks, or parts and
+ * components in the fused steps) per launch. */
 uint32_t gf_plan_num_steps(const gf_plan* p);
 int gf_plan_step_info(const gf_plan* p, uint32_t i, uint32_t* kind, uint32_t* jobs);
 int gf_plan_run_step(gf_plan* p, uint32_t i, hipStream_t s);

@@ -1,0 +1,101 @@
+"""GPU tests of the fused forms of the keyswitch path (fused ModUp, fused
+ModDown with its row-pass epilogue) at the sizes where they can go wrong:
+smallest and largest two-phase rings, one-tower levels, partial digits,
+in-place outputs.  Every result is a residue, compared with the oracle's."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gpu-resident-library_amd"))
+
+from common import make_params  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def G():
+    import gpufhe
+    return gpufhe
+
+
+def rand_rows(mods, n, rng):
+    return np.concatenate([rng.integers(0, int(m), n, dtype=np.uint64) for m in mods])
+
+
+class Setup:
+    def __init__(self, G, n, L, dnum, nkeys=1, **knobs):
+        self.G, self.n, self.L = G, n, L
+        self.P = make_params(n, L, dnum)
+        self.rng = np.random.default_rng(n + 100 * L + dnum)
+        self.ctx = G.Context(n, self.P.q, self.P.p, self.P.roots, dnum)
+        for k, v in knobs.items():
+            self.ctx.set_knob(k, v)
+        self.hk = [tuple(np.concatenate([rand_rows(self.P.mods, n, self.rng) for _ in range(self.P.dnum)])
+                         for _ in range(2)) for _ in range(nkeys)]
+        self.keys = [G.Key(self.ctx, av, bv, self.P.dnum) for av, bv in self.hk]
+        self.s = G.Stream()
+
+    def ct(self, level):
+        return rand_rows(self.P.q[:level], self.n, self.rng)
+
+
+# n, L, dnum: every two-phase split, a digit of one tower, six towers per digit
+FUSED = [(1 << 13, 3, 3), (1 << 13, 6, 1), (1 << 14, 7, 3), (1 << 15, 5, 2), (1 << 16, 4, 2)]
+
+
+@pytest.mark.parametrize("f64", [0, 1])
+@pytest.mark.parametrize("n,L,dnum", FUSED)
+def test_fused_moddown_of_keyswitches(G, n, L, dnum, f64):
+    """Keyswitch, EvalMult, rotation, hoisted rotations and the linear
+    transform with the fused ModDown forced on for single operations, also
+    with outputs over the inputs."""
+    t = Setup(G, n, L, dnum, nkeys=2, modup_min_wgs=0, modup_f64=f64)
+    P, ctx, s = t.P, t.ctx, t.s
+    key, (av, bv) = t.keys[0], t.hk[0]
+    ws = ctx.workspace()
+    ks = [pow(5, 3, 2 * n), 2 * n - 1]
+    for level in sorted({1, 2, L - 1, L}):
+        c = [t.ct(level) for _ in range(4)]
+        w = P.keyswitch(level, c[0], av, bv)
+        for inplace in (False, True):
+            d, b0, b1 = G.Dev.of(c[0]), G.Dev(level * n), G.Dev(level * n)
+            if inplace:
+                b0 = d
+            G.check(G.lib.gf_keyswitch(ctx.h, key.h, level, d.ptr, b0.ptr, b1.ptr, ws.ptr, s.s))
+            s.sync()
+            assert np.array_equal(b0.download(), w[0]) and np.array_equal(b1.download(), w[1]), ("ks", level, inplace)
+        w = P.evalmult(level, *c, av, bv)
+        d = [G.Dev.of(x) for x in c]
+        o = [G.Dev(level * n) for _ in range(2)]
+        G.check(G.lib.gf_evalmult(ctx.h, key.h, level, *[x.ptr for x in d], o[0].ptr, o[1].ptr, ws.ptr, s.s))
+        s.sync()
+        assert np.array_equal(o[0].download(), w[0]) and np.array_equal(o[1].download(), w[1]), ("mult", level)
+        w = P.rotate(level, c[0], c[1], ks[0], av, bv)
+        for inplace in (False, True):
+            d = [G.Dev.of(x) for x in c[:2]]
+            o = d if inplace else [G.Dev(level * n) for _ in range(2)]
+            G.check(G.lib.gf_rotate(ctx.h, key.h, level, ks[0], d[0].ptr, d[1].ptr, o[0].ptr, o[1].ptr, ws.ptr, s.s))
+            s.sync()
+            assert np.array_equal(o[0].download(), w[0]) and np.array_equal(o[1].download(), w[1]), ("rot", level, inplace)
+    level = L
+    wr = [ctx.workspace() for _ in range(3)]
+    c = [t.ct(level) for _ in range(2)]
+    d = [G.Dev.of(x) for x in c]
+    o = [[G.Dev(level * n) for _ in range(2)] for _ in range(2)]
+    G.rotate_hoisted(ctx, level, d[0].ptr, d[1].ptr, t.keys, ks, [x[0].ptr for x in o], [x[1].ptr for x in o], ws.ptr,
+                     [x.ptr for x in wr[:2]], s)
+    s.sync()
+    for (w0, w1), x in zip(P.rotate_hoisted(level, c[0], c[1], ks, t.hk), o):
+        assert np.array_equal(x[0].download(), w0) and np.array_equal(x[1].download(), w1), "hoisted"
+    pts = [t.ct(level) for _ in range(3)]
+    dp = [G.Dev.of(x) for x in pts]
+    a = [G.Dev(level * n) for _ in range(2)]
+    G.linear_transform(ctx, level, d[0].ptr, d[1].ptr, [None] + t.keys, [1] + ks, [x.ptr for x in dp], a[0].ptr, a[1].ptr,
+                       ws.ptr, [x.ptr for x in wr], s)
+    s.sync()
+    w0, w1 = P.linear_transform(level, c[0], c[1], [1] + ks, [None] + t.hk, pts)
+    assert np.array_equal(a[0].download(), w0) and np.array_equal(a[1].download(), w1), "linear"
