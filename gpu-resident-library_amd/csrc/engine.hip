@@ -427,6 +427,8 @@ void Ctx::set_knob(const std::string& name, uint32_t v) {
                                  : moddown_fused) = v;
     } else if (name == "modup_min_wgs") {
         modup_min_wgs = v;
+    } else if (name == "modup_split_wgs") {
+        modup_split_wgs = v;
     } else if (name == "rechunk_wgs") {
         rechunk_wgs = v;
     } else {
@@ -445,6 +447,7 @@ uint32_t Ctx::knob(const std::string& name) const {
     if (name == "ksi_rowpass") return ksi_rowpass;
     if (name == "moddown_fused") return moddown_fused;
     if (name == "modup_min_wgs") return modup_min_wgs;
+    if (name == "modup_split_wgs") return modup_split_wgs;
     if (name == "rechunk_wgs") return rechunk_wgs;
     throw std::runtime_error("gpufhe: unknown tuning knob " + name);
 }
@@ -916,7 +919,7 @@ void Plan::run_jobs(size_t i, hipStream_t s, uint32_t which, uint32_t first, uin
         case Step::KSI: launch_ksi(GF_J(KsiJob), cnt, geom, st.arg & 0xFF, st.arg >> 8, s); break;
         case Step::NTT_IB: launch_ntt(GF_J(NttJob), cnt, geom, false, s, 1); break;
         case Step::MODUP: launch_modup(GF_J(ModupJob), cnt, geom, st.arg, s); break;
-        case Step::MODDOWN: launch_moddown(GF_J(ModupJob), cnt, geom, st.arg, s); break;
+        case Step::MODDOWN: launch_moddown(GF_J(ModupJob), cnt, geom, st.arg & 0xff, s); break;
         case Step::KSDOWN: launch_modup(GF_J(ModupJob), cnt, geom, st.arg, s); break;
         case Step::NTT_FB: launch_ntt(GF_J(NttJob), cnt, geom, true, s, 2); break;
     }
@@ -964,6 +967,24 @@ static void split_chunks(std::vector<J>& v, uint32_t n, uint32_t min_wgs) {
     v.swap(out);
 }
 
+// The target ranges of a fused ModUp or ModDown stage's jobs: all of a job's
+// targets where the stage has min_wgs workgroups (Ctx::modup_split_wgs)
+// without splitting, else as many ranges as it takes (down to one target).
+static void split_targets(std::vector<ModupJob>& v, uint32_t n, uint32_t min_wgs) {
+    const size_t wgs = v.size() * (n / MODUP_TILE);
+    const uint32_t parts = (uint32_t)std::max<size_t>(1, (min_wgs + wgs - 1) / wgs);
+    std::vector<ModupJob> out;
+    for (ModupJob& j : v) {
+        const uint32_t len = std::max(1u, (j.sc + parts - 1) / parts);
+        for (uint32_t t = 0; t < j.sc; t += len) {
+            j.t0 = t;
+            j.t1 = std::min(j.sc, t + len);
+            out.push_back(j);
+        }
+    }
+    v.swap(out);
+}
+
 // Hybrid keyswitch up to the ModDown sources (src/keyswitch_resident.cpp:139-201):
 // ModUp of every digit, the key inner product over Q_l P, and the INTT of both
 // accumulators' P towers scaled by n^-1 PHatInv.  Optional extra inverse
@@ -989,16 +1010,13 @@ bool PlanBuilder::use_ksi(uint32_t l) const {
     return C_.fused && !C_.geom.single && C_.n % KSI_TILE == 0 && C_.lv[l].np <= KSI_MAXP;
 }
 // the fused ModUp: column sums over at most MODUP_MAXSRC sources below 2^60
-bool PlanBuilder::use_modup(uint32_t l) const {
-    return C_.modup_fused && use_ksi(l) && !C_.wide && C_.alpha <= MODUP_MAXSRC && C_.n % MODUP_TILE == 0;
+bool PlanBuilder::use_modup() const {
+    return C_.fused && C_.modup_fused && !C_.geom.single && !C_.wide && C_.alpha <= MODUP_MAXSRC &&
+           C_.n % MODUP_TILE == 0;
 }
-// the fused ModDown + rescale prologue: the fused ModUp's kernel over the K
-// P towers
-bool PlanBuilder::use_moddown(uint32_t l) const {
-    return C_.moddown_fused && use_modup(l) && C_.K <= MODUP_MAXSRC && l >= 2;
-}
-// the fused ModDown of a keyswitch: the same kernel without the dropped tower
-bool PlanBuilder::use_ks_moddown() const {
+// the fused ModDown, of a keyswitch or with the rescale prologue: the fused
+// ModUp's kernel over the K P towers
+bool PlanBuilder::use_moddown() const {
     return C_.fused && C_.moddown_fused && !C_.geom.single && !C_.wide && C_.K <= MODUP_MAXSRC &&
            C_.n % MODUP_TILE == 0;
 }
@@ -1065,7 +1083,7 @@ void PlanBuilder::modup(uint32_t l, const uint64_t* d, uint64_t* ws, const uint6
     uint64_t* dig = ws + w.dig * n;
     // fused: the inverse transforms' row pass here; their column pass, the
     // conversion and the digits' column pass in one ModUp kernel per part
-    const bool fuse = rowpass_in_ksi && use_modup(l);
+    const bool fuse = use_modup();
     // 1. part towers to coefficient form, scaled by n^-1 QHatInv (ModUp's first factor)
     for (uint32_t i = 0; i < l; ++i) {
         const uint32_t pi = i / C.alpha, ii = i - pi * C.alpha;
@@ -1084,7 +1102,7 @@ void PlanBuilder::modup(uint32_t l, const uint64_t* d, uint64_t* ws, const uint6
         const PartConst& P = lv.parts[pi];
         uint64_t* dp = dig + (size_t)pi * W * n;
         if (fuse) {
-            modup_src_.push_back(ModupSrc{l, pi, x, dp});
+            modup_src_.push_back(ModupSrc{l, pi, x, dp, rowpass_in_ksi});
             ModupJob J{};
             for (uint32_t i = 0; i < P.sp; ++i) {
                 const uint32_t r = P.st + i;
@@ -1112,6 +1130,11 @@ void PlanBuilder::modup(uint32_t l, const uint64_t* d, uint64_t* ws, const uint6
             J.sp = P.sp;
             J.sc = P.sc;
             modup_.push_back(J);
+            if (!rowpass_in_ksi)
+                for (uint32_t j = 0; j < P.sc; ++j) {
+                    const uint32_t r = P.compl_rows[j];
+                    ntt_digb_.push_back(NttJob{dp + (size_t)j * n, dp + (size_t)j * n, C.rt[r].fw2, nullptr, C.mods[r], 0, 0});
+                }
             continue;
         }
         modup_unfused(l, pi, x, dp, rowpass_in_ksi);
@@ -1193,7 +1216,7 @@ void PlanBuilder::keyswitch(uint32_t l, const uint64_t* d, uint64_t* ba0, uint64
                             const uint64_t* t1) {
     // with the fused ModDown the accumulators' Q rows only feed its
     // epilogue's lazy Shoup products
-    const bool fmd = use_ks_moddown();
+    const bool fmd = use_moddown();
     keyswitch_core(l, d, key, ws, nullptr, nullptr, nullptr, nullptr, fmd ? l : 0, fmd);
     moddown_tail(l, ws, ba0, ba1, t0, t1);
 }
@@ -1210,7 +1233,7 @@ void PlanBuilder::moddown_tail(uint32_t l, uint64_t* ws, uint64_t* ba0, uint64_t
     uint64_t* conv = ws + w.x * n;  // the part towers are dead once ModUp has converted them
     uint64_t* outs[2] = {ba0, ba1};
     const uint64_t* ts[2] = {t0, t1};
-    const bool fmd = use_ks_moddown();
+    const bool fmd = use_moddown();
     for (int c = 0; c < 2; ++c)
         ks_tail(ModdownSrc{l, (uint32_t)c, xp + (size_t)c * K * n, nullptr, nullptr, ts[c], res[c],
                            conv + (size_t)c * l * n, outs[c], true},
@@ -1302,7 +1325,7 @@ void PlanBuilder::evalmult_rescale_fused(uint32_t l, const uint64_t* c0a, const 
     }
     uint64_t* dt = ws + w.dt * n;
     uint64_t* dr = ws + w.dr * n;
-    const bool fmd = use_moddown(l);
+    const bool fmd = use_moddown();
     // accumulator rows below `last` only feed the epilogue's lazy Shoup products
     keyswitch_core(l, t[2], key, ws, t[0] + (size_t)last * n, t[1] + (size_t)last * n, dt, dt + n, last, fmd);
     uint64_t* res[2] = {ws + w.res0 * n, ws + w.res1 * n};
@@ -1491,7 +1514,7 @@ void PlanBuilder::rotate_hoisted(uint32_t l, uint32_t m, const uint64_t* ks, con
         // the inner product reads the shared digits through sigma_k: no permuted copies
         inner_moddown_src(
             l, *keys[j], ws, [&](uint32_t pi, uint32_t i) { return digit_tower(l, c1, dig, pi, i); }, ks[j],
-            use_ks_moddown());
+            use_moddown());
         moddown_tail(l, ws, o0[j], o1[j], a0, nullptr);
     }
 }
@@ -1634,7 +1657,8 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     if (!modup_.empty() && modup_.size() * (C_.n / MODUP_TILE) < C_.modup_min_wgs) {
         for (NttJob& j : intt_upb_) intt_up_.push_back(j);
         intt_upb_.clear();
-        for (const ModupSrc& m : modup_src_) modup_unfused(m.l, m.pi, m.x, m.dp, true);
+        ntt_digb_.clear();
+        for (const ModupSrc& m : modup_src_) modup_unfused(m.l, m.pi, m.x, m.dp, m.ksi);
         modup_.clear();
         modup_src_.clear();
     }
@@ -1657,7 +1681,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
             for (KsiJob& j : ksi_) j.lazy_out = 0;
         }
     }
-    for (auto* v : {&intt_up_, &intt_upb_, &ntt_dig_, &ntt_diga_, &intt_p_, &intt_pb_, &ntt_conv_, &intt_drop_,
+    for (auto* v : {&intt_up_, &intt_upb_, &ntt_dig_, &ntt_diga_, &ntt_digb_, &intt_p_, &intt_pb_, &ntt_conv_, &intt_drop_,
                     &ntt_sw_, &ntt_v_, &ntt_vb_}) {
         group_by(*v, [](const NttJob& j) { return (uintptr_t)j.tw; });
         // every transform of a plan uses the context's paired tables; its phase B
@@ -1669,9 +1693,10 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     }
     // forward transforms over moduli below 2^57 skip the butterflies'
     // conditional subtractions; the digits stay unreduced for the inner product
-    for (auto* v : {&ntt_dig_, &ntt_diga_, &ntt_conv_, &ntt_sw_, &ntt_v_, &ntt_vb_})
+    for (auto* v : {&ntt_dig_, &ntt_diga_, &ntt_digb_, &ntt_conv_, &ntt_sw_, &ntt_v_, &ntt_vb_})
         for (NttJob& j : *v) j.red = lazy_red_of(j.q);
-    for (NttJob& j : ntt_dig_) j.lazy_out = j.red != 0;
+    for (auto* v : {&ntt_dig_, &ntt_digb_})
+        for (NttJob& j : *v) j.lazy_out = j.red != 0;
     for (KsiJob& j : ksi_) {
         j.twr = C_.row_table_of(j.tw);
         if (!j.twr) throw std::runtime_error("gpufhe: transform table of another context");
@@ -1740,19 +1765,43 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         P->steps.push_back(Step{kind, off, (uint32_t)cnt});
     };
 #define GF_STAGE(k, v) stage(Step::k, v.data(), v.size(), sizeof(v[0]))
+    // one launch for every source count (per conversion reduction), the
+    // longest jobs first
+    auto stage_modup = [&](Step::Kind kind, std::vector<ModupJob>& v) {
+        if (v.empty()) return;
+        split_targets(v, C_.n, C_.modup_split_wgs);
+        std::stable_sort(v.begin(), v.end(), [](const ModupJob& a, const ModupJob& b) {
+            return a.c60 != b.c60 ? a.c60 > b.c60 : a.sp + a.t1 - a.t0 > b.sp + b.t1 - b.t0;
+        });
+        for (size_t i = 0; i < v.size();) {
+            size_t e = i;
+            uint32_t sp = 0;
+            for (; e < v.size() && v[e].c60 == v[i].c60; ++e) sp = std::max(sp, v[e].sp);
+            stage(kind, v.data() + i, e - i, sizeof(ModupJob));
+            P->steps.back().arg = sp | v[i].c60 << 8;
+            i = e;
+        }
+    };
     // the tensor product fused with the inverse row pass of its t2 where every
     // tensor job has that row pass (the fused EvalMult+Rescale with the fused
     // ModUp): t2 goes to the row pass in LDS instead of through HBM
-    if (C_.tensor_ib && !C_.geom.single && C_.geom.R * (1u << C_.geom.logN2) == NTT_TILE && !tensor_.empty() &&
-        tensor_.size() == intt_upb_.size()) {
+    if (C_.tensor_ib && !C_.geom.single && C_.geom.R * (1u << C_.geom.logN2) == NTT_TILE && !tensor_.empty()) {
         std::map<const uint64_t*, size_t> by_in;
         for (size_t i = 0; i < intt_upb_.size(); ++i) by_in[intt_upb_[i].in] = i;
         bool all = true;
         for (const TensorJob& t : tensor_) all &= t.pairs && by_in.count(t.t2) == 1;
-        if (all && by_in.size() == tensor_.size()) {
-            for (const TensorJob& t : tensor_) tensor_ib_.push_back(TensorIbJob{t, intt_upb_[by_in[t.t2]]});
+        if (all) {
+            std::vector<char> used(intt_upb_.size(), 0);
+            for (const TensorJob& t : tensor_) {
+                const size_t i = by_in[t.t2];
+                tensor_ib_.push_back(TensorIbJob{t, intt_upb_[i]});
+                used[i] = 1;
+            }
             tensor_.clear();
-            intt_upb_.clear();
+            std::vector<NttJob> rest;   // row passes of other operations' inputs (rotations in the same plan)
+            for (size_t i = 0; i < intt_upb_.size(); ++i)
+                if (!used[i]) rest.push_back(intt_upb_[i]);
+            intt_upb_.swap(rest);
         }
     }
     GF_STAGE(TENSOR_IB, tensor_ib_);
@@ -1760,20 +1809,11 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(PERM, perm_);
     GF_STAGE(NTT_IB, intt_upb_);
     GF_STAGE(NTT_I, intt_up_);
-    // fused ModUp jobs by source count and conversion reduction (one launch each)
-    auto mkey = [](const ModupJob& a) { return a.sp | a.c60 << 8; };
-    std::stable_sort(modup_.begin(), modup_.end(),
-                     [&](const ModupJob& a, const ModupJob& b) { return mkey(a) < mkey(b); });
-    for (size_t i = 0; i < modup_.size();) {
-        size_t e = i;
-        while (e < modup_.size() && mkey(modup_[e]) == mkey(modup_[i])) ++e;
-        stage(Step::MODUP, modup_.data() + i, e - i, sizeof(ModupJob));
-        P->steps.back().arg = mkey(modup_[i]);
-        i = e;
-    }
+    stage_modup(Step::MODUP, modup_);
     GF_STAGE(CONV, conv_up_);
     GF_STAGE(NTT_F, ntt_dig_);
     GF_STAGE(NTT_FA, ntt_diga_);
+    GF_STAGE(NTT_FB, ntt_digb_);
     GF_STAGE(INNER, inner_);
     for (size_t i = 0; i < ksi_.size();) {
         size_t e = i;
@@ -1785,20 +1825,8 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     }
     GF_STAGE(NTT_I, intt_p_);
     GF_STAGE(NTT_IB, intt_pb_);
-    // fused ModDown jobs by source count (one launch each)
-    std::stable_sort(moddown_.begin(), moddown_.end(),
-                     [](const ModupJob& a, const ModupJob& b) { return a.sp < b.sp; });
-    for (size_t i = 0; i < moddown_.size();) {
-        size_t e = i;
-        while (e < moddown_.size() && moddown_[e].sp == moddown_[i].sp) ++e;
-        stage(Step::MODDOWN, moddown_.data() + i, e - i, sizeof(ModupJob));
-        P->steps.back().arg = moddown_[i].sp;
-        i = e;
-    }
-    if (!ksdown_.empty()) {   // every job has the context's K sources
-        GF_STAGE(KSDOWN, ksdown_);
-        P->steps.back().arg = C_.K;
-    }
+    stage_modup(Step::MODDOWN, moddown_);
+    stage_modup(Step::KSDOWN, ksdown_);
     GF_STAGE(CONV, conv_dn_);
     GF_STAGE(NTT_F, ntt_conv_);
     GF_STAGE(COMBINE, combine_);

@@ -160,9 +160,13 @@ public:
     // one kernel (the fused ModUp kernel's rescale mode), where the fused
     // ModUp runs; stages below modup_min_wgs workgroups run them apart
     uint32_t moddown_fused = 1;
-    // a plan whose fused ModUp stage would launch fewer workgroups than this
-    // runs it unfused (a single operation's stage cannot fill the chip)
-    uint32_t modup_min_wgs = 2048;
+    // a plan whose fused ModUp (or ModDown) stage would launch fewer workgroups
+    // than this runs it unfused
+    uint32_t modup_min_wgs = 512;
+    // fused ModUp and ModDown stages that would launch fewer workgroups than
+    // this split their jobs' targets over more of them, down to one target
+    // each, every one of them transforming the sources anew
+    uint32_t modup_split_wgs = 1024;
     // conversion and prologue stages that would launch fewer workgroups than
     // this are re-split into 8-target jobs, whatever the chunk knobs say
     uint32_t rechunk_wgs = 8192;
@@ -174,7 +178,7 @@ public:
     std::string tune_report;
     // sets or reads a knob by name ("ntt_radix", "ksi_extra", "conv_chunk",
     // "rs_chunk", "modup_fused", "modup_f64", "ksi_f64", "moddown_fused", "tensor_ib", "ksi_rowpass",
-    // "modup_min_wgs", "rechunk_wgs")
+    // "modup_min_wgs", "modup_split_wgs", "rechunk_wgs")
     void set_knob(const std::string& name, uint32_t v);
     uint32_t knob(const std::string& name) const;
     std::string radix_report;   // the radix search of autotune(), as JSON
@@ -212,9 +216,9 @@ struct Step {
     // NTT_FA: a forward transform's first (column) pass only; KSI: the fused
     // row pass of the ModUp digits and the key inner product
     // NTT_IB: an inverse transform's first (row) pass only; MODUP: the fused
-    // ModUp (modup.hpp), arg = the jobs' source count
+    // ModUp (modup.hpp), arg = the jobs' largest source count (MODDOWN and
+    // KSDOWN, the fused ModDown of keyswitches, alike)
     // TENSOR_IB: the tensor product fused with the inverse row pass of its t2
-    // KSDOWN: the fused ModDown of keyswitches, arg = the jobs' source count
     enum Kind { NTT_F, NTT_I, TENSOR, CONV, INNER, COMBINE, SWITCH, FUSE, ADD, PERM, COPY, RSV, PTACC,
                 NTT_FA, KSI, NTT_IB, MODUP, MODDOWN, NTT_FB, TENSOR_IB, KSDOWN } kind;
     size_t off;     // byte offset of the first job in the plan's device buffer
@@ -303,11 +307,13 @@ private:
         uint32_t l, pi;
         const uint64_t* x;
         uint64_t* dp;
+        bool ksi;   // the digits' row pass runs in the KSI step
     };
     std::vector<ModupSrc> modup_src_;   // what each fused ModUp job converts, to run it unfused
     std::vector<ConvJob> conv_up_;
     std::vector<NttJob> ntt_dig_;
     std::vector<NttJob> ntt_diga_;   // digits whose row pass runs inside the KSI step
+    std::vector<NttJob> ntt_digb_;   // digits whose column pass runs in the fused ModUp, and their row pass alone
     std::vector<InnerJob> inner_;
     std::vector<KsiJob> ksi_;
     std::vector<NttJob> intt_p_;
@@ -338,12 +344,11 @@ private:
     // prologue and the epilogue transforms (apart), or the fused ModDown and
     // the epilogue's row pass
     void rescale_tail(const ModdownSrc& m, bool fused);
-    bool use_moddown(uint32_t l) const;
+    bool use_moddown() const;
     // the ModDown of one component of a keyswitch, fused with out = t + ba:
     // conversion, forward transforms and combine (apart), or the fused
     // ModDown and its row pass with the combine as epilogue
     void ks_tail(const ModdownSrc& m, bool fused);
-    bool use_ks_moddown() const;
     // the K P towers as the sources of a fused ModDown job
     void moddown_sources(ModupJob& J, const LevelConst& lv, const uint64_t* xp) const;
     void evalmult_rescale_fused(uint32_t l, const uint64_t* c0a, const uint64_t* c1a,
@@ -361,7 +366,7 @@ private:
     // the digits' row pass fused with the key inner product (two-phase rings,
     // up to KSI_MAXP parts, fused schedule on)
     bool use_ksi(uint32_t l) const;
-    bool use_modup(uint32_t l) const;
+    bool use_modup() const;
     void modup_unfused(uint32_t l, uint32_t pi, const uint64_t* x, uint64_t* dp, bool colpass_only);
     void ksi_moddown_src(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws, uint32_t lazy_rows,
                          bool p_rowpass = false);

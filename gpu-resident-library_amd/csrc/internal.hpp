@@ -229,7 +229,8 @@ void launch_ptacc(const PtAccJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 // job's transformed-part count), waves = workgroup size in waves (1..KSI_WAVES)
 void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, hipStream_t s);
 void launch_tensor_ib(const TensorIbJob* d, uint32_t nj, const NttGeom& g, hipStream_t s);
-// the fused ModUp over jobs of sp sources each
+// the fused ModUp over jobs of at most arg & 0xff sources each and of one c60
+// (arg >> 8)
 void launch_modup(const ModupJob* d, uint32_t nj, const NttGeom& g, uint32_t arg, hipStream_t s);
 void launch_moddown(const ModupJob* d, uint32_t nj, const NttGeom& g, uint32_t sp, hipStream_t s);
 

@@ -133,6 +133,7 @@ struct ModupJob {
     const uint64_t* tsw;
     uint64_t q_old, half, qd_neg, pinv, pinvp;
     uint32_t strided;
+    uint32_t t0, t1;   // the workgroup's targets: [t0, t1) of the sc
 };
 
 // Column access in fp64: the inverse transforms' row-pass output (lazy, below

@@ -99,3 +99,40 @@ def test_fused_moddown_of_keyswitches(G, n, L, dnum, f64):
     s.sync()
     w0, w1 = P.linear_transform(level, c[0], c[1], [1] + ks, [None] + t.hk, pts)
     assert np.array_equal(a[0].download(), w0) and np.array_equal(a[1].download(), w1), "linear"
+
+
+@pytest.mark.parametrize("split", [1, 1 << 20])
+@pytest.mark.parametrize("n,L,dnum", [(1 << 13, 7, 2), (1 << 14, 5, 5), (1 << 15, 8, 2)])
+def test_uneven_batch_in_one_launch(G, n, L, dnum, split):
+    """EvalMult+Rescale, rotations and hoisted rotations of every level in one
+    plan: parts of every source count share a launch, with each job's targets
+    in one workgroup (split 1) and one workgroup per target (2^20)."""
+    t = Setup(G, n, L, dnum, nkeys=2, modup_min_wgs=0, modup_split_wgs=split)
+    P, ctx, s = t.P, t.ctx, t.s
+    ks = [pow(5, 7, 2 * n), 3]
+    levels = list(range(2, L + 1))
+    c = [[t.ct(lv) for _ in range(4)] for lv in levels]
+    d = [[G.Dev.of(x) for x in v] for v in c]
+    ws = [ctx.workspace() for _ in range(3 * len(levels))]
+    o = [[G.Dev((lv - 1) * n) for _ in range(2)] for lv in levels]
+    plan = G.plan_evalmult_rescale(ctx, t.keys[0], levels, *[[x[j].ptr for x in d] for j in range(4)],
+                                   [x[0].ptr for x in o], [x[1].ptr for x in o], [w.ptr for w in ws[:len(levels)]])
+    r = [[G.Dev(lv * n) for _ in range(2)] for lv in levels]
+    rplan = G.plan_rotate(ctx, [t.keys[i % 2] for i in range(len(levels))], levels, [ks[i % 2] for i in range(len(levels))],
+                          [x[0].ptr for x in d], [x[1].ptr for x in d], [x[0].ptr for x in r], [x[1].ptr for x in r],
+                          [w.ptr for w in ws[:len(levels)]])
+    h = [[G.Dev(lv * n) for _ in range(2)] for lv in levels for _ in ks]
+    hplan = G.plan_rotate_hoisted(ctx, levels, [x[0].ptr for x in d], [x[1].ptr for x in d], t.keys, ks,
+                                  [x[0].ptr for x in h], [x[1].ptr for x in h], [w.ptr for w in ws[:len(levels)]],
+                                  [w.ptr for w in ws[len(levels):]])
+    for p in (plan, rplan, hplan):
+        p.run(s)
+    s.sync()
+    for i, lv in enumerate(levels):
+        w = P.evalmult_rescale(lv, *c[i], *t.hk[0])
+        assert np.array_equal(o[i][0].download(), w[0]) and np.array_equal(o[i][1].download(), w[1]), ("mult", lv)
+        w = P.rotate(lv, c[i][0], c[i][1], ks[i % 2], *t.hk[i % 2])
+        assert np.array_equal(r[i][0].download(), w[0]) and np.array_equal(r[i][1].download(), w[1]), ("rot", lv)
+        for j, w in enumerate(P.rotate_hoisted(lv, c[i][0], c[i][1], ks, t.hk)):
+            x = h[2 * i + j]
+            assert np.array_equal(x[0].download(), w[0]) and np.array_equal(x[1].download(), w[1]), ("hoist", lv, j)
