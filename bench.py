@@ -80,6 +80,17 @@ def step_bytes(n, L, K, alpha, np_parts, kinds, batch):
     by a fused transform epilogue)."""
     T = 8 * n
     key = 2 * np_parts / batch   # key rows read per tower row, per op
+    # the dropped tower's inverse transform inside the other steps: one per
+    # component, of t + res / P, its row pass in the Q rows' inner product (t's
+    # two towers in, two out; the accumulators' stay on chip) and its column
+    # pass in the fused ModDown (half of two transforms, and one operand of
+    # the prologue fewer per component: the same bytes)
+    if "ntt_inv" not in kinds and "moddown" in kinds:
+        up, dn = kinds.index("modup"), kinds.index("moddown")
+        full = step_bytes(n, L, K, alpha, np_parts, list(kinds[:up]) + ["ntt_inv"] + list(kinds[up:dn]) + ["ntt_inv"] +
+                          list(kinds[dn:]), batch)
+        return [(name, b + (2 * T if name == "rowpass_inner_q" else 0), e) for name, b, e in full
+                if name not in ("intt_extra", "intt_moddown_last")]
     # the tensor product fused with the inverse row pass of its t2 is charged
     # as the two steps it replaces
     tensor_ib = kinds[:1] == ["tensor_ib"]

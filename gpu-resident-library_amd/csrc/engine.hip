@@ -991,13 +991,14 @@ static void split_targets(std::vector<ModupJob>& v, uint32_t n, uint32_t min_wgs
 // transforms (plain n^-1) ride in the first INTT launch.
 void PlanBuilder::keyswitch_core(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws,
                                  const uint64_t* extra0, const uint64_t* extra1, uint64_t* dx0,
-                                 uint64_t* dx1, uint32_t lazy_rows, bool p_rowpass) {
+                                 uint64_t* dx1, uint32_t lazy_rows, bool p_rowpass, const uint64_t* drop0,
+                                 const uint64_t* drop1, uint64_t* dr) {
     const Ctx& C = C_;
     if (l < 1 || l > C.L) throw std::runtime_error("gpufhe: bad level");
     if (key.nparts < C.lv[l].np) throw std::runtime_error("gpufhe: key has too few parts for this level");
     if (use_ksi(l)) {
         modup(l, d, ws, extra0, extra1, dx0, dx1, true);
-        ksi_moddown_src(l, d, key, ws, lazy_rows, p_rowpass);
+        ksi_moddown_src(l, d, key, ws, lazy_rows, p_rowpass, drop0, drop1, dr);
         return;
     }
     modup(l, d, ws, extra0, extra1, dx0, dx1);
@@ -1028,7 +1029,8 @@ bool PlanBuilder::use_moddown() const {
 // the column-pass output of their forward transform (modup with
 // rowpass_in_ksi).
 void PlanBuilder::ksi_moddown_src(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws,
-                                  uint32_t lazy_rows, bool p_rowpass) {
+                                  uint32_t lazy_rows, bool p_rowpass, const uint64_t* drop0, const uint64_t* drop1,
+                                  uint64_t* dr) {
     const Ctx& C = C_;
     const uint32_t n = C.n, K = C.K, W = l + K;
     const LevelConst& lv = C.lv[l];
@@ -1060,6 +1062,25 @@ void PlanBuilder::ksi_moddown_src(uint32_t l, const uint64_t* d, const DevKey& k
         J.lazy_out = i < lazy_rows;
         J.pairs = aligned16({J.o0, J.o1});
         for (uint32_t pi = 0; pi < lv.np; ++pi) J.pairs &= aligned16({J.src[pi], J.kb[pi], J.ka[pi]});
+        if (drop0 && i + 1 == l) {
+            J.drop[0] = drop0;
+            J.drop[1] = drop1;
+            J.pairs &= aligned16({drop0, drop1});
+            J.dpinv = lv.pinv[i];
+            J.dpinvp = lv.pinvp[i];
+            J.rp_on = 1;
+            for (int c = 0; c < 2; ++c) {
+                NttJob& R = J.rp[c];
+                R = NttJob{nullptr, dr + (size_t)c * n, C.rt[row].iv2, nullptr, J.q, C.rc[row].ninv, C.rc[row].ninvp};
+                R.twr = C.rtr[row].inv;
+                if (C.modup_f64 && C.rt[row].iv2d) {
+                    R.twd = C.rt[row].iv2d;
+                    R.twrd = C.rtr[row].inv_d;
+                    R.fq = (double)J.q;
+                    R.fqinv = 1.0 / R.fq;
+                }
+            }
+        }
         ksi_.push_back(J);
     }
     for (int c = 0; c < 2; ++c)
@@ -1326,17 +1347,27 @@ void PlanBuilder::evalmult_rescale_fused(uint32_t l, const uint64_t* c0a, const 
     uint64_t* dt = ws + w.dt * n;
     uint64_t* dr = ws + w.dr * n;
     const bool fmd = use_moddown();
+    // The dropped tower needs INTT(t_last) + INTT(res_last) P^-1 = INTT(t_last +
+    // res_last P^-1).  Where the inner product can run row passes itself, it
+    // runs that transform's on the last row, and the fused ModDown its column
+    // pass: one inverse transform per component instead of two, and none of
+    // the four launches they took (170 of 7770 us for 64 operations at
+    // n = 2^16, L = 24; 38 of 293 us for one).
+    const uint64_t* tl[2] = {t[0] + (size_t)last * n, t[1] + (size_t)last * n};
+    const bool drop = fmd && use_ksi(l) && C.ksi_rowpass;
     // accumulator rows below `last` only feed the epilogue's lazy Shoup products
-    keyswitch_core(l, t[2], key, ws, t[0] + (size_t)last * n, t[1] + (size_t)last * n, dt, dt + n, last, fmd);
+    if (drop) keyswitch_core(l, t[2], key, ws, nullptr, nullptr, nullptr, nullptr, last, true, tl[0], tl[1], dr);
+    else keyswitch_core(l, t[2], key, ws, tl[0], tl[1], dt, dt + n, last, fmd);
     uint64_t* res[2] = {ws + w.res0 * n, ws + w.res1 * n};
     uint64_t* xp = ws + w.xp * n;
     uint64_t* v = ws + w.dig * n;     // digits are dead after the inner product
     uint64_t* outs[2] = {o0, o1};
     for (int c = 0; c < 2; ++c) {
-        intt_p_.push_back(NttJob{res[c] + (size_t)last * n, dr + (size_t)c * n, C.rt[last].iv2, nullptr,
-                                 C.mods[last], C.rt[last].ninv, C.rt[last].ninvp});
+        if (!drop)
+            intt_p_.push_back(NttJob{res[c] + (size_t)last * n, dr + (size_t)c * n, C.rt[last].iv2, nullptr,
+                                     C.mods[last], C.rt[last].ninv, C.rt[last].ninvp});
         const ModdownSrc m{l, (uint32_t)c, xp + (size_t)c * K * n, dt + (size_t)c * n, dr + (size_t)c * n,
-                           t[c], res[c], v + (size_t)c * last * n, outs[c]};
+                           t[c], res[c], v + (size_t)c * last * n, outs[c], false, drop};
         rescale_tail(m, fmd);
     }
 }
@@ -1356,6 +1387,19 @@ void PlanBuilder::rescale_tail(const ModdownSrc& m, bool fused) {
         J.sc = last;
         J.dt = m.dt;
         J.dr = m.dr;
+        if (m.drop) {
+            J.src[K] = m.dr;
+            J.stw[K] = C.rt[last].iv2;
+            J.sq[K] = C.mods[last];
+            J.post[K] = C.rt[last].ninv;
+            J.postp[K] = C.rt[last].ninvp;
+            if (C.modup_f64 && C.rt[last].iv2d) {
+                J.stwd[K] = C.rt[last].iv2d;
+                J.sqd[K] = (double)C.mods[last];
+                J.sqinv[K] = 1.0 / J.sqd[K];
+                f64_twiddle(C.rt[last].ninv, C.mods[last], J.spost[K], J.spostq[K]);
+            }
+        }
         J.tabd = lv.d_tabMD + last;   // PHatModq column of q_last, row stride l
         J.tg = lv.d_rstg;
         J.tsw = lv.d_rs_sw;
@@ -1672,7 +1716,21 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         moddown_.clear();
         std::vector<ModdownSrc> ms;
         ms.swap(moddown_src_);
-        for (const ModdownSrc& m : ms) rescale_tail(m, false);
+        for (const ModdownSrc& m : ms) {
+            rescale_tail(m, false);
+            if (!m.drop) continue;
+            // the prologue takes the dropped tower's two operands apart
+            const uint32_t last = m.l - 1;
+            intt_up_.push_back(NttJob{m.t + (size_t)last * C_.n, const_cast<uint64_t*>(m.dt), C_.rt[last].iv2, nullptr,
+                                      C_.mods[last], C_.rt[last].ninv, C_.rt[last].ninvp});
+            intt_p_.push_back(NttJob{m.res + (size_t)last * C_.n, const_cast<uint64_t*>(m.dr), C_.rt[last].iv2, nullptr,
+                                     C_.mods[last], C_.rt[last].ninv, C_.rt[last].ninvp});
+        }
+        for (KsiJob& j : ksi_) {
+            if (!j.drop[0]) continue;
+            j.drop[0] = j.drop[1] = nullptr;
+            j.rp_on = 0;
+        }
         if (!ksdown_.empty()) {
             ksdown_.clear();
             ms.clear();
@@ -1702,16 +1760,15 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         if (!j.twr) throw std::runtime_error("gpufhe: transform table of another context");
     }
     // with the fused ModDown, a P row's inner product runs the inverse row
-    // pass of its two output rows itself (jobs with at least two transformed
-    // parts: two LDS regions to hand the rows over in), and those row-pass
-    // jobs leave their stage
+    // pass of its two output rows itself (from two LDS regions, ksi_regions),
+    // and those row-pass jobs leave their stage
     if (C_.ksi_rowpass && !intt_pb_.empty()) {
         std::map<const uint64_t*, size_t> by_in;
         for (size_t i = 0; i < intt_pb_.size(); ++i) by_in[intt_pb_[i].in] = i;
         std::vector<char> used(intt_pb_.size(), 0);
         for (KsiJob& j : ksi_) {
             const auto a = by_in.find(j.o0), b = by_in.find(j.o1);
-            if (a == by_in.end() || b == by_in.end() || __builtin_popcount(j.xf) < 2 || j.lazy_out) continue;
+            if (a == by_in.end() || b == by_in.end() || j.lazy_out) continue;
             if (used[a->second] || used[b->second]) continue;
             j.rp_on = 1;
             j.rp[0] = intt_pb_[a->second];
@@ -1741,11 +1798,10 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
             for (KsiJob& j : ksi_) f64_job(j);
         for (NttJob& j : intt_upb_) f64_job(j);
     }
-    // KSI jobs by transformed-part count (one step each: that many LDS
-    // regions and waves), by key within a step
-    auto nxf = [](const KsiJob& j) { return (uint32_t)__builtin_popcount(j.xf); };
+    // KSI jobs by their LDS regions (one step each: that many regions and
+    // waves), by key within a step
     group_by(ksi_, [](const KsiJob& j) { return (uintptr_t)j.kb[0]; });
-    group_by(ksi_, nxf);
+    group_by(ksi_, ksi_regions);
     group_by(inner_, [](const InnerJob& j) { return (uintptr_t)j.kb[0]; });
     split_chunks(conv_up_, C_.n, C_.rechunk_wgs);
     split_chunks(conv_dn_, C_.n, C_.rechunk_wgs);
@@ -1817,8 +1873,8 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(INNER, inner_);
     for (size_t i = 0; i < ksi_.size();) {
         size_t e = i;
-        while (e < ksi_.size() && nxf(ksi_[e]) == nxf(ksi_[i])) ++e;
-        const uint32_t x = nxf(ksi_[i]), waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
+        while (e < ksi_.size() && ksi_regions(ksi_[e]) == ksi_regions(ksi_[i])) ++e;
+        const uint32_t x = ksi_regions(ksi_[i]), waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
         stage(Step::KSI, ksi_.data() + i, e - i, sizeof(KsiJob));
         P->steps.back().arg = x | waves << 8;
         i = e;

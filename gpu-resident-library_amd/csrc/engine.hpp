@@ -162,7 +162,7 @@ public:
     uint32_t moddown_fused = 1;
     // a plan whose fused ModUp (or ModDown) stage would launch fewer workgroups
     // than this runs it unfused
-    uint32_t modup_min_wgs = 512;
+    uint32_t modup_min_wgs = 0;
     // fused ModUp and ModDown stages that would launch fewer workgroups than
     // this split their jobs' targets over more of them, down to one target
     // each, every one of them transforming the sources anew
@@ -336,6 +336,7 @@ private:
         const uint64_t *xp, *dt, *dr, *t, *res;
         uint64_t *vc, *out;
         bool ks = false;   // a keyswitch's ModDown (ks_tail), not a rescale's
+        bool drop = false; // the dropped tower comes from the inner product's row pass (KsiJob::drop)
     };
     std::vector<ModdownSrc> moddown_src_;   // what each fused ModDown job computes, to run it apart
     std::vector<ModupJob> ksdown_;          // the fused ModDowns of keyswitches (no dropped tower)
@@ -357,10 +358,13 @@ private:
     // lazy_rows: accumulator rows below it only feed the fused rescale
     // epilogue, so the fused inner product may leave them unreduced
     // p_rowpass: the P towers' inverse transforms stop after their row pass
-    // (their column pass runs in the fused ModDown)
+    // (their column pass runs in the fused ModDown).  drop0/1, dr: the tensor's
+    // last towers and where the inner product leaves the row pass of the
+    // dropped tower's inverse transforms (KsiJob::drop)
     void keyswitch_core(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws,
                         const uint64_t* extra0, const uint64_t* extra1, uint64_t* dx0, uint64_t* dx1,
-                        uint32_t lazy_rows = 0, bool p_rowpass = false);
+                        uint32_t lazy_rows = 0, bool p_rowpass = false, const uint64_t* drop0 = nullptr,
+                        const uint64_t* drop1 = nullptr, uint64_t* dr = nullptr);
     void modup(uint32_t l, const uint64_t* d, uint64_t* ws, const uint64_t* extra0, const uint64_t* extra1,
                uint64_t* dx0, uint64_t* dx1, bool rowpass_in_ksi = false);
     // the digits' row pass fused with the key inner product (two-phase rings,
@@ -369,7 +373,7 @@ private:
     bool use_modup() const;
     void modup_unfused(uint32_t l, uint32_t pi, const uint64_t* x, uint64_t* dp, bool colpass_only);
     void ksi_moddown_src(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws, uint32_t lazy_rows,
-                         bool p_rowpass = false);
+                         bool p_rowpass, const uint64_t* drop0, const uint64_t* drop1, uint64_t* dr);
     const uint64_t* digit_tower(uint32_t l, const uint64_t* d, const uint64_t* dig, uint32_t pi,
                                 uint32_t i) const;
     // gk != 0: the digits are read through the automorphism of index gk

@@ -10,25 +10,29 @@ namespace gf {
 // unit arrays are indexed by constants and stay in registers); source I is
 // phase I and takes LDS tile I mod 2 and twiddle tile I mod 2; its twiddles
 // are requested with its first pass's data
+// source i's inverse column pass into the unit registers v, as phase i
+template <uint32_t S1>
+__device__ __forceinline__ void modup_source(const ModupJob& j, uint32_t i, const NttGeom& g, uint64_t* lds,
+                                             uint64_t (*twl)[2u << S1], uint32_t tid, uint32_t tile, uint64_t* v) {
+    constexpr uint32_t TWP = 1u << S1, TWPER = TWP > MODUP_THREADS ? TWP / MODUP_THREADS : 1;
+    Words2 tp[TWPER];
+#pragma unroll
+    for (uint32_t k = 0; k < TWPER; ++k)
+        if (tid + k * MODUP_THREADS < TWP) tp[k] = modup_src_tw_pair(j, i, tid + k * MODUP_THREADS);
+    uint64_t* tl = twl[i & 1];
+    modup_source_pass<S1, false>(j, i, g, tile, lds + (i & 1) * MODUP_TILE, tid, MODUP_THREADS, DevSync{}, v, tl, [&] {
+#pragma unroll
+        for (uint32_t k = 0; k < TWPER; ++k)
+            if (tid + k * MODUP_THREADS < TWP) modup_tw_put(tl, tid + k * MODUP_THREADS, tp[k]);
+    });
+}
 template <uint32_t S1, uint32_t SP, uint32_t I>
 __device__ __forceinline__ void modup_sources(const ModupJob& j, const NttGeom& g, uint64_t* lds,
                                               uint64_t (*twl)[2u << S1], uint32_t tid, uint32_t tile,
                                               ModupUnit<SP>& x) {
     if constexpr (I < SP) {
-        constexpr uint32_t TWP = 1u << S1, TWPER = TWP > MODUP_THREADS ? TWP / MODUP_THREADS : 1;
-        Words2 tp[TWPER];
-#pragma unroll
-        for (uint32_t k = 0; k < TWPER; ++k)
-            if (tid + k * MODUP_THREADS < TWP) tp[k] = modup_src_tw_pair(j, I, tid + k * MODUP_THREADS);
-        uint64_t* tl = twl[I & 1];
         uint64_t v[MODUP_UNIT];
-        modup_source_pass<S1, false>(j, I, g, tile, lds + (I & 1) * MODUP_TILE, tid, MODUP_THREADS, DevSync{}, v, tl,
-                                     [&] {
-#pragma unroll
-                                         for (uint32_t k = 0; k < TWPER; ++k)
-                                             if (tid + k * MODUP_THREADS < TWP)
-                                                 modup_tw_put(tl, tid + k * MODUP_THREADS, tp[k]);
-                                     });
+        modup_source<S1>(j, I, g, lds, twl, tid, tile, v);
         modup_take_unit<SP, S1>(j, I, v, x);
         modup_sources<S1, SP, I + 1>(j, g, lds, twl, tid, tile, x);
     }
@@ -43,17 +47,17 @@ __device__ __forceinline__ void modup_run(const ModupJob& j, const NttGeom& g, u
     constexpr uint32_t TWP = 1u << S1, TWPER = TWP > MODUP_THREADS ? TWP / MODUP_THREADS : 1;
     ModupUnit<SP> x;
     modup_sources<S1, SP, 0>(j, g, lds, twl, tid, tile, x);
-    // target t is phase SP + t - t0; its twiddles are requested before its
+    // target t is phase ph0 + t - t0; its twiddles are requested before its
     // conversion and stored to LDS after it
     uint64_t cv[MODUP_UNIT];
-    const uint32_t t0 = j.t0, t1 = j.t1;
+    const uint32_t t0 = j.t0, t1 = j.t1, ph0 = SP + (RS && j.src[SP] ? 1 : 0);
     auto target = [&](uint32_t t, auto&& convert) {
         Words2 tp[TWPER];
 #pragma unroll
         for (uint32_t k = 0; k < TWPER; ++k)
             if (tid + k * MODUP_THREADS < TWP) tp[k] = modup_tw_pair(j, t, tid + k * MODUP_THREADS);
         convert();
-        const uint32_t ph = (SP + t - t0) & 1;
+        const uint32_t ph = (ph0 + t - t0) & 1;
         uint64_t* tl = twl[ph];
 #pragma unroll
         for (uint32_t k = 0; k < TWPER; ++k)
@@ -62,7 +66,12 @@ __device__ __forceinline__ void modup_run(const ModupJob& j, const NttGeom& g, u
     };
     if constexpr (RS) {
         uint64_t dv[MODUP_UNIT];
-        modup_drop_unit<SP, S1>(j, g, tile, tid, x, dv);
+        if (j.src[SP]) {
+            modup_source<S1>(j, SP, g, lds, twl, tid, tile, cv);
+            modup_drop_src<SP, S1>(j, x, cv, dv);
+        } else {
+            modup_drop_unit<SP, S1>(j, g, tile, tid, x, dv);
+        }
         for (uint32_t t = t0; t < t1; ++t) target(t, [&] { modup_rs_unit<SP, S1>(j, t, x, dv, cv); });
     } else {
         for (uint32_t t = t0; t < t1; ++t) target(t, [&] { modup_convert_unit<SP, S1, C60>(j, t, x, cv); });
@@ -74,7 +83,7 @@ __device__ __forceinline__ void modup_run(const ModupJob& j, const NttGeom& g, u
 // of uneven levels has a few jobs of each count below the part width, and
 // launched apart those launches fill a part of the chip each (rotations of 64
 // ciphertexts at levels 8..20, n = 2^16: five launches of 63, 68, 81, 89 and
-// 744 us became one of 946).  SPMAX keeps the registers of small
+// 744 us became one of 898).  SPMAX keeps the registers of small
 // contexts down (8 per source).
 template <uint32_t S1, uint32_t SPMAX, bool RS, bool C60>
 __global__ __launch_bounds__(MODUP_THREADS) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_modup(const ModupJob* __restrict__ jobs, uint32_t off, NttGeom g) {

@@ -58,11 +58,21 @@ struct KsiJob {
     double fq, fqinv;
     // rp_on: the row's two outputs are not stored; instead the inverse
     // transforms' row pass rp[c] (its input tower o0 / o1) runs on them after
-    // the inner product, from LDS (at least two transformed parts, so two LDS
-    // regions)
+    // the inner product, from LDS (two LDS regions at least, ksi_regions)
     uint32_t rp_on;
     NttJob rp[2];
+    // with rp_on, the dropped tower of a rescale (else null): the row pass runs
+    // on drop[c] + output times dpinv (dpinv = P^-1 mod q), the evaluation form
+    // of the dropped tower but for its ModDown conversion
+    const uint64_t* drop[2];
+    uint64_t dpinv, dpinvp;
 };
+// LDS regions of a job: one per transformed part, and two where the row pass
+// takes its outputs
+inline uint32_t ksi_regions(const KsiJob& j) {
+    const uint32_t x = (uint32_t)__builtin_popcount(j.xf);
+    return j.rp_on && x < 2 ? 2 : x;
+}
 
 // V consecutive words from word i of a tower (V = 2: one 16-byte access; the
 // address is 16-byte aligned), addressed as base + 32-bit byte offset (gat)
@@ -101,10 +111,20 @@ template <uint32_t V>
 GF_HD void ksi_store(const KsiJob& j, uint64_t* lds, uint32_t idx, uint32_t gi, const uint64_t* r0,
                      const uint64_t* r1) {
     if (j.rp_on) {
+        uint64_t t0[V], t1[V];
+        if (j.drop[0]) {
+            load_words<V>(gcast(j.drop[0]), gi, t0);
+            load_words<V>(gcast(j.drop[1]), gi, t1);
+        }
 #pragma unroll
         for (uint32_t v = 0; v < V; ++v) {
-            lds[padded(idx + v)] = r0[v];
-            lds[KSI_PART_WORDS + padded(idx + v)] = r1[v];
+            uint64_t a = r0[v], b = r1[v];
+            if (j.drop[0]) {
+                a = addmod(t0[v], shoup(a, j.dpinv, j.dpinvp, j.q), j.q);
+                b = addmod(t1[v], shoup(b, j.dpinv, j.dpinvp, j.q), j.q);
+            }
+            lds[padded(idx + v)] = a;
+            lds[KSI_PART_WORDS + padded(idx + v)] = b;
         }
         return;
     }
@@ -296,8 +316,13 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
         bsync();
         for (uint32_t c = wave; c < 2; c += nwaves) {
             const NttJob& r = j.rp[c];
-            row_tile<false, false, true, S2, RM, ROWS, 0, true, WSync, false, true>(
-                r, d, nullptr, gcast(r.out), off, lds + c * KSI_PART_WORDS, lane, wlanes, wsync);
+            if (r.twd)
+                row_tile_f64<false, S2, RM, ROWS, false, WSync, true>(r.twd, r.twrd, r.fq, r.fqinv, d, nullptr,
+                                                                      gcast(r.out), off, lds + c * KSI_PART_WORDS, lane,
+                                                                      wlanes, wsync);
+            else
+                row_tile<false, false, true, S2, RM, ROWS, 0, true, WSync, false, true>(
+                    r, d, nullptr, gcast(r.out), off, lds + c * KSI_PART_WORDS, lane, wlanes, wsync);
         }
     }
 }

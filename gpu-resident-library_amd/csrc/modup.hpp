@@ -94,9 +94,10 @@ inline void rs_sw_consts(uint64_t q, uint64_t q_old, uint64_t s2, uint64_t& cs, 
 }
 
 struct ModupJob {
-    const uint64_t* src[MODUP_MAXSRC];   // the inverse transforms' row-pass output, tower st + i
-    const uint64_t* stw[MODUP_MAXSRC];   // their paired inverse twiddle tables
-    uint64_t sq[MODUP_MAXSRC], post[MODUP_MAXSRC], postp[MODUP_MAXSRC];   // modulus, n^-1 QHatInv
+    // sources (index sp: the dropped tower of the rescale mode, below)
+    const uint64_t* src[MODUP_MAXSRC + 1];   // the inverse transforms' row-pass output, tower st + i
+    const uint64_t* stw[MODUP_MAXSRC + 1];   // their paired inverse twiddle tables
+    uint64_t sq[MODUP_MAXSRC + 1], post[MODUP_MAXSRC + 1], postp[MODUP_MAXSRC + 1];   // modulus, n^-1 QHatInv
     uint64_t* dst;                        // complement digit j at dst + j n: its column-pass output
     const uint64_t* tab;                  // [sp][sc] conversion constants (Montgomery form)
     const uint64_t* tq;                   // [sc] target moduli
@@ -109,8 +110,8 @@ struct ModupJob {
     // with its fl(./q).  Target t: ttwd[t] the address of its forward pairs
     // (0: the integer passes), tqf[2t], tqf[2t+1] the bit patterns of q and
     // fl(1/q).
-    const uint64_t* stwd[MODUP_MAXSRC];
-    double sqd[MODUP_MAXSRC], sqinv[MODUP_MAXSRC], spost[MODUP_MAXSRC], spostq[MODUP_MAXSRC];
+    const uint64_t* stwd[MODUP_MAXSRC + 1];
+    double sqd[MODUP_MAXSRC + 1], sqinv[MODUP_MAXSRC + 1], spost[MODUP_MAXSRC + 1], spostq[MODUP_MAXSRC + 1];
     const uint64_t* ttwd;
     const uint64_t* tqf;
     // 1: tab holds the constants times 2^60 (not 2^64) and the conversion
@@ -124,7 +125,11 @@ struct ModupJob {
     // surviving Q towers.  Per position the dropped tower
     //   dv = dt + (dr - REDC(sum_k x_k tabd[k strided])) pinv   (mod q_old)
     // then per target rs_lazy_value(dv, dv > half, tg[t], sum_k x_k tab[k sc + t]),
-    // as the prologue kernel computes them (RsJob)
+    // as the prologue kernel computes them (RsJob).  With src[sp] set, dt and
+    // dr are unused: src[sp] is the row-pass output of the inverse transform
+    // of t + res pinv (which KsiJob::drop leaves), post[sp] = n^-1, and
+    //   dv = INTT(t + res pinv) - REDC(..) pinv,
+    // the same residue by linearity.
     const uint64_t* dt;
     const uint64_t* dr;
     const uint64_t* tabd;
@@ -323,6 +328,23 @@ GF_HD void modup_drop_unit(const ModupJob& j, const NttGeom& g, uint32_t tile, u
         const U128 acc = dot30<SP>(x.lo[u], x.hi[u], [&](uint32_t k) { return uniform_at(j.tabd, k * j.strided); });
         const uint64_t cd = redc(acc, q, j.qd_neg);
         dv[u] = addmod(gat(gcast(j.dt), gi), shoup(submod(gat(gcast(j.dr), gi), cd, q), j.pinv, j.pinvp, q), q);
+    }
+}
+// the same from the unit v that the source pass of src[sp] left: d = its value
+// times n^-1, less the conversion times P^-1
+template <uint32_t SP, uint32_t S1>
+GF_HD void modup_drop_src(const ModupJob& j, const ModupUnit<SP>& x, const uint64_t* v, uint64_t* dv) {
+    const uint64_t q = j.q_old;
+#pragma unroll
+    for (uint32_t u = 0; u < MODUP_UNIT; ++u) {
+        uint64_t r;
+        if (j.stwd[SP])
+            r = u52_from_f64(f64_reduce(f64_mulmod(f64_of_bits(v[u]), j.spost[SP], j.spostq[SP], j.sqd[SP]), j.sqd[SP],
+                                        j.sqinv[SP]));
+        else
+            r = shoup(v[u], j.post[SP], j.postp[SP], q);
+        const U128 acc = dot30<SP>(x.lo[u], x.hi[u], [&](uint32_t k) { return uniform_at(j.tabd, k * j.strided); });
+        dv[u] = submod(r, shoup(redc(acc, q, j.qd_neg), j.pinv, j.pinvp, q), q);
     }
 }
 // Rescale mode: target t's prologue value of this thread's unit into cv,
