@@ -21,9 +21,16 @@
 
 namespace gf {
 
+// Tiles of 512 positions: one radix-8 unit per lane and pass, half the LDS
+// and half the serial work per workgroup of 1024.  The row passes wait on
+// memory and the inner product on memory, so what counts is how many
+// workgroups a CU holds and how evenly they interleave (64 EvalMult+Rescale at
+// n = 2^16, L = 24: 7690 -> 7590 us; a 10-deep chain of 16 at n = 2^15: 3418 ->
+// 3231; one rotation at n = 2^15: 115 -> 98).  256 positions leave half the
+// lanes of a pass idle (8490 us).
 enum {
     KSI_MAXP = 7,                                    // parts per job (KSI_MAXP regions fit 64 KiB of LDS)
-    KSI_LOG_TILE = 10,
+    KSI_LOG_TILE = 9,
     KSI_TILE = 1 << KSI_LOG_TILE,                    // positions per workgroup
     KSI_PART_WORDS = KSI_TILE + KSI_TILE / 16,       // one part's padded LDS region
     KSI_WAVES = 5,                                   // largest workgroup, in waves
