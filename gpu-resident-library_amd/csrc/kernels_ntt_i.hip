@@ -30,7 +30,7 @@ void launch_tensor_ib(const TensorIbJob* d, uint32_t nj, const NttGeom& g, hipSt
             constexpr uint32_t S2 = decltype(B)::value;
             for (uint32_t off = 0; off < nj; off += MAXY) {
                 const uint32_t cnt = nj - off < MAXY ? nj - off : MAXY;
-                k_tensor_ib<S2, RM><<<dim3(g.n / NTT_TILE, cnt), NTT_THREADS, (size_t)NTT_TILE_PADDED * 8, s>>>(d, off, g);
+                k_tensor_ib<S2, RM><<<dim3(g.n / NTT_TILE, cnt), NTT_THREADS, (size_t)padded(NTT_TILE) * 8, s>>>(d, off, g);
             }
         });
         if (!geom_ok) throw std::runtime_error("gpufhe: unsupported ring dimension for the NTT");

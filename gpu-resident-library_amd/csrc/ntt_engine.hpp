@@ -104,17 +104,32 @@ inline uint64_t lazy_red_of(uint64_t q) {
 struct NttGeom {
     uint32_t n, logn;
     uint32_t logN1, logN2;  // phase A covers logN1 stages, phase B logN2
-    uint32_t C;             // columns per phase-A tile
+    uint32_t C;             // columns per phase-A tile of NTT_TILE
     uint32_t R;             // rows per phase-B tile
     uint32_t single;        // 1: whole tower in one tile
     uint32_t rmax;          // largest register radix log2 (tuning knob, 2..4)
 };
 
-enum { NTT_LOG_TILE = 12, NTT_TILE = 1 << NTT_LOG_TILE, NTT_SINGLE_MAX = 4096, NTT_THREADS = 256 };
+// Tiles of 1024 elements.  A row pass needs nothing larger (its rows are
+// contiguous): the smaller tile keeps 8.5 KiB of LDS and short register
+// passes, so more workgroups share a CU and a single operation's few towers
+// spread over 4 times as many CUs as with 4096 (the epilogue row pass of 4
+// towers at n = 2^14: 12.2 -> 7.9 us; of 2944 towers at n = 2^16: unchanged, at
+// the copy rate).  A column pass of a launch that fills the chip takes
+// 4096-element tiles (NTT_LOG_TILE_COLS): their rows of 2^(12 - S1) words are
+// whole L2 lines at n = 2^16 (column passes of 8 operations at L = 24, dnum = 2:
+// 1390 us a pass with them, 1677 with 1024).
+enum {
+    NTT_LOG_TILE = 10,
+    NTT_TILE = 1 << NTT_LOG_TILE,
+    NTT_LOG_TILE_COLS = 12,
+    NTT_SINGLE_MAX = 4096,
+    NTT_THREADS = 256
+};
 
 // row-tile padding: one spare word every 16, so strided radix units hit distinct LDS banks
 GF_HD constexpr uint32_t padded(uint32_t k) { return k + (k >> 4); }
-enum { NTT_TILE_PADDED = NTT_TILE + NTT_TILE / 16 };
+enum { NTT_TILE_PADDED = NTT_SINGLE_MAX + NTT_SINGLE_MAX / 16 };   // LDS words that any tile fits
 
 inline NttGeom make_geom(uint32_t n, uint32_t rmax = 3) {
     NttGeom g{};
@@ -495,11 +510,11 @@ struct ColOut {
     }
 };
 
-// Phase A: tile = columns [b0, b0+C) x all N1 = 2^S1 rows.
-template <bool FWD, bool LZ, bool PAIRED, uint32_t S1, uint32_t RM, class Sync>
+// Phase A: tile = columns [b0, b0+C) x all N1 = 2^S1 rows (2^LOGT elements).
+template <bool FWD, bool LZ, bool PAIRED, uint32_t S1, uint32_t RM, class Sync, uint32_t LOGT = NTT_LOG_TILE>
 GF_HD void phaseA_body(const NttJob& j, const NttGeom& g, uint32_t tile, uint64_t* lds,
                        uint32_t tid, uint32_t nthr, Sync sync) {
-    constexpr uint32_t logC = NTT_LOG_TILE - S1, C = 1u << logC;
+    constexpr uint32_t logC = LOGT - S1, C = 1u << logC;
     const uint32_t b0 = tile * C;
     const TileDesc d{logC, C, 1, 1, 0, true, false};
     // forward: phase A is the first phase (reads in); inverse: the second

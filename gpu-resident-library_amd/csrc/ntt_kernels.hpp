@@ -42,13 +42,13 @@ __device__ __forceinline__ void with_lz(const NttJob& j, F&& f) {
     }
 }
 
-template <bool FWD, bool PAIRED, uint32_t S1, uint32_t RM, class J>
+template <bool FWD, bool PAIRED, uint32_t S1, uint32_t RM, uint32_t LOGT, class J>
 __global__ __launch_bounds__(NTT_THREADS) void k_ntt_A(J jobs, NttGeom g) {
     extern __shared__ uint64_t lds[];
     const NttJob j = jobs.get(blockIdx.y);
     with_lz<FWD>(j, [&](auto L) {
-        phaseA_body<FWD, decltype(L)::value, PAIRED, S1, RM>(j, g, blockIdx.x, lds, threadIdx.x, blockDim.x,
-                                                             DevSync{});
+        phaseA_body<FWD, decltype(L)::value, PAIRED, S1, RM, DevSync, LOGT>(j, g, blockIdx.x, lds, threadIdx.x,
+                                                                            blockDim.x, DevSync{});
     });
 }
 template <bool FWD, bool PAIRED, uint32_t S2, uint32_t RM, class J>
@@ -76,6 +76,13 @@ __global__ __launch_bounds__(NTT_THREADS) void k_ntt_S(J jobs) {
     });
 }
 
+// A column pass of at least this many workgroups of 4096-element tiles takes
+// those tiles, a smaller one 1024-element tiles (four times the workgroups).
+// Measured with the line at 128, 512 and 2048: a keyswitch of 17 towers at
+// n = 2^16 with its launches' sequence 266, 279, 278 us; 16 operations at
+// n = 2^14, L = 16, dnum = 2: 406, 406, 429 us; larger ones alike.
+enum { NTT_COLS_WGS = 128 };
+
 // PAIRED: library plans use interleaved (w, Shoup precon) tables; the
 // reference ABI launchers take the two arrays separately.  g.rmax selects the
 // register radix (the tuning knob the autotuner sets).
@@ -94,15 +101,27 @@ inline void ntt_dispatch_dir(J jobs, uint32_t njobs, const NttGeom& g, hipStream
         } else {
             geom_ok = with_split(g.logN1, g.logN2, [&](auto A, auto B) {
                 constexpr uint32_t S1 = decltype(A)::value, S2 = decltype(B)::value;
-                const dim3 gA((1u << S2) / g.C, njobs), gB((1u << S1) / g.R, njobs);
-                const size_t shA = (size_t)NTT_TILE * 8, shB = (size_t)NTT_TILE_PADDED * 8;
+                const dim3 gB((1u << S1) / g.R, njobs);
+                const size_t shB = (size_t)padded(NTT_TILE) * 8;
+                // the column pass takes large tiles where they fill the chip
+                auto run_A = [&] {
+                    auto go = [&](auto T) {
+                        constexpr uint32_t LOGT = decltype(T)::value;
+                        k_ntt_A<FWD, PAIRED, S1, RM, LOGT>
+                            <<<dim3(g.n >> LOGT, njobs), thr, (size_t)8 << LOGT, s>>>(jobs, g);
+                    };
+                    if ((uint64_t)njobs * (g.n >> NTT_LOG_TILE_COLS) >= NTT_COLS_WGS)
+                        go(std::integral_constant<uint32_t, NTT_LOG_TILE_COLS>{});
+                    else
+                        go(std::integral_constant<uint32_t, NTT_LOG_TILE>{});
+                };
                 // which: bit 0 = first kernel of the transform, bit 1 = second
                 if (FWD) {
-                    if (which & 1) k_ntt_A<FWD, PAIRED, S1, RM><<<gA, thr, shA, s>>>(jobs, g);
+                    if (which & 1) run_A();
                     if (which & 2) k_ntt_B<FWD, PAIRED, S2, RM><<<gB, thr, shB, s>>>(jobs, g);
                 } else {
                     if (which & 1) k_ntt_B<FWD, PAIRED, S2, RM><<<gB, thr, shB, s>>>(jobs, g);
-                    if (which & 2) k_ntt_A<FWD, PAIRED, S1, RM><<<gA, thr, shA, s>>>(jobs, g);
+                    if (which & 2) run_A();
                 }
             });
         }

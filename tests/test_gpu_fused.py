@@ -136,3 +136,18 @@ def test_uneven_batch_in_one_launch(G, n, L, dnum, split):
         for j, w in enumerate(P.rotate_hoisted(lv, c[i][0], c[i][1], ks, t.hk)):
             x = h[2 * i + j]
             assert np.array_equal(x[0].download(), w[0]) and np.array_equal(x[1].download(), w[1]), ("hoist", lv, j)
+
+
+@pytest.mark.parametrize("n,L,dnum", [(1 << 13, 6, 2), (1 << 14, 5, 1), (1 << 16, 9, 1), (1 << 17, 4, 1)])
+def test_column_pass_tiles(G, n, L, dnum):
+    """Whole transforms (fused ModUp and ModDown off) in launches on both sides
+    of the column tile's line: a few towers, and enough to fill the chip."""
+    t = Setup(G, n, L, dnum, modup_fused=0, moddown_fused=0)
+    ws = t.ctx.workspace()
+    for level in (1, L):
+        d = t.ct(level)
+        w = t.P.keyswitch(level, d, *t.hk[0])
+        x, b0, b1 = G.Dev.of(d), G.Dev(level * n), G.Dev(level * n)
+        G.check(G.lib.gf_keyswitch(t.ctx.h, t.keys[0].h, level, x.ptr, b0.ptr, b1.ptr, ws.ptr, t.s.s))
+        t.s.sync()
+        assert np.array_equal(b0.download(), w[0]) and np.array_equal(b1.download(), w[1]), level
