@@ -80,6 +80,19 @@ def step_bytes(n, L, K, alpha, np_parts, kinds, batch):
     by a fused transform epilogue)."""
     T = 8 * n
     key = 2 * np_parts / batch   # key rows read per tower row, per op
+    # the Q rows' inner products in the launch that runs the outputs' row
+    # passes: the digits, keys, ModDown column passes and tensor towers in, the
+    # outputs out, no accumulators; the P rows (and the dropped tower's, with
+    # t's two towers in) store their inverse transforms' row passes
+    if kinds[-1] == "ksi":
+        up, dn = kinds.index("modup"), kinds.index("moddown")
+        assert list(kinds[up + 1:]) == ["ksi", "moddown", "ksi"], kinds
+        full = {name: (b, e) for name, b, e in
+                step_bytes(n, L, K, alpha, np_parts, list(kinds[:up + 1]) + ["ksi", "ksi", "moddown", "ntt_fwd_b"], batch)}
+        head = [(k, *v) for k, v in full.items() if k in ("tensor", "intt_modup_rowpass", "tensor_intt_rowpass", "modup_fused")]
+        return head + [("rowpass_inner_p_drop", T * K * (np_parts + key + 2) + T * (np_parts + key + 2 + 2), 0),
+                       ("moddown_fused", *full["moddown_fused"]),
+                       ("rowpass_inner_q_final", T * (L - 1) * (np_parts + key + 2 + 2 + 2), 0)]
     # the dropped tower's inverse transform inside the other steps: one per
     # component, of t + res / P, its row pass in the Q rows' inner product (t's
     # two towers in, two out; the accumulators' stay on chip) and its column
@@ -775,8 +788,8 @@ def main():
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(a / HBM_PEAK_GBS, 4),
                 "traffic": read_traffic(k["stage"] + ":" + k["kernel"], B), "algorithmic_bytes": k["bytes"],
                 "launch_ms": round(k["ms"], 4)}
-    # the keyswitch kernel on its own: the Q rows' fused row pass + inner product
-    ksi_q = [k for k in kernels if k["stage"] == "rowpass_inner_q"]
+    # the keyswitch kernel on its own: the Q rows' fused row pass + inner product (and their last step)
+    ksi_q = [k for k in kernels if k["stage"] in ("rowpass_inner_q", "rowpass_inner_q_final")]
     roofline_ksi = roofline_of(ksi_q[0]) if ksi_q else None
     # the whole operation against HBM: compulsory bytes per EvalMult+Rescale
     # (inputs 4L and outputs 2(L - 1) towers once, the key's 2 dnum (L + K)

@@ -418,12 +418,13 @@ void Ctx::set_knob(const std::string& name, uint32_t v) {
         if (v > 1) throw std::runtime_error("gpufhe: modup_fused must be 0 or 1");
         modup_fused = v;
     } else if (name == "modup_f64" || name == "ksi_f64" || name == "moddown_fused" || name == "tensor_ib" ||
-               name == "ksi_rowpass") {
+               name == "ksi_rowpass" || name == "ksi_fin") {
         if (v > 1) throw std::runtime_error("gpufhe: " + name + " must be 0 or 1");
         (name == "modup_f64"     ? modup_f64
          : name == "ksi_f64"     ? ksi_f64
          : name == "tensor_ib"   ? tensor_ib
          : name == "ksi_rowpass" ? ksi_rowpass
+         : name == "ksi_fin"     ? ksi_fin
                                  : moddown_fused) = v;
     } else if (name == "modup_min_wgs") {
         modup_min_wgs = v;
@@ -446,6 +447,7 @@ uint32_t Ctx::knob(const std::string& name) const {
     if (name == "tensor_ib") return tensor_ib;
     if (name == "ksi_rowpass") return ksi_rowpass;
     if (name == "moddown_fused") return moddown_fused;
+    if (name == "ksi_fin") return ksi_fin;
     if (name == "modup_min_wgs") return modup_min_wgs;
     if (name == "modup_split_wgs") return modup_split_wgs;
     if (name == "rechunk_wgs") return rechunk_wgs;
@@ -916,7 +918,9 @@ void Plan::run_jobs(size_t i, hipStream_t s, uint32_t which, uint32_t first, uin
         case Step::RSV: launch_rs(GF_J(RsJob), cnt, n, s); break;
         case Step::PTACC: launch_ptacc(GF_J(PtAccJob), cnt, n, s); break;
         case Step::NTT_FA: launch_ntt(GF_J(NttJob), cnt, geom, true, s, 1); break;
-        case Step::KSI: launch_ksi(GF_J(KsiJob), cnt, geom, st.arg & 0xFF, st.arg >> 8, s); break;
+        case Step::KSI:
+            launch_ksi(GF_J(KsiJob), cnt, geom, st.arg & 0xFF, st.arg >> 8 & 0xFF, st.arg >> 16, s);
+            break;
         case Step::NTT_IB: launch_ntt(GF_J(NttJob), cnt, geom, false, s, 1); break;
         case Step::MODUP: launch_modup(GF_J(ModupJob), cnt, geom, st.arg, s); break;
         case Step::MODDOWN: launch_moddown(GF_J(ModupJob), cnt, geom, st.arg & 0xff, s); break;
@@ -948,6 +952,7 @@ void Plan::run_graph(hipStream_t s) {
 // for all of its targets, so large chunks save work; a stage with few jobs
 // is split back into small chunks at layout (split_chunks) to fill the chip.
 static const uint32_t CONV_CHUNK_SMALL = 8;
+static const size_t KSI_JOIN = 1024;
 
 // Re-chunk conversion jobs ([j0, j1) target ranges) into CONV_CHUNK_SMALL
 // pieces when the stage would launch fewer than min_wgs workgroups
@@ -992,13 +997,13 @@ static void split_targets(std::vector<ModupJob>& v, uint32_t n, uint32_t min_wgs
 void PlanBuilder::keyswitch_core(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws,
                                  const uint64_t* extra0, const uint64_t* extra1, uint64_t* dx0,
                                  uint64_t* dx1, uint32_t lazy_rows, bool p_rowpass, const uint64_t* drop0,
-                                 const uint64_t* drop1, uint64_t* dr) {
+                                 const uint64_t* drop1, uint64_t* dr, uint64_t gk) {
     const Ctx& C = C_;
     if (l < 1 || l > C.L) throw std::runtime_error("gpufhe: bad level");
     if (key.nparts < C.lv[l].np) throw std::runtime_error("gpufhe: key has too few parts for this level");
     if (use_ksi(l)) {
-        modup(l, d, ws, extra0, extra1, dx0, dx1, true);
-        ksi_moddown_src(l, d, key, ws, lazy_rows, p_rowpass, drop0, drop1, dr);
+        modup(l, d, ws, extra0, extra1, dx0, dx1, true, gk);
+        ksi_moddown_src(l, d, key, ws, lazy_rows, p_rowpass, drop0, drop1, dr, gk);
         return;
     }
     modup(l, d, ws, extra0, extra1, dx0, dx1);
@@ -1022,6 +1027,96 @@ bool PlanBuilder::use_moddown() const {
            C_.n % MODUP_TILE == 0;
 }
 
+// a rotation reads its inputs through the automorphism where the fused inner
+// product and the fused ModDown run
+bool PlanBuilder::use_gather(uint32_t l) const { return use_ksi(l) && use_moddown(); }
+
+// Whether a tower that the last steps read overlaps one that they write (an
+// operation in place, or one operation's output as another's input): those
+// steps then need everything they read to be copies of the plan's own.
+bool PlanBuilder::late_overlap() const {
+    if (late_reads_.empty() || late_writes_.empty()) return false;
+    std::vector<Span> w = late_writes_;
+    std::sort(w.begin(), w.end(), [](const Span& a, const Span& b) { return a.p < b.p; });
+    const uint64_t* end = nullptr;   // the largest end among the writes up to each
+    std::vector<const uint64_t*> ends(w.size());
+    for (size_t i = 0; i < w.size(); ++i) ends[i] = end = std::max(end, w[i].p + w[i].words);
+    for (const Span& r : late_reads_) {
+        // the writes that start before the read's end
+        const size_t k = std::lower_bound(w.begin(), w.end(), r.p + r.words,
+                                          [](const Span& a, const uint64_t* b) { return a.p < b; }) - w.begin();
+        if (k && ends[k - 1] > r.p) return true;
+    }
+    return false;
+}
+
+// The rotation r from permuted copies of its inputs, made before anything is
+// written, instead of reads through the automorphism
+void PlanBuilder::permute_first(const RotSrc& r) {
+    const Ctx& C = C_;
+    const size_t n = C.n;
+    std::vector<NttJob>& ib = use_modup() ? intt_upb_ : intt_up_;
+    for (uint32_t i = 0; i < r.l; ++i) {
+        const size_t o = i * n;
+        perm_.push_back(PermJob{r.c0 + o, r.a0 + o, r.k});
+        ntt_vb_[r.vb0 + i].e1 = r.a0 + o;
+        ntt_vb_[r.vb0 + i].gk = 0;
+        if (!r.c1) continue;
+        perm_.push_back(PermJob{r.c1 + o, r.a1 + o, r.k});
+        ib[r.ib0 + i].in = r.a1 + o;
+        ib[r.ib0 + i].gk = 0;
+        ksi_[r.ksi0 + i].src[i / C.alpha] = r.a1 + o;
+    }
+    ModdownSrc& m = ksdown_src_[r.ks0];
+    m.t = r.a0;
+    m.gk = 0;
+    if (r.c1)
+        for (uint32_t i = 0; i < r.l + C.K; ++i) ksi_[r.ksi0 + i].gk = 0;
+}
+
+// The Q rows of every fused keyswitch take their last step (the output's row
+// pass and sums) in the launch that forms their inner products: the
+// accumulators' Q rows and a launch less
+// (res written and read again: 64 EvalMult+Rescale at n = 2^16, L = 24 7690 ->
+// 7570 us, 64 hoisted rotations at level 20 3150 -> 2900, one operation 228 ->
+// 205).  Below KSI_JOIN workgroups the stages are bound by their launches, not
+// their traffic, and every inner product shares one launch before the ModDown
+// instead (one multiply at 3 towers, n = 2^14: 51 us apart, 55 together).
+void PlanBuilder::finish_rows() {
+    size_t rows = 0;
+    for (const FinSrc& f : fin_src_) rows += f.rows;
+    if (rows * (C_.n / KSI_TILE) < KSI_JOIN) return;
+    std::vector<char> ku(ksi_.size(), 0), vu(ntt_vb_.size(), 0);
+    for (const FinSrc& f : fin_src_)
+        for (uint32_t i = 0; i < f.rows; ++i) {
+            KsiJob J = ksi_[f.ksi0 + i];
+            if (__builtin_popcount(J.xf) + 2 > KSI_MAXP) continue;
+            const NttJob* vb[2] = {&ntt_vb_[f.vb0 + i], &ntt_vb_[f.vb0 + f.rows + i]};
+            KsiFin& F = J.fin;
+            for (int c = 0; c < 2; ++c) {
+                F.v[c] = F.o[c] = vb[c]->out;
+                F.e[c] = vb[c]->e1;
+                J.pairs &= aligned16({F.v[c], F.e[c]});
+            }
+            F.ci = vb[0]->c0;
+            F.cip = vb[0]->c0p;
+            F.ce = vb[0]->c1;
+            F.cep = vb[0]->c1p;
+            F.e_plain = vb[0]->e1_plain;
+            ksi_fin_.push_back(J);
+            ku[f.ksi0 + i] = 1;
+            vu[f.vb0 + i] = vu[f.vb0 + f.rows + i] = 1;
+        }
+    auto keep = [](auto& v, const std::vector<char>& used) {
+        size_t k = 0;
+        for (size_t i = 0; i < v.size(); ++i)
+            if (!used[i]) v[k++] = v[i];
+        v.resize(k);
+    };
+    keep(ksi_, ku);
+    keep(ntt_vb_, vu);
+}
+
 // 3b-5. The digits' row pass fused with the inner product over Q_l P
 // (src/keyswitch_resident.cpp:171-200), into the workspace accumulators;
 // then their P towers to coefficient form (ModDown's sources), as
@@ -1030,12 +1125,12 @@ bool PlanBuilder::use_moddown() const {
 // rowpass_in_ksi).
 void PlanBuilder::ksi_moddown_src(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws,
                                   uint32_t lazy_rows, bool p_rowpass, const uint64_t* drop0, const uint64_t* drop1,
-                                  uint64_t* dr) {
+                                  uint64_t* dr, uint64_t gk, const uint64_t* hoisted) {
     const Ctx& C = C_;
     const uint32_t n = C.n, K = C.K, W = l + K;
     const LevelConst& lv = C.lv[l];
     const WsLayout w = WsLayout::make(C);
-    const uint64_t* dig = ws + w.dig * n;
+    const uint64_t* dig = hoisted ? hoisted : ws + w.dig * n;
     uint64_t* res[2] = {ws + w.res0 * n, ws + w.res1 * n};
     uint64_t* xp = ws + w.xp * n;
     for (uint32_t i = 0; i < W; ++i) {
@@ -1043,11 +1138,13 @@ void PlanBuilder::ksi_moddown_src(uint32_t l, const uint64_t* d, const DevKey& k
         const uint32_t krow = i < l ? i : key.fullQ + (i - l);
         KsiJob J{};
         J.np = lv.np;
+        J.gk = (uint32_t)gk;
+        J.glog = C.logn;
         for (uint32_t pi = 0; pi < lv.np; ++pi) {
             const PartConst& P = lv.parts[pi];
             const bool own = i >= P.st && i < P.st + P.sp;
             J.src[pi] = digit_tower(l, d, dig, pi, i);
-            if (!own) J.xf |= 1u << pi;
+            if (!own && !hoisted) J.xf |= 1u << pi;
             const size_t ko = ((size_t)pi * key.rows + krow) * n;
             J.kb[pi] = key.b.as<uint64_t>() + ko;
             J.ka[pi] = key.a.as<uint64_t>() + ko;
@@ -1095,7 +1192,7 @@ void PlanBuilder::ksi_moddown_src(uint32_t l, const uint64_t* d, const DevKey& k
 // 1-3. ModUp of d into the workspace digits (eval form); extra towers (the
 // last tower of t0/t1 in the fused EvalMult+Rescale) ride along the INTT.
 void PlanBuilder::modup(uint32_t l, const uint64_t* d, uint64_t* ws, const uint64_t* extra0,
-                        const uint64_t* extra1, uint64_t* dx0, uint64_t* dx1, bool rowpass_in_ksi) {
+                        const uint64_t* extra1, uint64_t* dx0, uint64_t* dx1, bool rowpass_in_ksi, uint64_t gk) {
     const Ctx& C = C_;
     const uint32_t n = C.n, K = C.K, W = l + K;
     const LevelConst& lv = C.lv[l];
@@ -1108,9 +1205,11 @@ void PlanBuilder::modup(uint32_t l, const uint64_t* d, uint64_t* ws, const uint6
     // 1. part towers to coefficient form, scaled by n^-1 QHatInv (ModUp's first factor)
     for (uint32_t i = 0; i < l; ++i) {
         const uint32_t pi = i / C.alpha, ii = i - pi * C.alpha;
-        (fuse ? intt_upb_ : intt_up_)
-            .push_back(NttJob{d + (size_t)i * n, x + (size_t)i * n, C.rt[i].iv2, nullptr, C.mods[i],
-                              lv.parts[pi].post[ii], lv.parts[pi].postp[ii]});
+        NttJob J{d + (size_t)i * n, x + (size_t)i * n, C.rt[i].iv2, nullptr, C.mods[i], lv.parts[pi].post[ii],
+                 lv.parts[pi].postp[ii]};
+        J.gk = (uint32_t)gk;
+        J.glog = C.logn;
+        (fuse ? intt_upb_ : intt_up_).push_back(J);
     }
     const uint64_t* ex[2] = {extra0, extra1};
     uint64_t* dx[2] = {dx0, dx1};
@@ -1234,18 +1333,23 @@ void PlanBuilder::inner_moddown_src(uint32_t l, const DevKey& key, uint64_t* ws,
 
 void PlanBuilder::keyswitch(uint32_t l, const uint64_t* d, uint64_t* ba0, uint64_t* ba1,
                             const DevKey& key, uint64_t* ws, const uint64_t* t0,
-                            const uint64_t* t1) {
+                            const uint64_t* t1, uint64_t gk) {
     // with the fused ModDown the accumulators' Q rows only feed its
     // epilogue's lazy Shoup products
     const bool fmd = use_moddown();
-    keyswitch_core(l, d, key, ws, nullptr, nullptr, nullptr, nullptr, fmd ? l : 0, fmd);
-    moddown_tail(l, ws, ba0, ba1, t0, t1);
+    const FinSrc f{ksi_.size(), ntt_vb_.size(), l};
+    keyswitch_core(l, d, key, ws, nullptr, nullptr, nullptr, nullptr, fmd ? l : 0, fmd, nullptr, nullptr, nullptr, gk);
+    moddown_tail(l, ws, ba0, ba1, t0, t1, gk);
+    if (fmd && use_ksi(l)) {
+        fin_src_.push_back(f);
+        late_reads_.push_back(Span{d, (size_t)l * C_.n});   // the input's own digits
+    }
 }
 
 // 6-8. ApproxModDown of both workspace accumulators, fused with
 // out_c = t_c + ba_c (src/keyswitch_resident.cpp:203-224)
 void PlanBuilder::moddown_tail(uint32_t l, uint64_t* ws, uint64_t* ba0, uint64_t* ba1, const uint64_t* t0,
-                               const uint64_t* t1) {
+                               const uint64_t* t1, uint64_t gk) {
     const Ctx& C = C_;
     const uint32_t n = C.n, K = C.K;
     const WsLayout w = WsLayout::make(C);
@@ -1257,7 +1361,7 @@ void PlanBuilder::moddown_tail(uint32_t l, uint64_t* ws, uint64_t* ba0, uint64_t
     const bool fmd = use_moddown();
     for (int c = 0; c < 2; ++c)
         ks_tail(ModdownSrc{l, (uint32_t)c, xp + (size_t)c * K * n, nullptr, nullptr, ts[c], res[c],
-                           conv + (size_t)c * l * n, outs[c], true},
+                           conv + (size_t)c * l * n, outs[c], true, false, gk},
                 fmd);
 }
 
@@ -1311,8 +1415,12 @@ void PlanBuilder::ks_tail(const ModdownSrc& m, bool fused) {
             T.c0p = lv.pinvp[i];
             T.e1 = m.t ? m.t + (size_t)i * n : nullptr;
             T.e1_plain = 1;
+            T.gk = (uint32_t)m.gk;
+            T.glog = C.logn;
             ntt_vb_.push_back(T);
         }
+        late_writes_.push_back(Span{m.out, (size_t)l * n});
+        if (m.gk && m.t) late_reads_.push_back(Span{m.t, (size_t)l * n});
         return;
     }
     for (uint32_t j0 = 0; j0 < l; j0 += C.conv_chunk)
@@ -1355,6 +1463,7 @@ void PlanBuilder::evalmult_rescale_fused(uint32_t l, const uint64_t* c0a, const 
     // n = 2^16, L = 24; 38 of 293 us for one).
     const uint64_t* tl[2] = {t[0] + (size_t)last * n, t[1] + (size_t)last * n};
     const bool drop = fmd && use_ksi(l) && C.ksi_rowpass;
+    const FinSrc f{ksi_.size(), ntt_vb_.size(), last};
     // accumulator rows below `last` only feed the epilogue's lazy Shoup products
     if (drop) keyswitch_core(l, t[2], key, ws, nullptr, nullptr, nullptr, nullptr, last, true, tl[0], tl[1], dr);
     else keyswitch_core(l, t[2], key, ws, tl[0], tl[1], dt, dt + n, last, fmd);
@@ -1370,6 +1479,7 @@ void PlanBuilder::evalmult_rescale_fused(uint32_t l, const uint64_t* c0a, const 
                            t[c], res[c], v + (size_t)c * last * n, outs[c], false, drop};
         rescale_tail(m, fmd);
     }
+    if (drop) fin_src_.push_back(f);
 }
 
 // The rescale tail of one component: from the K P towers (coefficient form,
@@ -1383,6 +1493,7 @@ void PlanBuilder::rescale_tail(const ModdownSrc& m, bool fused) {
         ModupJob J{};
         moddown_sources(J, lv, m.xp);
         J.dst = m.out;   // surviving tower i's column-pass output at out + i n
+        late_writes_.push_back(Span{m.out, (size_t)last * n});
         J.tab = lv.d_tabRS;
         J.sc = last;
         J.dt = m.dt;
@@ -1439,12 +1550,12 @@ void PlanBuilder::rescale_tail(const ModdownSrc& m, bool fused) {
         // fused: the column pass is done, this row pass reads and writes out
         NttJob J{fused ? m.out + (size_t)i * n : m.vc + (size_t)i * n, m.out + (size_t)i * n, C.rt[i].fw2, nullptr,
                  C.mods[i], 0, 0};
-        J.e0 = m.t + (size_t)i * n;
-        J.c0 = lv.s1[i];
-        J.c0p = lv.s1p[i];
-        J.e1 = m.res + (size_t)i * n;
-        J.c1 = lv.ps1[i];
-        J.c1p = lv.ps1p[i];
+        J.e0 = m.res + (size_t)i * n;
+        J.c0 = lv.ps1[i];
+        J.c0p = lv.ps1p[i];
+        J.e1 = m.t + (size_t)i * n;
+        J.c1 = lv.s1[i];
+        J.c1p = lv.s1p[i];
         (fused ? ntt_vb_ : ntt_v_).push_back(J);
     }
 }
@@ -1524,6 +1635,15 @@ void PlanBuilder::rotate(uint32_t l, uint64_t k, const uint64_t* c0, const uint6
     const WsLayout w = WsLayout::make(C);
     uint64_t* a0 = ws + w.t0 * n;
     uint64_t* a1 = ws + w.t2 * n;
+    if (l >= 1 && l <= C.L && use_gather(l)) {
+        // every step that reads c0 or c1 reads it through the automorphism:
+        // no permuted copies (310 of 4340 us for 64 rotations at levels 8..20,
+        // n = 2^16)
+        rot_src_.push_back(RotSrc{l, k, c0, c1, a0, a1, use_modup() ? intt_upb_.size() : intt_up_.size(), ksi_.size(),
+                                  ntt_vb_.size(), ksdown_src_.size()});
+        keyswitch(l, c1, o0, o1, key, ws, c0, nullptr, k);
+        return;
+    }
     for (uint32_t i = 0; i < l; ++i) {
         const size_t o = (size_t)i * n;
         perm_.push_back(PermJob{c0 + o, a0 + o, k});
@@ -1554,6 +1674,15 @@ void PlanBuilder::rotate_hoisted(uint32_t l, uint32_t m, const uint64_t* ks, con
     for (uint32_t j = 0; j < m; ++j) {
         uint64_t* ws = ws_rot[j];
         uint64_t* a0 = ws + w.t0 * n;
+        if (use_gather(l)) {
+            // as a rotation's, over the shared digits
+            rot_src_.push_back(RotSrc{l, ks[j], c0, nullptr, a0, nullptr, 0, ksi_.size(), ntt_vb_.size(), ksdown_src_.size()});
+            fin_src_.push_back(FinSrc{ksi_.size(), ntt_vb_.size(), l});
+            ksi_moddown_src(l, c1, *keys[j], ws, l, true, nullptr, nullptr, nullptr, ks[j], dig);
+            moddown_tail(l, ws, o0[j], o1[j], c0, nullptr, ks[j]);
+            late_reads_.push_back(Span{c1, (size_t)l * n});
+            continue;
+        }
         for (uint32_t i = 0; i < l; ++i) perm_.push_back(PermJob{c0 + (size_t)i * n, a0 + (size_t)i * n, ks[j]});
         // the inner product reads the shared digits through sigma_k: no permuted copies
         inner_moddown_src(
@@ -1592,7 +1721,7 @@ void PlanBuilder::linear_transform(uint32_t l, uint32_t m, const uint64_t* ks, c
             continue;
         }
         uint64_t* ws = ws_rot[j];
-        r0.push_back(ws + w.dig * n);   // not over sigma(c0) (t0), which the ModDown's last stage adds
+        r0.push_back(ws + w.t2 * n);   // not over sigma(c0) (t0), which the ModDown's last stage adds
         r1.push_back(ws + w.t1 * n);
         rk.push_back(ks[j]);
         rkey.push_back(keys[j]);
@@ -1696,6 +1825,9 @@ std::unique_ptr<Plan> PlanBuilder::finish_into(void* d_arena, void* h_stage, siz
 }
 
 std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
+    if ((moddown_.size() + ksdown_.size()) * (C_.n / MODUP_TILE) < C_.modup_min_wgs || late_overlap())
+        for (const RotSrc& r : rot_src_) permute_first(r);
+    else if (C_.ksi_fin) finish_rows();
     // a fused ModUp stage too small to fill the chip runs unfused: the
     // inverse transforms whole, then the conversion and the column passes
     if (!modup_.empty() && modup_.size() * (C_.n / MODUP_TILE) < C_.modup_min_wgs) {
@@ -1755,10 +1887,11 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         for (NttJob& j : *v) j.red = lazy_red_of(j.q);
     for (auto* v : {&ntt_dig_, &ntt_digb_})
         for (NttJob& j : *v) j.lazy_out = j.red != 0;
-    for (KsiJob& j : ksi_) {
-        j.twr = C_.row_table_of(j.tw);
-        if (!j.twr) throw std::runtime_error("gpufhe: transform table of another context");
-    }
+    for (auto* v : {&ksi_, &ksi_fin_})
+        for (KsiJob& j : *v) {
+            j.twr = C_.row_table_of(j.tw);
+            if (!j.twr) throw std::runtime_error("gpufhe: transform table of another context");
+        }
     // with the fused ModDown, a P row's inner product runs the inverse row
     // pass of its two output rows itself (from two LDS regions, ksi_regions),
     // and those row-pass jobs leave their stage
@@ -1785,7 +1918,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     // t2 or a ciphertext tower, are reduced residues), and with ksi_f64 so do
     // the row passes of the fused inner product (the ModUp leaves those
     // digits in [0, 2q)).
-    if (!modup_.empty() && C_.modup_f64 && !C_.geom.single) {
+    if (C_.modup_f64 && !C_.geom.single) {
         auto f64_job = [&](auto& j) {
             const uint64_t* td = C_.f64_table_of(j.tw);
             if (!td) return;
@@ -1794,14 +1927,19 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
             j.fq = (double)j.q;
             j.fqinv = 1.0 / j.fq;
         };
+        // (a last step's rows come from the fused ModDown, in [0, 2q) alike)
         if (C_.ksi_f64)
-            for (KsiJob& j : ksi_) f64_job(j);
-        for (NttJob& j : intt_upb_) f64_job(j);
+            for (auto* v : {&ksi_, &ksi_fin_})
+                for (KsiJob& j : *v)
+                    if (!j.xf || !modup_.empty()) f64_job(j);
+        if (!modup_.empty())
+            for (NttJob& j : intt_upb_) f64_job(j);
     }
-    // KSI jobs by their LDS regions (one step each: that many regions and
-    // waves), by key within a step
-    group_by(ksi_, [](const KsiJob& j) { return (uintptr_t)j.kb[0]; });
-    group_by(ksi_, ksi_regions);
+    // KSI jobs by their LDS regions, most first, by key within a region count
+    for (auto* v : {&ksi_, &ksi_fin_}) {
+        group_by(*v, [](const KsiJob& j) { return (uintptr_t)j.kb[0]; });
+        group_by(*v, [](const KsiJob& j) { return ~ksi_regions(j); });
+    }
     group_by(inner_, [](const InnerJob& j) { return (uintptr_t)j.kb[0]; });
     split_chunks(conv_up_, C_.n, C_.rechunk_wgs);
     split_chunks(conv_dn_, C_.n, C_.rechunk_wgs);
@@ -1871,14 +2009,28 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(NTT_FA, ntt_diga_);
     GF_STAGE(NTT_FB, ntt_digb_);
     GF_STAGE(INNER, inner_);
-    for (size_t i = 0; i < ksi_.size();) {
-        size_t e = i;
-        while (e < ksi_.size() && ksi_regions(ksi_[e]) == ksi_regions(ksi_[i])) ++e;
-        const uint32_t x = ksi_regions(ksi_[i]), waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
-        stage(Step::KSI, ksi_.data() + i, e - i, sizeof(KsiJob));
-        P->steps.back().arg = x | waves << 8;
-        i = e;
-    }
+    // One step per region count, with one wave per region; jobs of fewer
+    // regions join the step before them where they are few (below KSI_JOIN
+    // workgroups, or a quarter of that step's): a launch of their own would not
+    // fill the chip.
+    auto stage_ksi = [&](const std::vector<KsiJob>& v, uint32_t fin) {
+        const size_t tiles = C_.n / KSI_TILE;
+        for (size_t i = 0; i < v.size();) {
+            size_t e = i;
+            const uint32_t x = ksi_regions(v[i]);
+            while (e < v.size()) {
+                size_t g = e;
+                while (g < v.size() && ksi_regions(v[g]) == ksi_regions(v[e])) ++g;
+                if (e > i && (g - e) * tiles >= KSI_JOIN && (g - e) * 4 >= e - i) break;
+                e = g;
+            }
+            const uint32_t waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
+            stage(Step::KSI, v.data() + i, e - i, sizeof(KsiJob));
+            P->steps.back().arg = x | waves << 8 | fin << 16;
+            i = e;
+        }
+    };
+    stage_ksi(ksi_, 0);
     GF_STAGE(NTT_I, intt_p_);
     GF_STAGE(NTT_IB, intt_pb_);
     stage_modup(Step::MODDOWN, moddown_);
@@ -1895,6 +2047,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(RSV, rs_);
     GF_STAGE(NTT_F, ntt_v_);
     GF_STAGE(NTT_FB, ntt_vb_);
+    stage_ksi(ksi_fin_, 1);
     GF_STAGE(ADD, add_);
     GF_STAGE(COPY, copy_);
     GF_STAGE(PTACC, ptacc_);

@@ -160,6 +160,9 @@ public:
     // one kernel (the fused ModUp kernel's rescale mode), where the fused
     // ModUp runs; stages below modup_min_wgs workgroups run them apart
     uint32_t moddown_fused = 1;
+    // 1: with the fused ModDown, the Q rows' inner products run in the launch
+    // that runs the outputs' row passes (KsiFin)
+    uint32_t ksi_fin = 1;
     // a plan whose fused ModUp (or ModDown) stage would launch fewer workgroups
     // than this runs it unfused
     uint32_t modup_min_wgs = 0;
@@ -178,7 +181,7 @@ public:
     std::string tune_report;
     // sets or reads a knob by name ("ntt_radix", "ksi_extra", "conv_chunk",
     // "rs_chunk", "modup_fused", "modup_f64", "ksi_f64", "moddown_fused", "tensor_ib", "ksi_rowpass",
-    // "modup_min_wgs", "modup_split_wgs", "rechunk_wgs")
+    // "ksi_fin", "modup_min_wgs", "modup_split_wgs", "rechunk_wgs")
     void set_knob(const std::string& name, uint32_t v);
     uint32_t knob(const std::string& name) const;
     std::string radix_report;   // the radix search of autotune(), as JSON
@@ -223,8 +226,8 @@ struct Step {
                 NTT_FA, KSI, NTT_IB, MODUP, MODDOWN, NTT_FB, TENSOR_IB, KSDOWN } kind;
     size_t off;     // byte offset of the first job in the plan's device buffer
     uint32_t count;
-    // KSI: LDS regions (bits 0-7) and waves per workgroup (bits 8-15); the
-    // jobs of one KSI step share their transformed-part count
+    // KSI: the jobs' largest LDS region count (bits 0-7), waves per workgroup
+    // (bits 8-15), 1 << 16 where the jobs have a last step (KsiFin)
     uint32_t arg = 0;
 };
 
@@ -254,8 +257,10 @@ class PlanBuilder {
 public:
     explicit PlanBuilder(const Ctx& C) : C_(C) {}
     // per-op recipes (all buffers are device pointers, tower-major)
+    // t0, t1: added to ba0, ba1 (may be null).  gk: d and t0 are read through
+    // the automorphism gk (use_gather)
     void keyswitch(uint32_t l, const uint64_t* d, uint64_t* ba0, uint64_t* ba1, const DevKey& key,
-                   uint64_t* ws, const uint64_t* t0 = nullptr, const uint64_t* t1 = nullptr);
+                   uint64_t* ws, const uint64_t* t0 = nullptr, const uint64_t* t1 = nullptr, uint64_t gk = 0);
     void evalmult(uint32_t l, const uint64_t* c0a, const uint64_t* c1a, const uint64_t* c0b,
                   const uint64_t* c1b, uint64_t* r0, uint64_t* r1, const DevKey& key, uint64_t* ws);
     void rescale(uint32_t l, const uint64_t* c0, const uint64_t* c1, uint64_t* o0, uint64_t* o1,
@@ -337,10 +342,40 @@ private:
         uint64_t *vc, *out;
         bool ks = false;   // a keyswitch's ModDown (ks_tail), not a rescale's
         bool drop = false; // the dropped tower comes from the inner product's row pass (KsiJob::drop)
+        uint64_t gk = 0;   // t is read through this automorphism
     };
     std::vector<ModdownSrc> moddown_src_;   // what each fused ModDown job computes, to run it apart
     std::vector<ModupJob> ksdown_;          // the fused ModDowns of keyswitches (no dropped tower)
     std::vector<ModdownSrc> ksdown_src_;
+    // rows whose inner products (ksi_ from ksi0) and epilogues (ntt_vb_ from
+    // vb0, component 0 then 1) may run in one launch (KsiFin)
+    struct FinSrc {
+        size_t ksi0, vb0;
+        uint32_t rows;
+    };
+    std::vector<FinSrc> fin_src_;
+    std::vector<KsiJob> ksi_fin_;
+    // a rotation whose steps read c0 (and c1) through the automorphism k; a0
+    // (and a1) hold permuted copies where outputs overlap inputs.  c1, a1
+    // null: a hoisted rotation (its digits are read through k in any case)
+    struct RotSrc {
+        uint32_t l;
+        uint64_t k;
+        const uint64_t *c0, *c1;
+        uint64_t *a0, *a1;
+        size_t ib0, ksi0, vb0, ks0;
+    };
+    std::vector<RotSrc> rot_src_;
+    // towers that a keyswitch's steps read while outputs are written
+    struct Span {
+        const uint64_t* p;
+        size_t words;
+    };
+    std::vector<Span> late_reads_, late_writes_;
+    bool late_overlap() const;
+    void permute_first(const RotSrc& r);
+    bool use_gather(uint32_t l) const;
+    void finish_rows();
     // the rescale tail of one component of the fused EvalMult+Rescale: the
     // prologue and the epilogue transforms (apart), or the fused ModDown and
     // the epilogue's row pass
@@ -364,16 +399,18 @@ private:
     void keyswitch_core(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws,
                         const uint64_t* extra0, const uint64_t* extra1, uint64_t* dx0, uint64_t* dx1,
                         uint32_t lazy_rows = 0, bool p_rowpass = false, const uint64_t* drop0 = nullptr,
-                        const uint64_t* drop1 = nullptr, uint64_t* dr = nullptr);
+                        const uint64_t* drop1 = nullptr, uint64_t* dr = nullptr, uint64_t gk = 0);
+    // gk: d is read through that automorphism
     void modup(uint32_t l, const uint64_t* d, uint64_t* ws, const uint64_t* extra0, const uint64_t* extra1,
-               uint64_t* dx0, uint64_t* dx1, bool rowpass_in_ksi = false);
+               uint64_t* dx0, uint64_t* dx1, bool rowpass_in_ksi = false, uint64_t gk = 0);
     // the digits' row pass fused with the key inner product (two-phase rings,
     // up to KSI_MAXP parts, fused schedule on)
     bool use_ksi(uint32_t l) const;
     bool use_modup() const;
     void modup_unfused(uint32_t l, uint32_t pi, const uint64_t* x, uint64_t* dp, bool colpass_only);
     void ksi_moddown_src(uint32_t l, const uint64_t* d, const DevKey& key, uint64_t* ws, uint32_t lazy_rows,
-                         bool p_rowpass, const uint64_t* drop0, const uint64_t* drop1, uint64_t* dr);
+                         bool p_rowpass, const uint64_t* drop0, const uint64_t* drop1, uint64_t* dr, uint64_t gk,
+                         const uint64_t* hoisted = nullptr);
     const uint64_t* digit_tower(uint32_t l, const uint64_t* d, const uint64_t* dig, uint32_t pi,
                                 uint32_t i) const;
     // gk != 0: the digits are read through the automorphism of index gk
@@ -381,7 +418,7 @@ private:
     void inner_moddown_src(uint32_t l, const DevKey& key, uint64_t* ws, F digit, uint64_t gk = 0,
                            bool p_rowpass = false);
     void moddown_tail(uint32_t l, uint64_t* ws, uint64_t* ba0, uint64_t* ba1, const uint64_t* t0,
-                      const uint64_t* t1);
+                      const uint64_t* t1, uint64_t gk = 0);
     std::vector<PtAccJob> ptacc_;
     std::vector<AddJob> add_;
     std::vector<CopyJob> copy_;

@@ -226,8 +226,9 @@ void launch_ekgen(const EkJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 void launch_dec(const DecJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 void launch_ptacc(const PtAccJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 // fused digit row pass + key inner product: regions = LDS regions (at least every
-// job's transformed-part count), waves = workgroup size in waves (1..KSI_WAVES)
-void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, hipStream_t s);
+// job's ksi_regions), waves = workgroup size in waves (1..KSI_WAVES), fin: every
+// job has a last step, or none has
+void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, bool fin, hipStream_t s);
 void launch_tensor_ib(const TensorIbJob* d, uint32_t nj, const NttGeom& g, hipStream_t s);
 // the fused ModUp over jobs of at most arg & 0xff sources each and of one c60
 // (arg >> 8)

@@ -33,8 +33,23 @@ enum {
     KSI_LOG_TILE = 9,
     KSI_TILE = 1 << KSI_LOG_TILE,                    // positions per workgroup
     KSI_PART_WORDS = KSI_TILE + KSI_TILE / 16,       // one part's padded LDS region
-    KSI_WAVES = 5,                                   // largest workgroup, in waves
+    KSI_WAVES = 7,                                   // largest workgroup, in waves
     KSI_THREADS = 64 * KSI_WAVES
+};
+
+// The last step of an output row of both components c, in the launch that
+// forms its inner products r_c: v[c] is the column-pass output of the ModDown's
+// forward transform; its row pass runs beside the digits' (two more LDS
+// regions, after the parts'), and the row is stored as
+//   o[c] = NTT(v[c]) + r_c ci + e[c] (times ce unless e_plain; e[c] may be null
+//   with e_plain)
+// so the inner products never travel through HBM.
+struct KsiFin {
+    const uint64_t* v[2];
+    uint64_t* o[2];
+    const uint64_t* e[2];
+    uint64_t ci, cip, ce, cep;
+    uint32_t e_plain;
 };
 
 struct KsiJob {
@@ -73,12 +88,17 @@ struct KsiJob {
     // of the dropped tower but for its ModDown conversion
     const uint64_t* drop[2];
     uint64_t dpinv, dpinvp;
+    // parts that are not transformed here (and fin.e with fin.e_plain) are read
+    // through the automorphism of index gk (0: as they are), n = 2^glog
+    uint32_t gk, glog;
+    // fin.v[0] set: the row's last step (KsiFin) instead of o0, o1
+    KsiFin fin;
 };
-// LDS regions of a job: one per transformed part, and two where the row pass
-// takes its outputs
+// LDS regions of a job: one per transformed part, two at least where the row
+// pass takes its outputs, and two more for a last step's row passes
 inline uint32_t ksi_regions(const KsiJob& j) {
     const uint32_t x = (uint32_t)__builtin_popcount(j.xf);
-    return j.rp_on && x < 2 ? 2 : x;
+    return j.fin.v[0] ? x + 2 : j.rp_on && x < 2 ? 2 : x;
 }
 
 // V consecutive words from word i of a tower (V = 2: one 16-byte access; the
@@ -102,6 +122,25 @@ GF_HD void store_words(GF_GLOBAL uint64_t* base, uint32_t i, const uint64_t* in)
     }
 }
 
+// the same at position i of the automorphism gk's image (V = 2: i even; see
+// galois_index)
+template <uint32_t V>
+GF_HD void load_words_gk(const GF_GLOBAL uint64_t* base, uint32_t i, uint32_t gk, uint32_t glog, uint64_t* out) {
+    const uint32_t g = galois_index(i, gk, glog);
+    if constexpr (V == 2) {
+        const Words2 x = gat((const GF_GLOBAL Words2*)base, g / 2);
+        out[0] = g & 1 ? x.w[1] : x.w[0];
+        out[1] = g & 1 ? x.w[0] : x.w[1];
+    } else {
+        out[0] = gat(base, g);
+    }
+}
+template <uint32_t V>
+GF_HD void load_words_any(const GF_GLOBAL uint64_t* base, uint32_t i, const KsiJob& j, uint64_t* out) {
+    if (j.gk) load_words_gk<V>(base, i, j.gk, j.glog, out);
+    else load_words<V>(base, i, out);
+}
+
 // Digits and keys of a row fit the 30-bit column sums when both are below
 // 2^60: keys are residues (< q); digits are residues too, or with red (the
 // forward transform's unreduced values) below 72 q.
@@ -115,8 +154,43 @@ inline uint32_t ksi_d30(uint64_t q, uint64_t red) {
 // slots for the row pass after it; each thread writes only its own
 // positions, whose digits it has already read
 template <uint32_t V>
+struct KsiEps {
+    uint64_t e0[V], e1[V];   // fin.e[c] at the step's positions
+};
+// the last step's operands, requested with the step's other loads
+template <bool FIN, uint32_t V>
+GF_HD void ksi_load_eps(const KsiJob& j, uint32_t gi, KsiEps<V>& x) {
+    if constexpr (FIN) {
+        if (j.fin.e_plain) {
+            if (j.fin.e[0]) load_words_any<V>(gcast(j.fin.e[0]), gi, j, x.e0);
+            if (j.fin.e[1]) load_words_any<V>(gcast(j.fin.e[1]), gi, j, x.e1);
+        } else {
+            load_words<V>(gcast(j.fin.e[0]), gi, x.e0);
+            load_words<V>(gcast(j.fin.e[1]), gi, x.e1);
+        }
+    }
+}
+template <bool FIN, bool LZ, uint32_t V>
 GF_HD void ksi_store(const KsiJob& j, uint64_t* lds, uint32_t idx, uint32_t gi, const uint64_t* r0,
-                     const uint64_t* r1) {
+                     const uint64_t* r1, const KsiEps<V>& x, const NttJob& t) {
+    if constexpr (FIN) {
+        const uint32_t k0 = (uint32_t)__builtin_popcount(j.xf) * KSI_PART_WORDS;
+        auto comp = [&](uint32_t c, const uint64_t* r, const uint64_t* e) {
+            uint64_t y[V];
+            const int ep = !j.fin.e_plain ? 0 : j.fin.e[c] ? 1 : 2;
+#pragma unroll
+            for (uint32_t v = 0; v < V; ++v) {
+                const uint64_t z = lds[k0 + c * KSI_PART_WORDS + padded(idx + v)];
+                y[v] = ep == 0   ? ntt_ep_value<LZ, 0>(z, t, r[v], e[v])
+                       : ep == 1 ? ntt_ep_value<LZ, 1>(z, t, r[v], e[v])
+                                 : ntt_ep_value<LZ, 2>(z, t, r[v], 0);
+            }
+            store_words<V>(gcast(j.fin.o[c]), gi, y);
+        };
+        comp(0, r0, x.e0);
+        comp(1, r1, x.e1);
+        return;
+    }
     if (j.rp_on) {
         uint64_t t0[V], t1[V];
         if (j.drop[0]) {
@@ -157,7 +231,7 @@ GF_HD U128 cols_to_u128(uint64_t lo, uint64_t mid, uint64_t hi) {
 // sums are 30-bit column sums (j.d30): per part and component four 32 x 32
 // multiply-adds with no carries.  NP <= 7 keeps every column below 2^64
 // (lo, hi < 7 2^60; mid < 14 2^60).
-template <uint32_t NP, uint32_t V, bool LZ>
+template <uint32_t NP, uint32_t V, bool LZ, bool FIN>
 GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t tid, uint32_t nthr,
                           const NttJob& t) {
     const GF_GLOBAL uint64_t *src[NP], *kb[NP], *ka[NP];
@@ -181,11 +255,13 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
 #pragma unroll
                 for (uint32_t v = 0; v < V; ++v) dv[p][v] = lds[reg[p] + padded(idx + v)];
             } else {
-                load_words<V>(src[p], gi, dv[p]);
+                load_words_any<V>(src[p], gi, j, dv[p]);
             }
             load_words<V>(kb[p], gi, bv[p]);
             load_words<V>(ka[p], gi, av[p]);
         }
+        KsiEps<V> ep;
+        ksi_load_eps<FIN, V>(j, gi, ep);
         uint64_t r0[V], r1[V];
 #pragma unroll
         for (uint32_t v = 0; v < V; ++v) {
@@ -208,7 +284,7 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
                 h1 = mad32(d1, a1, h1);
             }
             const U128 s0 = cols_to_u128(l0, m0, h0), s1 = cols_to_u128(l1, m1, h1);
-            if (j.lazy_out) {
+            if (FIN || j.lazy_out) {
                 r0[v] = redc_lazy(s0, q, qneg);
                 r1[v] = redc_lazy(s1, q, qneg);
             } else if constexpr (LZ) {
@@ -219,26 +295,26 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
                 r1[v] = redc(s1, q, qneg);
             }
         }
-        ksi_store<V>(j, lds, idx, gi, r0, r1);
+        ksi_store<FIN, LZ, V>(j, lds, idx, gi, r0, r1, ep, t);
     }
 }
 
 // ksi_inner_cols for the job's part count, when it has an instantiation
-template <uint32_t V, bool LZ>
+template <uint32_t V, bool LZ, bool FIN>
 GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t tid, uint32_t nthr,
                              const NttJob& t) {
     switch (j.np) {
-        case 1: ksi_inner_cols<1, V, LZ>(j, lds, off, tid, nthr, t); return true;
-        case 2: ksi_inner_cols<2, V, LZ>(j, lds, off, tid, nthr, t); return true;
-        case 3: ksi_inner_cols<3, V, LZ>(j, lds, off, tid, nthr, t); return true;
-        case 4: ksi_inner_cols<4, V, LZ>(j, lds, off, tid, nthr, t); return true;
+        case 1: ksi_inner_cols<1, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
+        case 2: ksi_inner_cols<2, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
+        case 3: ksi_inner_cols<3, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
+        case 4: ksi_inner_cols<4, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
         default: return false;
     }
 }
 
-// LZ = (j.red != 0).  The wave-level sync wsync separates the row passes of
+// LZ = (j.red != 0), FIN = (j.fin.v[0] != null).  The wave-level sync wsync separates the row passes of
 // one wave's region; bsync is the workgroup barrier before the inner product.
-template <uint32_t S2, uint32_t RM, bool LZ, class WSync, class BSync>
+template <uint32_t S2, uint32_t RM, bool LZ, class WSync, class BSync, bool FIN = false>
 GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, uint32_t wave, uint32_t nwaves,
                     uint32_t lane, uint32_t wlanes, uint32_t tid, uint32_t nthr, WSync wsync, BSync bsync) {
     constexpr uint32_t ROWS = KSI_TILE >> S2, LOGR = KSI_LOG_TILE - S2;
@@ -249,26 +325,41 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
     t.q = j.q;
     t.red = j.red;
     const TileDesc d{LOGR, 1, padded(1u << S2), N1 + a0, 1, false, true};
-    // transformed part k (in part order) -> LDS region k
+    // transformed part k (in part order) -> LDS region k, then a last step's
+    // two components
     uint32_t k = 0;
-    for (uint32_t p = 0; p < j.np; ++p) {
-        if (!((j.xf >> p) & 1)) continue;
+    auto row_pass = [&](const uint64_t* src) {
         if (k % nwaves == wave) {
             if (j.twd)
-                row_tile_f64<true, S2, RM, ROWS, true>(j.twd, j.twrd, j.fq, j.fqinv, d, gcast(j.src[p]), nullptr, off,
+                row_tile_f64<true, S2, RM, ROWS, true>(j.twd, j.twrd, j.fq, j.fqinv, d, gcast(src), nullptr, off,
                                                        lds + k * KSI_PART_WORDS, lane, wlanes, wsync);
             else
                 row_tile<true, LZ, true, S2, RM, ROWS, 2, true, WSync, true>(
-                    t, d, gcast(j.src[p]), nullptr, off, lds + k * KSI_PART_WORDS, lane, wlanes, wsync);
+                    t, d, gcast(src), nullptr, off, lds + k * KSI_PART_WORDS, lane, wlanes, wsync);
         }
         ++k;
+    };
+    const uint32_t np = j.np, rows = FIN ? np + 2 : np;
+    for (uint32_t p = 0; p < rows; ++p) {
+        if (p < np) {
+            if ((j.xf >> p) & 1) row_pass(j.src[p]);
+        } else {
+            row_pass(j.fin.v[p - np]);
+        }
+    }
+    if constexpr (FIN) {
+        // the last step as a forward transform's epilogue (ntt_ep_value)
+        t.c0 = j.fin.ci;
+        t.c0p = j.fin.cip;
+        t.c1 = j.fin.ce;
+        t.c1p = j.fin.cep;
     }
     bsync();
     // up to 4 parts with every value below 2^60: column sums, loads first
     bool done = false;
     if (j.d30)
-        done = j.pairs ? ksi_inner_cols_np<2, LZ>(j, lds, off, tid, nthr, t)
-                       : ksi_inner_cols_np<1, LZ>(j, lds, off, tid, nthr, t);
+        done = j.pairs ? ksi_inner_cols_np<2, LZ, FIN>(j, lds, off, tid, nthr, t)
+                       : ksi_inner_cols_np<1, LZ, FIN>(j, lds, off, tid, nthr, t);
     // positions idx .. idx + V - 1 per step (V = 2: one 16-byte access per operand)
     auto inner = [&](auto Vc) {
         constexpr uint32_t V = decltype(Vc)::value;
@@ -287,7 +378,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
                         if constexpr (!LZ) dv[v] = ntt_final<true>(dv[v], t);
                     }
                 } else {
-                    load_words<V>(gcast(j.src[p]), gi, dv);
+                    load_words_any<V>(gcast(j.src[p]), gi, j, dv);
                 }
                 load_words<V>(gcast(j.kb[p]), gi, kb);
                 load_words<V>(gcast(j.ka[p]), gi, ka);
@@ -298,7 +389,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
             }
             uint64_t r0[V], r1[V];
             for (uint32_t v = 0; v < V; ++v) {
-                if (j.lazy_out) {
+                if (FIN || j.lazy_out) {
                     r0[v] = redc_lazy(s0[v], q, qneg);
                     r1[v] = redc_lazy(s1[v], q, qneg);
                 } else if constexpr (LZ) {
@@ -309,7 +400,9 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
                     r1[v] = redc(s1[v], q, qneg);
                 }
             }
-            ksi_store<V>(j, lds, idx, gi, r0, r1);
+            KsiEps<V> ep;
+            ksi_load_eps<FIN, V>(j, gi, ep);
+            ksi_store<FIN, LZ, V>(j, lds, idx, gi, r0, r1, ep, t);
         }
     };
     if (!done) {
@@ -319,7 +412,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
     // the inverse transforms' row pass of the two output rows (inputs in
     // [0, q), lazy outputs for the column pass after it), component c by
     // wave c
-    if (j.rp_on) {
+    if (!FIN && j.rp_on) {
         bsync();
         for (uint32_t c = wave; c < 2; c += nwaves) {
             const NttJob& r = j.rp[c];

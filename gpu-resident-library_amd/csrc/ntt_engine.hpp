@@ -92,7 +92,30 @@ struct NttJob {
     // forward epilogue: 1: e1 is added as it is (residues in [0, q), or null
     // for none; c1 unused), out = NTT(in) + e0*c0 + e1
     uint32_t e1_plain;
+    // inverse row pass, and e1_plain operands: the tower is read through the
+    // evaluation-domain automorphism of index gk (0: as it is), n = 2^glog
+    uint32_t gk, glog;
 };
+
+// Evaluation-domain automorphism sigma_k of a tower in bit-reversed order:
+// sigma_k(x)[i] = x[galois_index(i, k, log n)], k odd.  e = (2 brv(i) + 1) k mod
+// 2n names the evaluation point (e fits 32 bits: its high bits fall to the
+// mask).  For even i the point of i + 1 is n further (k is odd), so
+// galois_index(i + 1) = galois_index(i) ^ 1: an aligned pair of positions is
+// read as the aligned pair, swapped where that index is odd.
+GF_HD uint32_t brv32(uint32_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __brev(v);
+#else
+    uint32_t r = 0;
+    for (int b = 0; b < 32; ++b) r |= ((v >> b) & 1u) << (31 - b);
+    return r;
+#endif
+}
+GF_HD uint32_t galois_index(uint32_t i, uint32_t k, uint32_t logn) {
+    const uint32_t e = (2 * (brv32(i) >> (32 - logn)) + 1) * k & ((2u << logn) - 1);
+    return brv32(e >> 1) >> (32 - logn);
+}
 
 // floor(2^64 / q) for the moduli whose forward transforms run without
 // per-butterfly reductions, else 0 (NttJob::red)
@@ -473,7 +496,8 @@ GF_HD uint64_t ntt_final_ep(uint64_t v, const NttJob& j, uint64_t gi) {
         uint64_t r = 0;
         with_ep(j, [&](auto E) {
             constexpr int EP = decltype(E)::value;
-            r = ntt_ep_value<LZ, EP>(v, j, gat(gcast(j.e0), gi), EP == 2 ? 0 : gat(gcast(j.e1), gi));
+            const uint32_t g1 = EP == 1 && j.gk ? galois_index((uint32_t)gi, j.gk, j.glog) : (uint32_t)gi;
+            r = ntt_ep_value<LZ, EP>(v, j, gat(gcast(j.e0), gi), EP == 2 ? 0 : gat(gcast(j.e1), g1));
         });
         return r;
     }
@@ -588,7 +612,7 @@ GF_HD void row_out_ep(const NttJob& j, GF_GLOBAL uint64_t* dst, uint32_t off, co
                 const uint32_t idx = (u0 << R) + (mb + m) * W + lane;
                 if (U % 64 == 0 || idx < WORDS) {
                     x0[m] = gat(e0, off + idx);
-                    x1[m] = EP == 2 ? 0 : gat(e1, off + idx);
+                    x1[m] = EP == 2 ? 0 : gat(e1, EP == 1 && j.gk ? galois_index(off + idx, j.gk, j.glog) : off + idx);
                 }
             }
             GF_SCHED_FENCE();
@@ -622,7 +646,11 @@ GF_HD void row_tile(const NttJob& j, const TileDesc& d, const GF_GLOBAL uint64_t
     static_assert(!KEEP || !out_direct, "a kept tile ends in LDS");
     static_assert(!IN_LDS || !in_direct, "a tile given in LDS starts with a staged pass");
     if constexpr (!in_direct && !IN_LDS) {
-        wave_units<P0::R, WORDS>(tid, nthr, [&](uint32_t idx) { lds[padded(idx)] = gat(src, off + idx); });
+        if (!FWD && j.gk)
+            wave_units<P0::R, WORDS>(tid, nthr, [&](uint32_t idx) {
+                lds[padded(idx)] = gat(src, galois_index(off + idx, j.gk, j.glog));
+            });
+        else wave_units<P0::R, WORDS>(tid, nthr, [&](uint32_t idx) { lds[padded(idx)] = gat(src, off + idx); });
         sync.wave();
     }
     const RowIn gin{src + off, N};

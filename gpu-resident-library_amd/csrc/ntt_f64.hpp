@@ -369,12 +369,12 @@ struct LdsOutU52 {
 //   forward, KEEP: the keyswitch digits' row pass, inputs below 2q, the tile
 //     left in LDS for the inner product (element idx at lds[padded(idx)], in
 //     [0, 2q));
-//   inverse: a phase B, inputs below 4q, its output in [0, 2q) to dst for
-//     phase A.
+//   inverse: a phase B, inputs below 4q (gk: read through an automorphism, as
+//     NttJob::gk), its output in [0, 2q) to dst for phase A.
 template <bool FWD, uint32_t S, uint32_t RM, uint32_t ROWS, bool KEEP, class Sync, bool IN_LDS = false>
 GF_HD void row_tile_f64(const uint64_t* twd, const uint64_t* twrd, double q, double qinv, const TileDesc& d,
                         const GF_GLOBAL uint64_t* src, GF_GLOBAL uint64_t* dst, uint32_t off, uint64_t* lds,
-                        uint32_t tid, uint32_t nthr, Sync sync) {
+                        uint32_t tid, uint32_t nthr, Sync sync, uint32_t gk = 0, uint32_t glog = 0) {
     constexpr uint32_t N = 1u << S, NC = num_chunks(S, RM), WORDS = ROWS * N;
     using P0 = PassOf<FWD, S, RM, 0>;
     using PL = PassOf<FWD, S, RM, NC - 1>;
@@ -384,7 +384,11 @@ GF_HD void row_tile_f64(const uint64_t* twd, const uint64_t* twrd, double q, dou
     const double c2 = F64_2P52 + (FWD ? q : 2 * q);
     static_assert(!IN_LDS || !in_direct, "a tile given in LDS starts with a staged pass");
     if constexpr (!in_direct && !IN_LDS) {
-        wave_units<P0::R, WORDS>(tid, nthr, [&](uint32_t idx) { lds[padded(idx)] = gat(src, off + idx); });
+        if (!FWD && gk)
+            wave_units<P0::R, WORDS>(tid, nthr, [&](uint32_t idx) {
+                lds[padded(idx)] = gat(src, galois_index(off + idx, gk, glog));
+            });
+        else wave_units<P0::R, WORDS>(tid, nthr, [&](uint32_t idx) { lds[padded(idx)] = gat(src, off + idx); });
         sync.wave();
     }
     constexpr uint32_t RL = row_pass_r(S, RM), LOGU = S - RL;
@@ -412,7 +416,7 @@ GF_HD void phaseB_inv_f64(const NttJob& j, const NttGeom& g, uint32_t tile, uint
     const uint32_t a0 = tile * R;
     const TileDesc d{logR, 1, padded(N2), N1 + a0, 1, false, true};
     row_tile_f64<false, S2, RM, R, false, Sync, IN_LDS>(j.twd, j.twrd, j.fq, j.fqinv, d, gcast(j.in), gcast(j.out),
-                                                         a0 << S2, lds, tid, nthr, sync);
+                                                         a0 << S2, lds, tid, nthr, sync, j.gk, j.glog);
 }
 
 }  // namespace gf

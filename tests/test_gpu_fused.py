@@ -151,3 +151,63 @@ def test_column_pass_tiles(G, n, L, dnum):
         G.check(G.lib.gf_keyswitch(t.ctx.h, t.keys[0].h, level, x.ptr, b0.ptr, b1.ptr, ws.ptr, t.s.s))
         t.s.sync()
         assert np.array_equal(b0.download(), w[0]) and np.array_equal(b1.download(), w[1]), level
+
+
+@pytest.mark.parametrize("f64", [0, 1])
+@pytest.mark.parametrize("n,L,dnum,count", [(1 << 13, 6, 2, 16), (1 << 13, 7, 7, 12), (1 << 14, 6, 6, 8), (1 << 16, 5, 1, 3)])
+def test_last_step_in_the_inner_product(G, n, L, dnum, count, f64):
+    """Batches large enough that the Q rows' inner products take the outputs'
+    row passes with them, 1 to 7 parts (7 transform more rows than fit), and
+    rotations read their inputs through the automorphism; rotations whose
+    outputs are their own or another's inputs take permuted copies instead."""
+    t = Setup(G, n, L, dnum, nkeys=2, modup_f64=f64)
+    P, ctx, s = t.P, t.ctx, t.s
+    ks = [pow(5, 11, 2 * n), 2 * n - 1]
+    c = [[t.ct(L) for _ in range(4)] for _ in range(count)]
+    ws = [ctx.workspace() for _ in range(3 * count)]
+    wp = [w.ptr for w in ws]
+
+    def fresh():
+        return [[G.Dev.of(x) for x in v] for v in c]
+
+    def col(d, j):
+        return [x[j].ptr for x in d]
+
+    def check(dev, want, what):
+        assert np.array_equal(dev[0].download(want[0].size), want[0]), what
+        assert np.array_equal(dev[1].download(want[1].size), want[1]), what
+
+    last = "ksi" if dnum < 7 else "ntt_fwd_b"
+    some = sorted({0, 1, count - 1})
+    d = fresh()
+    o = [[G.Dev((L - 1) * n) for _ in range(2)] for _ in range(count)]
+    plan = G.plan_evalmult_rescale(ctx, t.keys[0], [L] * count, *[col(d, j) for j in range(4)], col(o, 0), col(o, 1), wp[:count])
+    assert plan.steps()[-1][0] == last, plan.steps()
+    plan.run_graph(s)
+    s.sync()
+    for i in some:
+        check(o[i], P.evalmult_rescale(L, *c[i], *t.hk[0]), ("mult", i))
+    kk, kh = [ks[i % 2] for i in range(count)], [t.keys[i % 2] for i in range(count)]
+    rot = {i: P.rotate(L, c[i][0], c[i][1], kk[i], *t.hk[i % 2]) for i in some}
+    # apart; in place; every output over the next one's input
+    for shift in (None, 0, 1):
+        d = fresh()
+        o = [[G.Dev(L * n) for _ in range(2)] for _ in range(count)]
+        if shift is not None:
+            o = [d[(i + shift) % count] for i in range(count)]
+        plan = G.plan_rotate(ctx, kh, [L] * count, kk, col(d, 0), col(d, 1), col(o, 0), col(o, 1), wp[:count])
+        kinds = [k for k, _ in plan.steps()]
+        assert ("perm" in kinds) == (shift is not None) and kinds[-1] == (last if shift is None else "ntt_fwd_b"), kinds
+        plan.run(s)
+        s.sync()
+        for i in some:
+            check(o[i], rot[i], ("rot", shift, i))
+    d = fresh()
+    h = [[G.Dev(L * n) for _ in range(2)] for _ in range(2 * count)]
+    plan = G.plan_rotate_hoisted(ctx, [L] * count, col(d, 0), col(d, 1), t.keys, ks, col(h, 0), col(h, 1), wp[:count], wp[count:])
+    assert plan.steps()[-1][0] == "ksi", plan.steps()
+    plan.run(s)
+    s.sync()
+    for i in some:
+        for j, w in enumerate(P.rotate_hoisted(L, c[i][0], c[i][1], ks, t.hk)):
+            check(h[2 * i + j], w, ("hoist", i, j))
