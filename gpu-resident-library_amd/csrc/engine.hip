@@ -1382,6 +1382,29 @@ void PlanBuilder::moddown_sources(ModupJob& J, const LevelConst& lv, const uint6
         }
     }
     J.sp = C.K;
+    moddown_targets(J);
+}
+
+// a dropped tower as source k of a fused ModDown or rescale: x is the row-pass
+// output of its inverse transform
+void PlanBuilder::drop_source(ModupJob& J, uint32_t k, uint32_t row, const uint64_t* x) const {
+    const Ctx& C = C_;
+    J.src[k] = x;
+    J.stw[k] = C.rt[row].iv2;
+    J.sq[k] = C.mods[row];
+    J.post[k] = C.rt[row].ninv;
+    J.postp[k] = C.rt[row].ninvp;
+    if (C.modup_f64 && C.rt[row].iv2d) {
+        J.stwd[k] = C.rt[row].iv2d;
+        J.sqd[k] = (double)C.mods[row];
+        J.sqinv[k] = 1.0 / J.sqd[k];
+        f64_twiddle(C.rt[row].ninv, C.mods[row], J.spost[k], J.spostq[k]);
+    }
+}
+
+// the Q towers as the targets of a fused ModDown or rescale job
+void PlanBuilder::moddown_targets(ModupJob& J) const {
+    const Ctx& C = C_;
     J.tq = C.d_md_tq;
     J.tqneg = C.d_md_tqneg;
     J.ttw = C.d_md_ttw;
@@ -1498,19 +1521,7 @@ void PlanBuilder::rescale_tail(const ModdownSrc& m, bool fused) {
         J.sc = last;
         J.dt = m.dt;
         J.dr = m.dr;
-        if (m.drop) {
-            J.src[K] = m.dr;
-            J.stw[K] = C.rt[last].iv2;
-            J.sq[K] = C.mods[last];
-            J.post[K] = C.rt[last].ninv;
-            J.postp[K] = C.rt[last].ninvp;
-            if (C.modup_f64 && C.rt[last].iv2d) {
-                J.stwd[K] = C.rt[last].iv2d;
-                J.sqd[K] = (double)C.mods[last];
-                J.sqinv[K] = 1.0 / J.sqd[K];
-                f64_twiddle(C.rt[last].ninv, C.mods[last], J.spost[K], J.spostq[K]);
-            }
-        }
+        if (m.drop) drop_source(J, K, last, m.dr);
         J.tabd = lv.d_tabMD + last;   // PHatModq column of q_last, row stride l
         J.tg = lv.d_rstg;
         J.tsw = lv.d_rs_sw;
@@ -1580,6 +1591,37 @@ void PlanBuilder::rescale_comp(uint32_t l, const uint64_t* c, uint64_t* o, uint6
     const Ctx& C = C_;
     const uint32_t n = C.n, last = l - 1;
     const LevelConst& lv = C.lv[l];
+    if (C.fused && C.moddown_fused && !C.geom.single && !C.wide && n % MODUP_TILE == 0) {
+        // o_i = c_i s1_i + NTT_i(s2_i switch(INTT(c_last))): the inverse row
+        // pass, one kernel for its column pass, the switch and every target's
+        // column pass, and the row pass with the other term as it stores: 3
+        // launches instead of 6 and 3 trips of a tower through HBM instead
+        // of 6 (a component of 17 towers at n = 2^16: 50 -> 27 us).  sw keeps o free
+        // to be c.
+        NttJob J{c + (size_t)last * n, drop, C.rt[last].iv2, nullptr, C.mods[last], C.rt[last].ninv, C.rt[last].ninvp};
+        intt_dropb_.push_back(J);
+        ModupJob M{};
+        moddown_targets(M);
+        M.sp = 0;
+        M.sc = last;
+        M.dst = sw;
+        drop_source(M, 0, last, drop);
+        M.tg = lv.d_rstg;
+        M.tsw = lv.d_rs_sw;
+        M.q_old = C.mods[last];
+        M.half = C.mods[last] >> 1;
+        rsdown_.push_back(M);
+        for (uint32_t i = 0; i < last; ++i) {
+            NttJob T{nullptr, o + (size_t)i * n, C.rt[i].fw2, nullptr, C.mods[i], 0, 0};
+            T.mid = sw + (size_t)i * n;
+            T.e0 = c + (size_t)i * n;
+            T.c0 = lv.s1[i];
+            T.c0p = lv.s1p[i];
+            T.e1_plain = 1;
+            ntt_rsb_.push_back(T);
+        }
+        return;
+    }
     intt_drop_.push_back(NttJob{c + (size_t)last * n, drop, C.rt[last].iv2, nullptr, C.mods[last],
                                 C.rt[last].ninv, C.rt[last].ninvp});
     for (uint32_t i = 0; i < last; ++i) {
@@ -1872,7 +1914,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         }
     }
     for (auto* v : {&intt_up_, &intt_upb_, &ntt_dig_, &ntt_diga_, &ntt_digb_, &intt_p_, &intt_pb_, &ntt_conv_, &intt_drop_,
-                    &ntt_sw_, &ntt_v_, &ntt_vb_}) {
+                    &intt_dropb_, &ntt_sw_, &ntt_v_, &ntt_vb_, &ntt_rsb_}) {
         group_by(*v, [](const NttJob& j) { return (uintptr_t)j.tw; });
         // every transform of a plan uses the context's paired tables; its phase B
         // reads the matching row table of the current radix
@@ -1883,7 +1925,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     }
     // forward transforms over moduli below 2^57 skip the butterflies'
     // conditional subtractions; the digits stay unreduced for the inner product
-    for (auto* v : {&ntt_dig_, &ntt_diga_, &ntt_digb_, &ntt_conv_, &ntt_sw_, &ntt_v_, &ntt_vb_})
+    for (auto* v : {&ntt_dig_, &ntt_diga_, &ntt_digb_, &ntt_conv_, &ntt_sw_, &ntt_v_, &ntt_vb_, &ntt_rsb_})
         for (NttJob& j : *v) j.red = lazy_red_of(j.q);
     for (auto* v : {&ntt_dig_, &ntt_digb_})
         for (NttJob& j : *v) j.lazy_out = j.red != 0;
@@ -1934,6 +1976,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
                     if (!j.xf || !modup_.empty()) f64_job(j);
         if (!modup_.empty())
             for (NttJob& j : intt_upb_) f64_job(j);
+        for (NttJob& j : intt_dropb_) f64_job(j);
     }
     // KSI jobs by their LDS regions, most first, by key within a region count
     for (auto* v : {&ksi_, &ksi_fin_}) {
@@ -2044,6 +2087,9 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(SWITCH, switch_);
     GF_STAGE(NTT_F, ntt_sw_);
     GF_STAGE(FUSE, fuse_);
+    GF_STAGE(NTT_IB, intt_dropb_);
+    stage_modup(Step::MODDOWN, rsdown_);
+    GF_STAGE(NTT_FB, ntt_rsb_);
     GF_STAGE(RSV, rs_);
     GF_STAGE(NTT_F, ntt_v_);
     GF_STAGE(NTT_FB, ntt_vb_);

@@ -331,6 +331,9 @@ private:
     std::vector<SwitchJob> switch_;
     std::vector<NttJob> ntt_sw_;
     std::vector<FuseJob> fuse_;
+    std::vector<NttJob> intt_dropb_;   // a fused rescale: its dropped towers' inverse row pass,
+    std::vector<ModupJob> rsdown_;     // the switched towers from it (ModupJob with sp = 0),
+    std::vector<NttJob> ntt_rsb_;      // and the surviving towers' row pass
     std::vector<RsJob> rs_;
     std::vector<NttJob> ntt_v_;
     std::vector<NttJob> intt_pb_;    // P towers whose inverse column pass runs in the fused ModDown
@@ -387,6 +390,8 @@ private:
     void ks_tail(const ModdownSrc& m, bool fused);
     // the K P towers as the sources of a fused ModDown job
     void moddown_sources(ModupJob& J, const LevelConst& lv, const uint64_t* xp) const;
+    void moddown_targets(ModupJob& J) const;
+    void drop_source(ModupJob& J, uint32_t k, uint32_t row, const uint64_t* x) const;
     void evalmult_rescale_fused(uint32_t l, const uint64_t* c0a, const uint64_t* c1a,
                                 const uint64_t* c0b, const uint64_t* c1b, uint64_t* o0, uint64_t* o1,
                                 const DevKey& key, uint64_t* ws);

@@ -69,7 +69,7 @@ __device__ __forceinline__ void modup_run(const ModupJob& j, const NttGeom& g, u
         if (j.src[SP]) {
             modup_source<S1>(j, SP, g, lds, twl, tid, tile, cv);
             modup_drop_src<SP, S1>(j, x, cv, dv);
-        } else {
+        } else if constexpr (SP > 0) {
             modup_drop_unit<SP, S1>(j, g, tile, tid, x, dv);
         }
         for (uint32_t t = t0; t < t1; ++t) target(t, [&] { modup_rs_unit<SP, S1>(j, t, x, dv, cv); });
@@ -105,9 +105,9 @@ __global__ __launch_bounds__(MODUP_THREADS) __attribute__((amdgpu_waves_per_eu(4
     switch (j.sp) {
 #define GF_SP(k) \
     case k: \
-        if constexpr (k <= SPMAX) modup_run<S1, k, RS, C60>(j, g, lds, twl, tid, tile); \
+        if constexpr (k <= SPMAX && (k > 0 || RS)) modup_run<S1, k, RS, C60>(j, g, lds, twl, tid, tile); \
         break;
-        GF_SP(1) GF_SP(2) GF_SP(3) GF_SP(4) GF_SP(5) GF_SP(6)
+        GF_SP(0) GF_SP(1) GF_SP(2) GF_SP(3) GF_SP(4) GF_SP(5) GF_SP(6)
 #undef GF_SP
     }
 }
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(MODUP_THREADS) __attribute__((amdgpu_waves_per_eu(4
 // sp: the largest source count of the jobs
 template <bool RS, bool C60>
 static void launch_modup_t(const ModupJob* d, uint32_t nj, const NttGeom& g, uint32_t sp, hipStream_t s) {
-    if (g.single || g.n % MODUP_TILE || sp < 1 || sp > MODUP_MAXSRC)
+    if (g.single || g.n % MODUP_TILE || (sp < 1 && !RS) || sp > MODUP_MAXSRC)
         throw std::runtime_error("gpufhe: fused ModUp / ModDown launch shape out of range");
     const bool ok = with_split(g.logN1, g.logN2, [&](auto A, auto) {
         constexpr uint32_t S1 = decltype(A)::value;

@@ -129,7 +129,8 @@ struct ModupJob {
     // dr are unused: src[sp] is the row-pass output of the inverse transform
     // of t + res pinv (which KsiJob::drop leaves), post[sp] = n^-1, and
     //   dv = INTT(t + res pinv) - REDC(..) pinv,
-    // the same residue by linearity.
+    // the same residue by linearity.  sp = 0: a plain rescale of one component,
+    // src[0] the row-pass output of its dropped tower's inverse transform.
     const uint64_t* dt;
     const uint64_t* dr;
     const uint64_t* tabd;
@@ -163,7 +164,7 @@ struct ColOutF64 {
 // 2^60) as its low and high 30 bits
 template <uint32_t SP>
 struct ModupUnit {
-    uint32_t lo[MODUP_UNIT][SP], hi[MODUP_UNIT][SP];
+    uint32_t lo[MODUP_UNIT][SP ? SP : 1], hi[MODUP_UNIT][SP ? SP : 1];
 };
 
 // chunk 0 is one full radix-4 pass with one unit per thread
@@ -343,8 +344,12 @@ GF_HD void modup_drop_src(const ModupJob& j, const ModupUnit<SP>& x, const uint6
                                         j.sqinv[SP]));
         else
             r = shoup(v[u], j.post[SP], j.postp[SP], q);
-        const U128 acc = dot30<SP>(x.lo[u], x.hi[u], [&](uint32_t k) { return uniform_at(j.tabd, k * j.strided); });
-        dv[u] = submod(r, shoup(redc(acc, q, j.qd_neg), j.pinv, j.pinvp, q), q);
+        if constexpr (SP == 0) {
+            dv[u] = r;   // a plain rescale: nothing to take off
+        } else {
+            const U128 acc = dot30<SP>(x.lo[u], x.hi[u], [&](uint32_t k) { return uniform_at(j.tabd, k * j.strided); });
+            dv[u] = submod(r, shoup(redc(acc, q, j.qd_neg), j.pinv, j.pinvp, q), q);
+        }
     }
 }
 // Rescale mode: target t's prologue value of this thread's unit into cv,

@@ -95,6 +95,8 @@ struct NttJob {
     // inverse row pass, and e1_plain operands: the tower is read through the
     // evaluation-domain automorphism of index gk (0: as it is), n = 2^glog
     uint32_t gk, glog;
+    // forward row pass alone: the column-pass output it reads (null: out)
+    const uint64_t* mid;
 };
 
 // Evaluation-domain automorphism sigma_k of a tower in bit-reversed order:
@@ -699,7 +701,7 @@ GF_HD void phaseB_body(const NttJob& j, const NttGeom& g, uint32_t tile, uint64_
     // forward: phase B is the second phase (reads out); inverse: the first.
     // Inverse phase B hands lazy values in [0,4q) to phase A.
     row_tile<FWD, LZ, PAIRED, S2, RM, R, FWD ? 2 : 0, PAIRED, Sync, false, IN_LDS>(
-        j, d, gcast(FWD ? j.out : j.in), gcast(j.out), a0 << S2, lds, tid, nthr, sync);
+        j, d, gcast(!FWD ? j.in : j.mid ? j.mid : j.out), gcast(j.out), a0 << S2, lds, tid, nthr, sync);
 }
 
 // Single phase: the whole tower (n = 2^S <= NTT_SINGLE_MAX) is one tile.

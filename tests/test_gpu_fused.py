@@ -211,3 +211,31 @@ def test_last_step_in_the_inner_product(G, n, L, dnum, count, f64):
     for i in some:
         for j, w in enumerate(P.rotate_hoisted(L, c[i][0], c[i][1], ks, t.hk)):
             check(h[2 * i + j], w, ("hoist", i, j))
+
+
+@pytest.mark.parametrize("f64", [0, 1])
+@pytest.mark.parametrize("n,L,ascending", [(1 << 13, 2, False), (1 << 14, 6, True), (1 << 15, 7, False), (1 << 16, 3, True),
+                                           (1 << 17, 3, False)])
+def test_fused_rescale(G, n, L, ascending, f64):
+    """The rescale's fused form at every ring split, the dropped modulus below
+    and above the others, two towers and more, one component in place."""
+    import oracle as O
+    P = make_params(n, L, 1)
+    if ascending:
+        q = sorted(int(m) for m in P.q)
+        roots = [int(O.lib.or_native_root(n, m)) for m in q + [int(m) for m in P.p]]
+        P = O.Params(n, q, P.p, roots, 1)
+    ctx = G.Context(n, P.q, P.p, P.roots, 1)
+    ctx.set_knob("modup_f64", f64)
+    rng, s = np.random.default_rng(n + L), G.Stream()
+    ws, rs = ctx.workspace(), G.Dev(G.lib.gf_rescale_ws_bytes(ctx.h) // 8)
+    for level in sorted({2, L}):
+        c = [rand_rows(P.q[:level], n, rng) for _ in range(2)]
+        w = [P.rescale(x, level) for x in c]
+        d = [G.Dev.of(x) for x in c]
+        o = [G.Dev((level - 1) * n) for _ in range(2)]
+        G.check(G.lib.gf_rescale(ctx.h, level, d[0].ptr, d[1].ptr, o[0].ptr, o[1].ptr, ws.ptr, s.s))
+        G.check(G.lib.gf_rescale_comp(ctx.h, level, d[1].ptr, d[1].ptr, rs.ptr, s.s))
+        s.sync()
+        assert np.array_equal(o[0].download(), w[0]) and np.array_equal(o[1].download(), w[1]), level
+        assert np.array_equal(d[1].download((level - 1) * n), w[1]), ("in place", level)
