@@ -119,11 +119,13 @@ struct RsJob {
     uint32_t wide;          // as ConvJob::wide
 };
 
-// one tower of a freshly sampled small polynomial: dst = src mod q (signed src)
+// one tower of a freshly sampled small polynomial: dst = src mod q (signed
+// src; src16 instead where set)
 struct EmbedJob {
     const int64_t* src;
     uint64_t* dst;
     uint64_t q;
+    const int16_t* src16;
 };
 // switching-key rows of one part and one tower (src/evalkeygen.cpp:42-96):
 // a = pkA u + ns e1, b = pkB u + ns e0 (+ (P mod q) sOld on the part's own Q
@@ -224,6 +226,8 @@ void launch_rs(const RsJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 void launch_embed(const EmbedJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 void launch_ekgen(const EkJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 void launch_dec(const DecJob* d, uint32_t nj, uint32_t n, hipStream_t s);
+// x in [0, q) to its centred representative as a signed word, in place
+void launch_center(uint64_t* x, uint64_t q, uint32_t n, hipStream_t s);
 void launch_ptacc(const PtAccJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 // fused digit row pass + key inner product: regions = LDS regions (at least every
 // job's ksi_regions), waves = workgroup size in waves (1..KSI_WAVES), fin: every

@@ -301,7 +301,7 @@ __global__ __launch_bounds__(PW_THREADS) void k_embed(const EmbedJob* __restrict
                                                       uint32_t off, uint32_t n) {
     const EmbedJob j = jobs[off + blockIdx.y];
     PW_FOR(n) {
-        const int64_t v = j.src[i];
+        const int64_t v = j.src16 ? j.src16[i] : j.src[i];
         const uint64_t m = (uint64_t)(v < 0 ? -v : v);
         const uint64_t r = m < j.q ? m : m % j.q;   // |v| is small: the remainder is not taken in practice
         j.dst[i] = (v < 0 && r) ? j.q - r : r;
@@ -352,6 +352,13 @@ __global__ __launch_bounds__(PW_THREADS) void k_ekgen(const EkJob* __restrict__ 
 __global__ __launch_bounds__(PW_THREADS) void k_dec(const DecJob* __restrict__ jobs, uint32_t off, uint32_t n) {
     const DecJob j = jobs[off + blockIdx.y];
     PW_FOR(n) { ga(j.out, i) = addmod(ga(j.c0, i), mulmod(ga(j.c1, i), ga(j.s, i), j.q, j.qneg, j.r2), j.q); }
+}
+
+__global__ __launch_bounds__(PW_THREADS) void k_center(uint64_t* x, uint64_t q, uint32_t n) {
+    PW_FOR(n) {
+        const uint64_t v = ga(x, i);
+        ga(x, i) = v > q / 2 ? v - q : v;
+    }
 }
 
 __global__ __launch_bounds__(PW_THREADS) void k_ptacc(const PtAccJob* __restrict__ jobs,
@@ -446,6 +453,10 @@ void launch_sample(const SampleJob* d, uint32_t nj, uint32_t n, uint64_t seed, c
 }
 GF_PW_LAUNCH(launch_dec, k_dec, DecJob)
 GF_PW_LAUNCH(launch_ptacc, k_ptacc, PtAccJob)
+
+void launch_center(uint64_t* x, uint64_t q, uint32_t n, hipStream_t s) {
+    k_center<<<pw_grid(n, 1), PW_THREADS, 0, s>>>(x, q, n);
+}
 
 void launch_fill(uint64_t* d, const uint64_t* d_mods, uint32_t towers, uint32_t n, uint64_t seed,
                  hipStream_t s) {
