@@ -418,13 +418,14 @@ void Ctx::set_knob(const std::string& name, uint32_t v) {
         if (v > 1) throw std::runtime_error("gpufhe: modup_fused must be 0 or 1");
         modup_fused = v;
     } else if (name == "modup_f64" || name == "ksi_f64" || name == "moddown_fused" || name == "tensor_ib" ||
-               name == "ksi_rowpass" || name == "ksi_fin") {
+               name == "ksi_rowpass" || name == "ksi_fin" || name == "ksi_tensor") {
         if (v > 1) throw std::runtime_error("gpufhe: " + name + " must be 0 or 1");
         (name == "modup_f64"     ? modup_f64
          : name == "ksi_f64"     ? ksi_f64
          : name == "tensor_ib"   ? tensor_ib
          : name == "ksi_rowpass" ? ksi_rowpass
          : name == "ksi_fin"     ? ksi_fin
+         : name == "ksi_tensor"  ? ksi_tensor
                                  : moddown_fused) = v;
     } else if (name == "modup_min_wgs") {
         modup_min_wgs = v;
@@ -448,6 +449,7 @@ uint32_t Ctx::knob(const std::string& name) const {
     if (name == "ksi_rowpass") return ksi_rowpass;
     if (name == "moddown_fused") return moddown_fused;
     if (name == "ksi_fin") return ksi_fin;
+    if (name == "ksi_tensor") return ksi_tensor;
     if (name == "modup_min_wgs") return modup_min_wgs;
     if (name == "modup_split_wgs") return modup_split_wgs;
     if (name == "rechunk_wgs") return rechunk_wgs;
@@ -1042,14 +1044,14 @@ bool PlanBuilder::use_gather(uint32_t l) const { return use_ksi(l) && use_moddow
 // Whether a tower that the last steps read overlaps one that they write (an
 // operation in place, or one operation's output as another's input): those
 // steps then need everything they read to be copies of the plan's own.
-bool PlanBuilder::late_overlap() const {
-    if (late_reads_.empty() || late_writes_.empty()) return false;
+bool PlanBuilder::late_overlap(const std::vector<Span>& reads) const {
+    if (reads.empty() || late_writes_.empty()) return false;
     std::vector<Span> w = late_writes_;
     std::sort(w.begin(), w.end(), [](const Span& a, const Span& b) { return a.p < b.p; });
     const uint64_t* end = nullptr;   // the largest end among the writes up to each
     std::vector<const uint64_t*> ends(w.size());
     for (size_t i = 0; i < w.size(); ++i) ends[i] = end = std::max(end, w[i].p + w[i].words);
-    for (const Span& r : late_reads_) {
+    for (const Span& r : reads) {
         // the writes that start before the read's end
         const size_t k = std::lower_bound(w.begin(), w.end(), r.p + r.words,
                                           [](const Span& a, const uint64_t* b) { return a.p < b; }) - w.begin();
@@ -1510,7 +1512,10 @@ void PlanBuilder::evalmult_rescale_fused(uint32_t l, const uint64_t* c0a, const 
                            t[c], res[c], v + (size_t)c * last * n, outs[c], false, drop};
         rescale_tail(m, fmd);
     }
-    if (drop) fin_src_.push_back(f);
+    if (drop) {
+        fin_src_.push_back(f);
+        for (const uint64_t* p : {c0a, c1a, c0b, c1b}) tensor_reads_.push_back(Span{p, (size_t)last * n});
+    }
 }
 
 // The rescale tail of one component: from the K P towers (coefficient form,
@@ -1875,7 +1880,7 @@ std::unique_ptr<Plan> PlanBuilder::finish_into(void* d_arena, void* h_stage, siz
 }
 
 std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
-    if ((moddown_.size() + ksdown_.size()) * (C_.n / MODUP_TILE) < C_.modup_min_wgs || late_overlap())
+    if ((moddown_.size() + ksdown_.size()) * (C_.n / MODUP_TILE) < C_.modup_min_wgs || late_overlap(late_reads_))
         for (const RotSrc& r : rot_src_) permute_first(r);
     else if (C_.ksi_fin) finish_rows();
     // a fused ModUp stage too small to fill the chip runs unfused: the
@@ -2037,8 +2042,28 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         for (const TensorJob& t : tensor_) all &= t.pairs && by_in.count(t.t2) == 1;
         if (all) {
             std::vector<char> used(intt_upb_.size(), 0);
-            for (const TensorJob& t : tensor_) {
+            // Rows whose last step can form the three products itself: nothing
+            // but the row pass's input is formed here (2 rows in and 1 out
+            // instead of 4 in and 4 out, for one row more in the last step: 64
+            // EvalMult+Rescale at n = 2^16, L = 24 7800 -> 7160 us, one 214 -> 196)
+            std::map<const uint64_t*, KsiJob*> fin;
+            if (C_.ksi_tensor && !late_overlap(tensor_reads_))
+                for (KsiJob& j : ksi_fin_)
+                    if (!j.fin.e_plain && ksi_tensor_here(j))
+                        for (uint32_t p = 0; p < j.np; ++p)
+                            if (!((j.xf >> p) & 1)) fin[j.src[p]] = &j;
+            for (TensorJob& t : tensor_) {
                 const size_t i = by_in[t.t2];
+                const auto f = fin.find(t.t2);
+                if (f != fin.end()) {
+                    KsiFin& F = f->second->fin;
+                    F.in[0] = t.c0a;
+                    F.in[1] = t.c1a;
+                    F.in[2] = t.c0b;
+                    F.in[3] = t.c1b;
+                    F.r2 = t.r2;
+                    t.lds_only = 1;
+                }
                 tensor_ib_.push_back(TensorIbJob{t, intt_upb_[i]});
                 used[i] = 1;
             }
@@ -2101,7 +2126,12 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(RSV, rs_);
     GF_STAGE(NTT_F, ntt_v_);
     GF_STAGE(NTT_FB, ntt_vb_);
-    stage_ksi(ksi_fin_, 1);
+    {
+        std::vector<KsiJob> ten, fin;
+        for (const KsiJob& j : ksi_fin_) (j.fin.in[0] ? ten : fin).push_back(j);
+        stage_ksi(ten, KSI_FIN_TENSOR);
+        stage_ksi(fin, KSI_FIN);
+    }
     GF_STAGE(ADD, add_);
     GF_STAGE(COPY, copy_);
     GF_STAGE(PTACC, ptacc_);

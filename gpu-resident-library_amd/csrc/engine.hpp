@@ -163,6 +163,9 @@ public:
     // 1: with the fused ModDown, the Q rows' inner products run in the launch
     // that runs the outputs' row passes (KsiFin)
     uint32_t ksi_fin = 1;
+    // 1 (with ksi_fin and tensor_ib): that launch forms a multiply's tensor
+    // products itself (KsiFin::in)
+    uint32_t ksi_tensor = 1;
     // a plan whose fused ModUp (or ModDown) stage would launch fewer workgroups
     // than this runs it unfused
     uint32_t modup_min_wgs = 0;
@@ -181,7 +184,7 @@ public:
     std::string tune_report;
     // sets or reads a knob by name ("ntt_radix", "ksi_extra", "conv_chunk",
     // "rs_chunk", "modup_fused", "modup_f64", "ksi_f64", "moddown_fused", "tensor_ib", "ksi_rowpass",
-    // "ksi_fin", "modup_min_wgs", "modup_split_wgs", "rechunk_wgs")
+    // "ksi_fin", "ksi_tensor", "modup_min_wgs", "modup_split_wgs", "rechunk_wgs")
     void set_knob(const std::string& name, uint32_t v);
     uint32_t knob(const std::string& name) const;
     std::string radix_report;   // the radix search of autotune(), as JSON
@@ -227,7 +230,7 @@ struct Step {
     size_t off;     // byte offset of the first job in the plan's device buffer
     uint32_t count;
     // KSI: the jobs' largest LDS region count (bits 0-7), waves per workgroup
-    // (bits 8-15), 1 << 16 where the jobs have a last step (KsiFin)
+    // (bits 8-15), the jobs' form (bits 16-17: KSI_PLAIN, ..)
     uint32_t arg = 0;
 };
 
@@ -375,7 +378,9 @@ private:
         size_t words;
     };
     std::vector<Span> late_reads_, late_writes_;
-    bool late_overlap() const;
+    std::vector<Span> tensor_reads_;   // ciphertexts whose products a last step may form itself
+    // whether a tower of r overlaps one of late_writes_
+    bool late_overlap(const std::vector<Span>& r) const;
     void permute_first(const RotSrc& r);
     bool use_gather(uint32_t l) const;
     void finish_rows();

@@ -192,7 +192,7 @@ inline uint32_t aligned16(std::initializer_list<const void*> ps) {
 inline TensorJob tensor_job(const uint64_t* c0a, const uint64_t* c1a, const uint64_t* c0b, const uint64_t* c1b,
                             uint64_t* t0, uint64_t* t1, uint64_t* t2, const RowConst& rc, uint32_t n) {
     const uint32_t pairs = n % 2 == 0 && aligned16({c0a, c1a, c0b, c1b, t0, t1, t2});
-    return TensorJob{c0a, c1a, c0b, c1b, t0, t1, t2, rc.q, rc.qneg, rc.r2, pairs};
+    return TensorJob{c0a, c1a, c0b, c1b, t0, t1, t2, rc.q, rc.qneg, rc.r2, pairs, 0};
 }
 
 inline void hip_check(hipError_t e, const char* what) {
@@ -230,9 +230,9 @@ void launch_dec(const DecJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 void launch_center(uint64_t* x, uint64_t q, uint32_t n, hipStream_t s);
 void launch_ptacc(const PtAccJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 // fused digit row pass + key inner product: regions = LDS regions (at least every
-// job's ksi_regions), waves = workgroup size in waves (1..KSI_WAVES), fin: every
-// job has a last step, or none has
-void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, bool fin, hipStream_t s);
+// job's ksi_regions), waves = workgroup size in waves (1..KSI_WAVES), fin: the
+// jobs' one form (KSI_PLAIN, ..)
+void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, uint32_t fin, hipStream_t s);
 void launch_tensor_ib(const TensorIbJob* d, uint32_t nj, const NttGeom& g, hipStream_t s);
 // the fused ModUp over jobs of at most arg & 0xff sources each and of one c60
 // (arg >> 8)

@@ -17,8 +17,8 @@ struct WaveSync {
 // in flight set the time.  Four parts with their last step take 5 waves of
 // 107 VGPRs uncapped: 64 EvalMult+Rescale at n = 2^16, L = 24 ran 8300 us with 4
 // waves per SIMD, 7570 with 5, 8280 with 6 (spills).
-// FIN: the jobs' last step (KsiFin).
-template <uint32_t S2, uint32_t RM, bool FIN>
+// FIN: KSI_PLAIN, KSI_FIN, KSI_FIN_TENSOR.
+template <uint32_t S2, uint32_t RM, int FIN>
 __global__ __launch_bounds__(KSI_THREADS) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_ksi(const KsiJob* __restrict__ jobs, uint32_t off, uint32_t N1) {
     extern __shared__ uint64_t lds[];
     const KsiJob& j = jobs[off + blockIdx.y];
@@ -31,7 +31,7 @@ __global__ __launch_bounds__(KSI_THREADS) __attribute__((amdgpu_waves_per_eu(5, 
     else go(std::false_type{});
 }
 
-void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, bool fin, hipStream_t s) {
+void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, uint32_t fin, hipStream_t s) {
     if (g.single || g.n % KSI_TILE) throw std::runtime_error("gpufhe: fused inner product needs a two-phase ring");
     if (regions > KSI_MAXP || waves < 1 || waves > KSI_WAVES)
         throw std::runtime_error("gpufhe: fused inner product launch shape out of range");
@@ -43,8 +43,9 @@ void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions
             for (uint32_t off = 0; off < nj; off += MAXY) {
                 const uint32_t cnt = nj - off < MAXY ? nj - off : MAXY;
                 const dim3 grid(g.n / KSI_TILE, cnt);
-                if (fin) k_ksi<S2, RM, true><<<grid, 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
-                else k_ksi<S2, RM, false><<<grid, 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
+                if (fin == KSI_FIN_TENSOR) k_ksi<S2, RM, KSI_FIN_TENSOR><<<grid, 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
+                else if (fin) k_ksi<S2, RM, KSI_FIN><<<grid, 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
+                else k_ksi<S2, RM, KSI_PLAIN><<<grid, 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
             }
         });
         if (!geom_ok) throw std::runtime_error("gpufhe: unsupported ring dimension for the NTT");

@@ -18,6 +18,7 @@
 #pragma once
 #include "ntt_engine.hpp"
 #include "ntt_f64.hpp"
+#include "tensor.hpp"
 
 namespace gf {
 
@@ -50,6 +51,12 @@ struct KsiFin {
     const uint64_t* e[2];
     uint64_t ci, cip, ce, cep;
     uint32_t e_plain;
+    // in[0] set (ksi_tensor_here): the two ciphertexts' rows c0a, c1a, c0b, c1b.
+    // e[0], e[1] and the untransformed digit are their tensor products, formed
+    // here and not read: the row's three products are not stored and read
+    // again for the price of one more input row.
+    const uint64_t* in[4];
+    uint64_t r2;   // 2^128 mod q
 };
 
 struct KsiJob {
@@ -153,14 +160,42 @@ inline uint32_t ksi_d30(uint64_t q, uint64_t red) {
 // row): to HBM, or (j.rp_on) into LDS regions 0 and 1 at those positions'
 // slots for the row pass after it; each thread writes only its own
 // positions, whose digits it has already read
+// the forms of the kernel: inner products stored (or through rp), with the
+// rows' last step, and with the tensor products formed there
+enum { KSI_PLAIN = 0, KSI_FIN = 1, KSI_FIN_TENSOR = 2 };
+
+// the jobs whose last step may form the tensor products itself: the column
+// sums' form of the inner product with two positions per access
+inline bool ksi_tensor_here(const KsiJob& j) { return j.fin.v[0] && j.d30 && j.np <= 4 && j.pairs; }
+
+// The tensor products of one position: t0, t1 for the lazy Shoup products and
+// t2 as a digit below 2^60.  fp64 rows: exact products in (-q, q) each, shifted
+// into [0, 4q).
+GF_HD void ksi_tensor(const KsiJob& j, const uint64_t* x, uint64_t& t0, uint64_t& t1, uint64_t& t2) {
+    if (j.twd) {
+        const double q = j.fq, qi = j.fqinv;
+        const double a0 = f64_from_u52(x[0], F64_2P52), a1 = f64_from_u52(x[1], F64_2P52),
+                     b0 = f64_from_u52(x[2], F64_2P52), b1 = f64_from_u52(x[3], F64_2P52);
+        t0 = u52_from_f64(f64_mulres(a0, b0, q, qi) + q);
+        t1 = u52_from_f64(f64_mulres(a0, b1, q, qi) + f64_mulres(a1, b0, q, qi) + 2 * q);
+        t2 = u52_from_f64(f64_mulres(a1, b1, q, qi) + q);
+        return;
+    }
+    TensorJob t{};
+    t.q = j.q;
+    t.qneg = j.qneg;
+    t.r2 = j.fin.r2;
+    tensor_one(t, x[0], x[1], x[2], x[3], t0, t1, t2);
+}
+
 template <uint32_t V>
 struct KsiEps {
     uint64_t e0[V], e1[V];   // fin.e[c] at the step's positions
 };
 // the last step's operands, requested with the step's other loads
-template <bool FIN, uint32_t V>
+template <int FIN, uint32_t V>
 GF_HD void ksi_load_eps(const KsiJob& j, uint32_t gi, KsiEps<V>& x) {
-    if constexpr (FIN) {
+    if constexpr (FIN == KSI_FIN) {
         if (j.fin.e_plain) {
             if (j.fin.e[0]) load_words_any<V>(gcast(j.fin.e[0]), gi, j, x.e0);
             if (j.fin.e[1]) load_words_any<V>(gcast(j.fin.e[1]), gi, j, x.e1);
@@ -170,14 +205,14 @@ GF_HD void ksi_load_eps(const KsiJob& j, uint32_t gi, KsiEps<V>& x) {
         }
     }
 }
-template <bool FIN, bool LZ, uint32_t V>
+template <int FIN, bool LZ, uint32_t V>
 GF_HD void ksi_store(const KsiJob& j, uint64_t* lds, uint32_t idx, uint32_t gi, const uint64_t* r0,
                      const uint64_t* r1, const KsiEps<V>& x, const NttJob& t) {
     if constexpr (FIN) {
         const uint32_t k0 = (uint32_t)__builtin_popcount(j.xf) * KSI_PART_WORDS;
         auto comp = [&](uint32_t c, const uint64_t* r, const uint64_t* e) {
             uint64_t y[V];
-            const int ep = !j.fin.e_plain ? 0 : j.fin.e[c] ? 1 : 2;
+            const int ep = FIN == KSI_FIN_TENSOR || !j.fin.e_plain ? 0 : j.fin.e[c] ? 1 : 2;
 #pragma unroll
             for (uint32_t v = 0; v < V; ++v) {
                 const uint64_t z = lds[k0 + c * KSI_PART_WORDS + padded(idx + v)];
@@ -231,7 +266,7 @@ GF_HD U128 cols_to_u128(uint64_t lo, uint64_t mid, uint64_t hi) {
 // sums are 30-bit column sums (j.d30): per part and component four 32 x 32
 // multiply-adds with no carries.  NP <= 7 keeps every column below 2^64
 // (lo, hi < 7 2^60; mid < 14 2^60).
-template <uint32_t NP, uint32_t V, bool LZ, bool FIN>
+template <uint32_t NP, uint32_t V, bool LZ, int FIN>
 GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t tid, uint32_t nthr,
                           const NttJob& t) {
     const GF_GLOBAL uint64_t *src[NP], *kb[NP], *ka[NP];
@@ -254,7 +289,7 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
             if (xf[p]) {
 #pragma unroll
                 for (uint32_t v = 0; v < V; ++v) dv[p][v] = lds[reg[p] + padded(idx + v)];
-            } else {
+            } else if constexpr (FIN != KSI_FIN_TENSOR) {
                 load_words_any<V>(src[p], gi, j, dv[p]);
             }
             load_words<V>(kb[p], gi, bv[p]);
@@ -262,6 +297,20 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
         }
         KsiEps<V> ep;
         ksi_load_eps<FIN, V>(j, gi, ep);
+        if constexpr (FIN == KSI_FIN_TENSOR) {
+            uint64_t x[4][V];
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) load_words<V>(gcast(j.fin.in[k]), gi, x[k]);
+#pragma unroll
+            for (uint32_t v = 0; v < V; ++v) {
+                const uint64_t y[4] = {x[0][v], x[1][v], x[2][v], x[3][v]};
+                uint64_t t2;
+                ksi_tensor(j, y, ep.e0[v], ep.e1[v], t2);
+#pragma unroll
+                for (uint32_t p = 0; p < NP; ++p)
+                    if (!xf[p]) dv[p][v] = t2;
+            }
+        }
         uint64_t r0[V], r1[V];
 #pragma unroll
         for (uint32_t v = 0; v < V; ++v) {
@@ -300,7 +349,7 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
 }
 
 // ksi_inner_cols for the job's part count, when it has an instantiation
-template <uint32_t V, bool LZ, bool FIN>
+template <uint32_t V, bool LZ, int FIN>
 GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t tid, uint32_t nthr,
                              const NttJob& t) {
     switch (j.np) {
@@ -312,9 +361,10 @@ GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint3
     }
 }
 
-// LZ = (j.red != 0), FIN = (j.fin.v[0] != null).  The wave-level sync wsync separates the row passes of
+// LZ = (j.red != 0), FIN = KSI_FIN where j.fin.v[0] is set, KSI_FIN_TENSOR
+// where j.fin.in[0] is too, else KSI_PLAIN.  The wave-level sync wsync separates the row passes of
 // one wave's region; bsync is the workgroup barrier before the inner product.
-template <uint32_t S2, uint32_t RM, bool LZ, class WSync, class BSync, bool FIN = false>
+template <uint32_t S2, uint32_t RM, bool LZ, class WSync, class BSync, int FIN = KSI_PLAIN>
 GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, uint32_t wave, uint32_t nwaves,
                     uint32_t lane, uint32_t wlanes, uint32_t tid, uint32_t nthr, WSync wsync, BSync bsync) {
     constexpr uint32_t ROWS = KSI_TILE >> S2, LOGR = KSI_LOG_TILE - S2;
@@ -358,8 +408,8 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
     // up to 4 parts with every value below 2^60: column sums, loads first
     bool done = false;
     if (j.d30)
-        done = j.pairs ? ksi_inner_cols_np<2, LZ, FIN>(j, lds, off, tid, nthr, t)
-                       : ksi_inner_cols_np<1, LZ, FIN>(j, lds, off, tid, nthr, t);
+        done = FIN == KSI_FIN_TENSOR || j.pairs ? ksi_inner_cols_np<2, LZ, FIN>(j, lds, off, tid, nthr, t)
+                                                : ksi_inner_cols_np<1, LZ, FIN>(j, lds, off, tid, nthr, t);
     // positions idx .. idx + V - 1 per step (V = 2: one 16-byte access per operand)
     auto inner = [&](auto Vc) {
         constexpr uint32_t V = decltype(Vc)::value;
@@ -405,7 +455,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
             ksi_store<FIN, LZ, V>(j, lds, idx, gi, r0, r1, ep, t);
         }
     };
-    if (!done) {
+    if (FIN != KSI_FIN_TENSOR && !done) {   // (those jobs have the column sums' form)
         if (j.pairs) inner(std::integral_constant<uint32_t, 2>{});
         else inner(std::integral_constant<uint32_t, 1>{});
     }

@@ -69,6 +69,18 @@ GF_HD double f64_mulmod(double y, double w, double wq, double q) {
     const double r = __builtin_fma(-k, q, p);
     return r + e;
 }
+// Product of two residues a, b in [0, q), q < 2^50, as a representative in
+// (-q, q): k = rint(fl(fl(a b) / q)) lies within 1/2 + 3 2^-53 q < 1 of
+// a b / q (three roundings of a quotient below q), e = a b - fl(a b) is
+// exact, and r = fma(-k, q, fl(a b)) is the integer (a b - k q) - e, below
+// q + 2^47 < 2^53, so nothing is rounded away.
+GF_HD double f64_mulres(double a, double b, double q, double qinv) {
+    GF_NO_CONTRACT
+    const double p = a * b;
+    const double e = __builtin_fma(a, b, -p);
+    const double k = __builtin_rint(p * qinv);
+    return __builtin_fma(-k, q, p) + e;
+}
 // centred representative: |result| <= q/2 + 2 for any integer |x| < 2^53
 // (fl(x / q) is within 8 2^-52 of x / q, so rint misses by one only next to
 // a half-integer)

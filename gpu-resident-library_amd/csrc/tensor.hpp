@@ -12,6 +12,9 @@ struct TensorJob {
     uint64_t *t0, *t1, *t2;
     uint64_t q, qneg, r2;
     uint32_t pairs;   // 1: every pointer 16-byte aligned (two residues per lane and access)
+    // 1 (in a TensorIbJob): only the row pass needs the products here, so t2 goes
+    // to it through LDS and nothing is stored (KsiFin::in forms them again)
+    uint32_t lds_only;
 };
 
 GF_HD void tensor_one(const TensorJob& j, uint64_t a0, uint64_t a1, uint64_t b0, uint64_t b1, uint64_t& t0,
@@ -29,6 +32,28 @@ GF_HD void tensor_one(const TensorJob& j, uint64_t a0, uint64_t a1, uint64_t b0,
 // per 16-byte access (j.pairs), the operands of 4 pairs requested at once.
 GF_HD void tensor_tile_lds(const TensorJob& j, uint32_t base, uint64_t* lds, uint32_t tid, uint32_t nthr) {
     constexpr uint32_t NP = NTT_TILE / 2, NB = 4;
+    if (j.lds_only) {
+        const GF_GLOBAL Words2* ap = (const GF_GLOBAL Words2*)gcast(j.c1a + base);
+        const GF_GLOBAL Words2* bp = (const GF_GLOBAL Words2*)gcast(j.c1b + base);
+        for (uint32_t pb = tid; pb < NP; pb += 2 * nthr) {
+            Words2 a[2], b[2];
+#pragma unroll
+            for (uint32_t e = 0; e < 2; ++e)
+                if (pb + e * nthr < NP) {
+                    a[e] = ap[pb + e * nthr];
+                    b[e] = bp[pb + e * nthr];
+                }
+#pragma unroll
+            for (uint32_t e = 0; e < 2; ++e) {
+                const uint32_t p = pb + e * nthr;
+                if (p >= NP) continue;
+#pragma unroll
+                for (uint32_t k = 0; k < 2; ++k)
+                    lds[padded(2 * p + k)] = mulmod(a[e].w[k], b[e].w[k], j.q, j.qneg, j.r2);
+            }
+        }
+        return;
+    }
     const GF_GLOBAL Words2* a0p = (const GF_GLOBAL Words2*)gcast(j.c0a + base);
     const GF_GLOBAL Words2* a1p = (const GF_GLOBAL Words2*)gcast(j.c1a + base);
     const GF_GLOBAL Words2* b0p = (const GF_GLOBAL Words2*)gcast(j.c0b + base);

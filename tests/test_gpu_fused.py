@@ -187,6 +187,15 @@ def test_last_step_in_the_inner_product(G, n, L, dnum, count, f64):
     s.sync()
     for i in some:
         check(o[i], P.evalmult_rescale(L, *c[i], *t.hk[0]), ("mult", i))
+    # a product over its own first factor, then over the next one's
+    for shift in (0, 1):
+        d = fresh()
+        o = [d[(i + shift) % count][:2] for i in range(count)]
+        plan = G.plan_evalmult_rescale(ctx, t.keys[0], [L] * count, *[col(d, j) for j in range(4)], col(o, 0), col(o, 1), wp[:count])
+        plan.run(s)
+        s.sync()
+        for i in some:
+            check(o[i], P.evalmult_rescale(L, *c[i], *t.hk[0]), ("mult over an input", shift, i))
     kk, kh = [ks[i % 2] for i in range(count)], [t.keys[i % 2] for i in range(count)]
     rot = {i: P.rotate(L, c[i][0], c[i][1], kk[i], *t.hk[i % 2]) for i in some}
     # apart; in place; every output over the next one's input
