@@ -345,12 +345,15 @@ uint32_t Ctx::autotune(hipStream_t s, float* best_ms) {
     // 256 MiB of towers (enough workgroups to fill the chip several times
     // over, as the batched stages do) cycling through every modulus, forward
     // then inverse, in place; each radix is timed twice, interleaved, and
-    // keeps its faster round
+    // keeps its faster round.  Radix 2^4 is not a candidate: its 16-element
+    // units leave three quarters of a 1024-element row tile's lanes idle (64
+    // EvalMult+Rescale at n = 2^16, L = 24: 9156 us, 7519 at 2^3, 7549 at 2^2),
+    // which whole transforms alone, bound by memory here, do not show.
     const uint32_t towers = std::max<uint32_t>(96, (1u << 25) / n);
     DevBuf buf((size_t)towers * n * 8);
     // job arrays per radix (the row tables differ): [r - 2][fwd towers, inv towers]
     std::vector<NttJob> jobs;
-    for (uint32_t r = 2; r <= 4; ++r)
+    for (uint32_t r = 2; r <= 3; ++r)
         for (int inv = 0; inv < 2; ++inv)
             for (uint32_t t = 0; t < towers; ++t) {
                 const uint32_t m = t % (L + K);
@@ -372,7 +375,7 @@ uint32_t Ctx::autotune(hipStream_t s, float* best_ms) {
     float bms = 1e30f;
     float per[5] = {1e30f, 1e30f, 1e30f, 1e30f, 1e30f};
     for (int round = 0; round < 2; ++round)
-        for (uint32_t r = 2; r <= 4; ++r) {
+        for (uint32_t r = 2; r <= 3; ++r) {
             NttGeom g = make_geom(n, r);
             const NttJob* fw = dj.as<NttJob>() + (size_t)(r - 2) * 2 * towers;
             const NttJob* iv = fw + towers;
@@ -396,7 +399,7 @@ uint32_t Ctx::autotune(hipStream_t s, float* best_ms) {
     {
         std::ostringstream o;
         o << "{\"workload_towers\": " << towers << ", \"ms_per_fwd_inv_pass\": {";
-        for (uint32_t r = 2; r <= 4; ++r) o << (r > 2 ? ", " : "") << "\"" << r << "\": " << per[r] / 3;
+        for (uint32_t r = 2; r <= 3; ++r) o << (r > 2 ? ", " : "") << "\"" << r << "\": " << per[r] / 3;
         o << "}, \"chosen\": " << best << "}";
         radix_report = o.str();
     }
@@ -503,14 +506,16 @@ void Ctx::autotune_plan(hipStream_t s, uint32_t B) {
     hipEvent_t e0, e1;
     hip_check(hipEventCreate(&e0), "event");
     hip_check(hipEventCreate(&e1), "event");
-    // the steps of the given kinds, timed together
+    // the steps of the given kinds (every step if none is given), timed together
     auto time_steps = [&](const Plan& P, std::initializer_list<Step::Kind> kinds) {
         P.run(s);
         hip_check(hipEventRecord(e0, s), "event");
         for (int r = 0; r < 5; ++r)
-            for (size_t i = 0; i < P.steps.size(); ++i)
+            for (size_t i = 0; i < P.steps.size(); ++i) {
+                if (kinds.size() == 0) P.run_step(i, s);
                 for (Step::Kind k : kinds)
                     if (P.steps[i].kind == k) P.run_step(i, s);
+            }
         hip_check(hipEventRecord(e1, s), "event");
         hip_check(hipEventSynchronize(e1), "event sync");
         float ms = 0;
@@ -535,6 +540,9 @@ void Ctx::autotune_plan(hipStream_t s, uint32_t B) {
         rep << "}, \"chosen\": " << knob << "}";
     };
     rep << ", \"batch\": " << B << ", \"level\": " << l;
+    // The knobs that decide which fused forms a plan takes change steps beside
+    // their own (one inverse transform or two for the dropped tower, the last
+    // step's launch), so they are timed on the whole plan.
     if (fused && !geom.single && n % KSI_TILE == 0) tune("ksi_extra", ksi_extra, {0, 1}, {Step::KSI});
     // the conversion chunk width matters where the ModUp runs unfused: tuned
     // with it unfused, then the fused ModUp is weighed against that
@@ -550,9 +558,9 @@ void Ctx::autotune_plan(hipStream_t s, uint32_t B) {
         tune("modup_f64", modup_f64, {0, 1}, {Step::NTT_IB, Step::MODUP});
         if (modup_f64) tune("ksi_f64", ksi_f64, {0, 1}, {Step::KSI});
         modup_fused = mf;
-        tune("modup_fused", modup_fused, {0, 1}, {Step::NTT_IB, Step::NTT_I, Step::MODUP, Step::CONV, Step::NTT_FA});
+        tune("modup_fused", modup_fused, {0, 1}, {});
         // the tensor product fused with the row pass in front of the fused ModUp
-        if (modup_fused) tune("tensor_ib", tensor_ib, {0, 1}, {Step::TENSOR, Step::NTT_IB, Step::TENSOR_IB});
+        if (modup_fused) tune("tensor_ib", tensor_ib, {0, 1}, {});
     }
     if (fused) {
         // the prologue's chunk width matters where the ModDown runs apart:
@@ -563,13 +571,12 @@ void Ctx::autotune_plan(hipStream_t s, uint32_t B) {
         moddown_fused = md;
         if (modup_fused && !geom.single && n % KSI_TILE == 0 && n % MODUP_TILE == 0 && !wide &&
             alpha <= MODUP_MAXSRC && K <= MODUP_MAXSRC)
-            tune("moddown_fused", moddown_fused, {0, 1},
-                 {Step::NTT_IB, Step::NTT_I, Step::MODDOWN, Step::RSV, Step::NTT_F, Step::NTT_FB});
+            tune("moddown_fused", moddown_fused, {0, 1}, {});
         // the P part's inverse row pass inside the P rows' inner product
         // (listed first: on a tie the tuner keeps the first candidate, and
         // this one moves fewer bytes in one launch fewer)
         if (moddown_fused && !geom.single && n % KSI_TILE == 0)
-            tune("ksi_rowpass", ksi_rowpass, {1, 0}, {Step::KSI, Step::NTT_IB});
+            tune("ksi_rowpass", ksi_rowpass, {1, 0}, {});
     }
     rep << "}";
     (void)hipEventDestroy(e0);
@@ -1791,13 +1798,15 @@ void PlanBuilder::linear_transform(uint32_t l, uint32_t m, const uint64_t* ks, c
         const size_t o = (size_t)i * n;
         PtAccJob J{};
         J.m = m;
+        J.o0 = o0 + o;
+        J.o1 = o1 + o;
+        J.pairs = n % 2 == 0 && aligned16({J.o0, J.o1});
         for (uint32_t j = 0; j < m; ++j) {
             J.pt[j] = pts[j] + o;
             J.x0[j] = x0[j] + o;
             J.x1[j] = x1[j] + o;
+            J.pairs &= aligned16({J.pt[j], J.x0[j], J.x1[j]});
         }
-        J.o0 = o0 + o;
-        J.o1 = o1 + o;
         J.q = C.rc[i].q;
         J.qneg = C.rc[i].qneg;
         J.r2 = C.rc[i].r2;
@@ -1829,6 +1838,7 @@ void PlanBuilder::mul_plain(uint32_t l, const uint64_t* c0, const uint64_t* c1, 
         J.x1[0] = c1 + o;
         J.o0 = o0 + o;
         J.o1 = o1 + o;
+        J.pairs = n % 2 == 0 && aligned16({J.pt[0], J.x0[0], J.x1[0], J.o0, J.o1});
         J.q = C_.rc[i].q;
         J.qneg = C_.rc[i].qneg;
         J.r2 = C_.rc[i].r2;
@@ -2089,24 +2099,29 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     // regions join the step before them where they are few (below KSI_JOIN
     // workgroups, or a quarter of that step's): a launch of their own would not
     // fill the chip.
-    auto stage_ksi = [&](const std::vector<KsiJob>& v, uint32_t fin) {
+    auto stage_ksi = [&](const std::vector<KsiJob>& v, uint32_t form) {
         const size_t tiles = C_.n / KSI_TILE;
+        std::vector<std::pair<size_t, size_t>> steps;
         for (size_t i = 0; i < v.size();) {
             size_t e = i;
-            const uint32_t x = ksi_regions(v[i]);
             while (e < v.size()) {
                 size_t g = e;
                 while (g < v.size() && ksi_regions(v[g]) == ksi_regions(v[e])) ++g;
                 if (e > i && (g - e) * tiles >= KSI_JOIN && (g - e) * 4 >= e - i) break;
                 e = g;
             }
-            const uint32_t waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
-            stage(Step::KSI, v.data() + i, e - i, sizeof(KsiJob));
-            P->steps.back().arg = x | waves << 8 | fin << 16;
+            steps.push_back({i, e});
             i = e;
         }
+        // launched the fewest regions first
+        for (size_t k = steps.size(); k-- > 0;) {
+            const KsiJob* first = v.data() + steps[k].first;
+            const uint32_t x = ksi_regions(*first), waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
+            stage(Step::KSI, first, steps[k].second - steps[k].first, sizeof(KsiJob));
+            P->steps.back().arg = x | waves << 8 | form << 16;
+        }
     };
-    stage_ksi(ksi_, 0);
+    stage_ksi(ksi_, KSI_PLAIN);
     GF_STAGE(NTT_I, intt_p_);
     GF_STAGE(NTT_IB, intt_pb_);
     stage_modup(Step::MODDOWN, moddown_);

@@ -174,6 +174,7 @@ struct PtAccJob {
     uint64_t* o1;
     uint64_t q, qneg, r2;
     uint32_t m;
+    uint32_t pairs;   // as TensorJob::pairs
 };
 
 // copy one tower
