@@ -970,6 +970,13 @@ void Plan::run_graph(hipStream_t s) {
 // is split back into small chunks at layout (split_chunks) to fill the chip.
 static const uint32_t CONV_CHUNK_SMALL = 8;
 static const size_t KSI_JOIN = 1024;
+// Hoisted rotations read every digit once per rotation.  In key order each
+// rotation goes through all of them, which is fine while they stay in the
+// 256 MiB last-level cache (8 terms at n = 2^15, 12 MiB of digits: 200 us, 204
+// row by row); above half of it all rotations of a row run together (4
+// ciphertexts at n = 2^16, L = 20, 200 MiB, 16 rotations: 2900 us in key order,
+// 2610 row by row).
+static const size_t HOIST_BY_ROW = (size_t)128 << 20;
 
 // Re-chunk conversion jobs ([j0, j1) target ranges) into CONV_CHUNK_SMALL
 // pieces when the stage would launch fewer than min_wgs workgroups
@@ -1732,6 +1739,7 @@ void PlanBuilder::rotate_hoisted(uint32_t l, uint32_t m, const uint64_t* ks, con
     }
     const WsLayout w = WsLayout::make(C);
     modup(l, c1, ws_base, nullptr, nullptr, nullptr, nullptr);
+    hoist_bytes_ += (size_t)lv.np * (l + C.K) * n * 8;
     const uint64_t* dig = ws_base + w.dig * n;
     for (uint32_t j = 0; j < m; ++j) {
         uint64_t* ws = ws_rot[j];
@@ -2004,6 +2012,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     // KSI jobs by their LDS regions, most first, by key within a region count
     for (auto* v : {&ksi_, &ksi_fin_}) {
         group_by(*v, [](const KsiJob& j) { return (uintptr_t)j.kb[0]; });
+        if (hoist_bytes_ > HOIST_BY_ROW) group_by(*v, [](const KsiJob& j) { return (uintptr_t)j.tw; });
         group_by(*v, [](const KsiJob& j) { return ~ksi_regions(j); });
     }
     group_by(inner_, [](const InnerJob& j) { return (uintptr_t)j.kb[0]; });

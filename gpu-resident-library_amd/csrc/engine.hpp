@@ -383,6 +383,7 @@ private:
     bool late_overlap(const std::vector<Span>& r) const;
     void permute_first(const RotSrc& r);
     bool use_gather(uint32_t l) const;
+    size_t hoist_bytes_ = 0;   // digits shared by hoisted rotations
     void finish_rows();
     // the rescale tail of one component of the fused EvalMult+Rescale: the
     // prologue and the epilogue transforms (apart), or the fused ModDown and
