@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <sstream>
 #include <tuple>
+#include <unordered_map>
 
 #include "ctr_sampler.hpp"
 #include "engine.hpp"
@@ -321,24 +322,26 @@ void Ctx::set_radix(uint32_t r) {
     for (uint32_t i = 0; i < L + K; ++i) t[i] = row_tables(n, mods[i], roots[i], r);
     geom = make_geom(n, r);
     rtr = std::move(t);
+    row_of_.clear();
+    f64_of_.clear();
+    for (uint32_t i = 0; i < L + K; ++i) {
+        row_of_[rt[i].fw2] = rtr[i].fwd;
+        row_of_[rt[i].iv2] = rtr[i].inv;
+        if (!rt[i].fw2d) continue;
+        row_of_[rt[i].fw2d] = rtr[i].fwd_d;
+        row_of_[rt[i].iv2d] = rtr[i].inv_d;
+        f64_of_[rt[i].fw2] = rt[i].fw2d;
+        f64_of_[rt[i].iv2] = rt[i].iv2d;
+    }
 }
 
 const uint64_t* Ctx::row_table_of(const uint64_t* paired) const {
-    if (!paired) return nullptr;
-    for (uint32_t i = 0; i < L + K; ++i) {
-        if (paired == rt[i].fw2) return rtr[i].fwd;
-        if (paired == rt[i].iv2) return rtr[i].inv;
-        if (paired == rt[i].fw2d) return rtr[i].fwd_d;
-        if (paired == rt[i].iv2d) return rtr[i].inv_d;
-    }
-    return nullptr;
+    const auto it = row_of_.find(paired);
+    return it == row_of_.end() ? nullptr : it->second;
 }
 const uint64_t* Ctx::f64_table_of(const uint64_t* paired) const {
-    for (uint32_t i = 0; i < L + K; ++i) {
-        if (paired == rt[i].fw2) return rt[i].fw2d;
-        if (paired == rt[i].iv2) return rt[i].iv2d;
-    }
-    return nullptr;
+    const auto it = f64_of_.find(paired);
+    return it == f64_of_.end() ? nullptr : it->second;
 }
 
 uint32_t Ctx::autotune(hipStream_t s, float* best_ms) {
@@ -1111,6 +1114,7 @@ void PlanBuilder::finish_rows() {
     for (const FinSrc& f : fin_src_) rows += f.rows;
     if (rows * (C_.n / KSI_TILE) < KSI_JOIN) return;
     std::vector<char> ku(ksi_.size(), 0), vu(ntt_vb_.size(), 0);
+    ksi_fin_.reserve(rows);
     for (const FinSrc& f : fin_src_)
         for (uint32_t i = 0; i < f.rows; ++i) {
             KsiJob J = ksi_[f.ksi0 + i];
@@ -1870,9 +1874,22 @@ void PlanBuilder::add_plain(uint32_t l, const uint64_t* c0, const uint64_t* c1, 
 // workgroups share a twiddle table (transforms), a key row (inner product) or a
 // constant table (conversions) keeps those operands in L2 across the batch
 // instead of re-reading them per ciphertext.
+// (Keys are sorted, not the jobs, which are up to 1 KiB each: one move per job.)
 template <class T, class K>
 static void group_by(std::vector<T>& v, K key) {
-    std::stable_sort(v.begin(), v.end(), [&](const T& a, const T& b) { return key(a) < key(b); });
+    using Key = decltype(key(v[0]));
+    std::vector<std::pair<Key, uint32_t>> k(v.size());
+    bool ordered = true;
+    for (size_t i = 0; i < v.size(); ++i) {
+        k[i] = {key(v[i]), (uint32_t)i};
+        ordered = ordered && (i == 0 || !(k[i] < k[i - 1]));
+    }
+    if (ordered) return;
+    std::sort(k.begin(), k.end());
+    std::vector<T> out;
+    out.reserve(v.size());
+    for (const auto& x : k) out.push_back(v[x.second]);
+    v.swap(out);
 }
 
 std::unique_ptr<Plan> PlanBuilder::finish() {
@@ -1969,7 +1986,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     // pass of its two output rows itself (from two LDS regions, ksi_regions),
     // and those row-pass jobs leave their stage
     if (C_.ksi_rowpass && !intt_pb_.empty()) {
-        std::map<const uint64_t*, size_t> by_in;
+        std::unordered_map<const uint64_t*, size_t> by_in(intt_pb_.size());
         for (size_t i = 0; i < intt_pb_.size(); ++i) by_in[intt_pb_[i].in] = i;
         std::vector<char> used(intt_pb_.size(), 0);
         for (KsiJob& j : ksi_) {
@@ -2009,12 +2026,6 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
             for (NttJob& j : intt_upb_) f64_job(j);
         for (NttJob& j : intt_dropb_) f64_job(j);
     }
-    // KSI jobs by their LDS regions, most first, by key within a region count
-    for (auto* v : {&ksi_, &ksi_fin_}) {
-        group_by(*v, [](const KsiJob& j) { return (uintptr_t)j.kb[0]; });
-        if (hoist_bytes_ > HOIST_BY_ROW) group_by(*v, [](const KsiJob& j) { return (uintptr_t)j.tw; });
-        group_by(*v, [](const KsiJob& j) { return ~ksi_regions(j); });
-    }
     group_by(inner_, [](const InnerJob& j) { return (uintptr_t)j.kb[0]; });
     split_chunks(conv_up_, C_.n, C_.rechunk_wgs);
     split_chunks(conv_dn_, C_.n, C_.rechunk_wgs);
@@ -2039,9 +2050,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     auto stage_modup = [&](Step::Kind kind, std::vector<ModupJob>& v) {
         if (v.empty()) return;
         split_targets(v, C_.n, C_.modup_split_wgs);
-        std::stable_sort(v.begin(), v.end(), [](const ModupJob& a, const ModupJob& b) {
-            return a.c60 != b.c60 ? a.c60 > b.c60 : a.sp + a.t1 - a.t0 > b.sp + b.t1 - b.t0;
-        });
+        group_by(v, [](const ModupJob& a) { return std::make_pair(!a.c60, ~(a.sp + a.t1 - a.t0)); });
         for (size_t i = 0; i < v.size();) {
             size_t e = i;
             uint32_t sp = 0;
@@ -2055,7 +2064,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     // tensor job has that row pass (the fused EvalMult+Rescale with the fused
     // ModUp): t2 goes to the row pass in LDS instead of through HBM
     if (C_.tensor_ib && !C_.geom.single && C_.geom.R * (1u << C_.geom.logN2) == NTT_TILE && !tensor_.empty()) {
-        std::map<const uint64_t*, size_t> by_in;
+        std::unordered_map<const uint64_t*, size_t> by_in(intt_upb_.size());
         for (size_t i = 0; i < intt_upb_.size(); ++i) by_in[intt_upb_[i].in] = i;
         bool all = true;
         for (const TensorJob& t : tensor_) all &= t.pairs && by_in.count(t.t2) == 1;
@@ -2065,7 +2074,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
             // but the row pass's input is formed here (2 rows in and 1 out
             // instead of 4 in and 4 out, for one row more in the last step: 64
             // EvalMult+Rescale at n = 2^16, L = 24 7800 -> 7160 us, one 214 -> 196)
-            std::map<const uint64_t*, KsiJob*> fin;
+            std::unordered_map<const uint64_t*, KsiJob*> fin(ksi_fin_.size());
             if (C_.ksi_tensor && !late_overlap(tensor_reads_))
                 for (KsiJob& j : ksi_fin_)
                     if (!j.fin.e_plain && ksi_tensor_here(j))
@@ -2104,18 +2113,26 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(NTT_FA, ntt_diga_);
     GF_STAGE(NTT_FB, ntt_digb_);
     GF_STAGE(INNER, inner_);
-    // One step per region count, with one wave per region; jobs of fewer
-    // regions join the step before them where they are few (below KSI_JOIN
-    // workgroups, or a quarter of that step's): a launch of their own would not
-    // fill the chip.
-    auto stage_ksi = [&](const std::vector<KsiJob>& v, uint32_t form) {
+    // KSI jobs by form, then by their LDS regions, most first, then by row (where
+    // hoisted digits exceed the cache) and key.  One step per region count, with
+    // one wave per region; jobs of fewer regions join the step before them where
+    // they are few (below KSI_JOIN workgroups, or a quarter of that step's): a
+    // launch of their own would not fill the chip.
+    const bool by_row = hoist_bytes_ > HOIST_BY_ROW;
+    auto ksi_form = [](const KsiJob& j) {
+        return !j.fin.v[0] ? (uint32_t)KSI_PLAIN : j.fin.in[0] ? (uint32_t)KSI_FIN_TENSOR : (uint32_t)KSI_FIN;
+    };
+    auto stage_ksi = [&](std::vector<KsiJob>& v) {
+        group_by(v, [&](const KsiJob& j) {
+            return std::make_tuple(ksi_form(j), ~ksi_regions(j), by_row ? (uintptr_t)j.tw : 0, (uintptr_t)j.kb[0]);
+        });
         const size_t tiles = C_.n / KSI_TILE;
         std::vector<std::pair<size_t, size_t>> steps;
         for (size_t i = 0; i < v.size();) {
             size_t e = i;
-            while (e < v.size()) {
+            while (e < v.size() && ksi_form(v[e]) == ksi_form(v[i])) {
                 size_t g = e;
-                while (g < v.size() && ksi_regions(v[g]) == ksi_regions(v[e])) ++g;
+                while (g < v.size() && ksi_form(v[g]) == ksi_form(v[e]) && ksi_regions(v[g]) == ksi_regions(v[e])) ++g;
                 if (e > i && (g - e) * tiles >= KSI_JOIN && (g - e) * 4 >= e - i) break;
                 e = g;
             }
@@ -2127,10 +2144,10 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
             const KsiJob* first = v.data() + steps[k].first;
             const uint32_t x = ksi_regions(*first), waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
             stage(Step::KSI, first, steps[k].second - steps[k].first, sizeof(KsiJob));
-            P->steps.back().arg = x | waves << 8 | form << 16;
+            P->steps.back().arg = x | waves << 8 | ksi_form(*first) << 16;
         }
     };
-    stage_ksi(ksi_, KSI_PLAIN);
+    stage_ksi(ksi_);
     GF_STAGE(NTT_I, intt_p_);
     GF_STAGE(NTT_IB, intt_pb_);
     stage_modup(Step::MODDOWN, moddown_);
@@ -2150,12 +2167,7 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(RSV, rs_);
     GF_STAGE(NTT_F, ntt_v_);
     GF_STAGE(NTT_FB, ntt_vb_);
-    {
-        std::vector<KsiJob> ten, fin;
-        for (const KsiJob& j : ksi_fin_) (j.fin.in[0] ? ten : fin).push_back(j);
-        stage_ksi(ten, KSI_FIN_TENSOR);
-        stage_ksi(fin, KSI_FIN);
-    }
+    stage_ksi(ksi_fin_);
     GF_STAGE(ADD, add_);
     GF_STAGE(COPY, copy_);
     GF_STAGE(PTACC, ptacc_);

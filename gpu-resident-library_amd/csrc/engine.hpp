@@ -8,6 +8,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "internal.hpp"
@@ -125,6 +126,7 @@ public:
     // the fp64 pairs of the same twiddles as a paired table (fw2 -> fw2d,
     // iv2 -> iv2d), null for moduli of 2^50 and above
     const uint64_t* f64_table_of(const uint64_t* paired) const;
+    std::unordered_map<const uint64_t*, const uint64_t*> row_of_, f64_of_;   // what those two look up (set_radix)
     uint32_t row_q(uint32_t i) const { return i; }
     uint32_t row_p(uint32_t k) const { return L + k; }
     uint32_t num_parts(uint32_t l) const { return (l + alpha - 1) / alpha; }
