@@ -173,8 +173,10 @@ public:
     uint32_t modup_min_wgs = 0;
     // fused ModUp and ModDown stages that would launch fewer workgroups than
     // this split their jobs' targets over more of them, down to one target
-    // each, every one of them transforming the sources anew
-    uint32_t modup_split_wgs = 1024;
+    // each, every one of them transforming the sources anew (one operation at
+    // n = 2^16, L = 24: 216 us at 256, 188 at 512, 185 at 768, 196 at 1024, 218 at
+    // 1536; a keyswitch sequence of 17 towers 233, 216, 209, 217, 233)
+    uint32_t modup_split_wgs = 768;
     // conversion and prologue stages that would launch fewer workgroups than
     // this are re-split into 8-target jobs, whatever the chunk knobs say
     uint32_t rechunk_wgs = 8192;
