@@ -237,8 +237,10 @@ Ctx::Ctx(uint32_t n_, const std::vector<uint64_t>& q, const std::vector<uint64_t
         // the same times -P^-1: the fused ModDown of a keyswitch
         std::vector<uint64_t> tabKS((size_t)K * l);
         for (uint32_t i = 0; i < l; ++i)
-            for (uint32_t k = 0; k < K; ++k)
-                tabKS[(size_t)k * l + i] = host_mulmod(tab[(size_t)k * l + i], mods[i] - c.pinv[i], mods[i]);
+            for (uint32_t k = 0; k < K; ++k) {
+                const uint64_t x = shoup(tab[(size_t)k * l + i], c.pinv[i], c.pinvp[i], mods[i]);
+                tabKS[(size_t)k * l + i] = x ? mods[i] - x : 0;
+            }
         put(tabKS, &c.d_tabKS);
         // rescale dropping tower l-1: s1 = q_{l-1}^-1 mod q_i, s2 = -s1 mod q_i
         // (s2 = floor(Q' [Q'^-1]_{q_l} / q_l) mod q_i is congruent to -s1, src/params.cpp:50-75)
@@ -257,9 +259,10 @@ Ctx::Ctx(uint32_t n_, const std::vector<uint64_t>& q, const std::vector<uint64_t
                 const uint64_t ps1 = host_mulmod(c.pinv[i], s1, qi);
                 c.ps1.push_back(ps1);
                 c.ps1p.push_back(host_precon(ps1, qi));
-                const uint64_t neg = ps1 ? qi - ps1 : 0;
-                for (uint32_t k = 0; k < K; ++k)
-                    tabRS[(size_t)k * (l - 1) + i] = host_mulmod(tab[(size_t)k * l + i], neg, qi);
+                for (uint32_t k = 0; k < K; ++k) {
+                    const uint64_t x = shoup(tab[(size_t)k * l + i], ps1, c.ps1p.back(), qi);
+                    tabRS[(size_t)k * (l - 1) + i] = x ? qi - x : 0;
+                }
                 const SwitchJob sj = make_switch(nullptr, nullptr, ql, qi);
                 const RsTarget t{qi, host_qneg(qi), sj.diff, sj.new_larger, s2, host_precon(s2, qi), sj.red};
                 const uint64_t* tw = (const uint64_t*)&t;
@@ -2045,16 +2048,16 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         P->steps.push_back(Step{kind, off, (uint32_t)cnt});
     };
 #define GF_STAGE(k, v) stage(Step::k, v.data(), v.size(), sizeof(v[0]))
-    // one launch for every source count (per conversion reduction), the
-    // longest jobs first
+    // one launch for every source count (per conversion reduction, and 7 or
+    // more sources apart), the longest jobs first
     auto stage_modup = [&](Step::Kind kind, std::vector<ModupJob>& v) {
         if (v.empty()) return;
         split_targets(v, C_.n, C_.modup_split_wgs);
-        group_by(v, [](const ModupJob& a) { return std::make_pair(!a.c60, ~(a.sp + a.t1 - a.t0)); });
+        group_by(v, [](const ModupJob& a) { return std::make_tuple(!a.c60, a.sp > 6, ~(a.sp + a.t1 - a.t0)); });
         for (size_t i = 0; i < v.size();) {
             size_t e = i;
             uint32_t sp = 0;
-            for (; e < v.size() && v[e].c60 == v[i].c60; ++e) sp = std::max(sp, v[e].sp);
+            for (; e < v.size() && v[e].c60 == v[i].c60 && (v[e].sp > 6) == (v[i].sp > 6); ++e) sp = std::max(sp, v[e].sp);
             stage(kind, v.data() + i, e - i, sizeof(ModupJob));
             P->steps.back().arg = sp | v[i].c60 << 8;
             i = e;

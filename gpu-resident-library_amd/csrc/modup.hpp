@@ -58,7 +58,7 @@ enum {
     MODUP_RM = 2,                                  // register radix 2^2: 4 elements per unit
     MODUP_UNIT = 1 << MODUP_RM,
     MODUP_THREADS = MODUP_TILE / MODUP_UNIT,       // one chunk-0 unit per thread
-    MODUP_MAXSRC = 6
+    MODUP_MAXSRC = 12
 };
 
 // per surviving tower constants of the fused ModDown + rescale prologue
@@ -159,6 +159,13 @@ struct ColOutF64 {
         gat(dst, (k << logN2) + b0 + s) = u52_from_f64(f64_center(v, q, qinv) + q);
     }
 };
+
+// dot30 over any number of terms up to 16: the column sums hold 8
+template <uint32_t NS, class B>
+GF_HD U128 dot30_any(const uint32_t* alo, const uint32_t* ahi, B b) {
+    if constexpr (NS <= 8) return dot30<NS>(alo, ahi, b);
+    else return add128(dot30<8>(alo, ahi, b), dot30<NS - 8>(alo + 8, ahi + 8, [&](uint32_t s) { return b(s + 8); }));
+}
 
 // one thread's unit of every source: element u of source i (reduced, below
 // 2^60) as its low and high 30 bits
@@ -288,7 +295,8 @@ GF_HD void modup_take_unit(const ModupJob& j, uint32_t i, const uint64_t* v, Mod
     }
 }
 // target t's conversion of this thread's unit into cv: the exact column sums
-// over the part's sources, REDC without its correction ([0, 2 q_t)), as the
+// over the part's sources, REDC without its correction (below 1.75 q_t for 12
+// sources below 2^60), as the
 // conversion kernel leaves them for the forward transforms (with c60 the
 // R = 2^60 reduction of the columns, below 2.2 q_t); for an fp64 target as
 // the double v - q_t (|.| <= 1.25 q_t)
@@ -310,7 +318,7 @@ GF_HD void modup_convert_unit(const ModupJob& j, uint32_t t, ModupUnit<SP>& x, u
         auto cst = [&](uint32_t s) { return uniform_at(j.tab, s * j.sc + t); };
         uint64_t v;
         if constexpr (C60) v = redc60_lazy(dot30_cols<SP>(x.lo[u], x.hi[u], cst), q, qn);
-        else v = redc_lazy(dot30<SP>(x.lo[u], x.hi[u], cst), q, qn);
+        else v = redc_lazy(dot30_any<SP>(x.lo[u], x.hi[u], cst), q, qn);
         cv[u] = f64 ? bits_of_f64(f64_from_u52(v, c2)) : v;
     }
 }
@@ -326,7 +334,7 @@ GF_HD void modup_drop_unit(const ModupJob& j, const NttGeom& g, uint32_t tile, u
 #pragma unroll
     for (uint32_t u = 0; u < MODUP_UNIT; ++u) {
         const uint32_t gi = ((k0 + u * TL) << g.logN2) + tile * C + s;
-        const U128 acc = dot30<SP>(x.lo[u], x.hi[u], [&](uint32_t k) { return uniform_at(j.tabd, k * j.strided); });
+        const U128 acc = dot30_any<SP>(x.lo[u], x.hi[u], [&](uint32_t k) { return uniform_at(j.tabd, k * j.strided); });
         const uint64_t cd = redc(acc, q, j.qd_neg);
         dv[u] = addmod(gat(gcast(j.dt), gi), shoup(submod(gat(gcast(j.dr), gi), cd, q), j.pinv, j.pinvp, q), q);
     }
@@ -347,7 +355,7 @@ GF_HD void modup_drop_src(const ModupJob& j, const ModupUnit<SP>& x, const uint6
         if constexpr (SP == 0) {
             dv[u] = r;   // a plain rescale: nothing to take off
         } else {
-            const U128 acc = dot30<SP>(x.lo[u], x.hi[u], [&](uint32_t k) { return uniform_at(j.tabd, k * j.strided); });
+            const U128 acc = dot30_any<SP>(x.lo[u], x.hi[u], [&](uint32_t k) { return uniform_at(j.tabd, k * j.strided); });
             dv[u] = submod(r, shoup(redc(acc, q, j.qd_neg), j.pinv, j.pinvp, q), q);
         }
     }
@@ -358,7 +366,6 @@ GF_HD void modup_drop_src(const ModupJob& j, const ModupUnit<SP>& x, const uint6
 template <uint32_t SP, uint32_t S1>
 GF_HD void modup_rs_unit(const ModupJob& j, uint32_t t, ModupUnit<SP>& x, const uint64_t* dv, uint64_t* cv) {
     static_assert(sizeof(RsTarget) == 7 * 8, "RsTarget layout");
-    static_assert(SP + 2 <= 8, "the column sums take at most 8 terms");
     const uint64_t* w = (const uint64_t*)j.tg + 7 * t;
     const uint64_t q = uniform_at(w, 0), qneg = uniform_at(w, 1);
     const bool f64 = uniform_at(j.ttwd, t) != 0;
@@ -372,7 +379,7 @@ GF_HD void modup_rs_unit(const ModupJob& j, uint32_t t, ModupUnit<SP>& x, const 
             x.hi[u][i] = opaque32(x.hi[u][i]);
         }
         // the sources, dv (below q_old < 2^60) and the centring flag as one
-        // sum of SP + 2 terms: REDC leaves it below 1.44 q + 1
+        // sum of SP + 2 terms: REDC leaves it below 1.44 q + 1 (6 sources; 1.88 q for 12)
         uint32_t al[SP + 2], ah[SP + 2];
 #pragma unroll
         for (uint32_t i = 0; i < SP; ++i) {
@@ -383,7 +390,7 @@ GF_HD void modup_rs_unit(const ModupJob& j, uint32_t t, ModupUnit<SP>& x, const 
         ah[SP] = split30_hi(dv[u]);
         al[SP + 1] = dv[u] > j.half ? 1u : 0u;
         ah[SP + 1] = 0;
-        const U128 acc = dot30<SP + 2>(al, ah, [&](uint32_t s) {
+        const U128 acc = dot30_any<SP + 2>(al, ah, [&](uint32_t s) {
             return s < SP ? uniform_at(j.tab, s * j.sc + t) : uniform_at(j.tsw, 2 * t + (s - SP));
         });
         const uint64_t v = redc_lazy(acc, q, qneg);

@@ -248,3 +248,42 @@ def test_fused_rescale(G, n, L, ascending, f64):
         s.sync()
         assert np.array_equal(o[0].download(), w[0]) and np.array_equal(o[1].download(), w[1]), level
         assert np.array_equal(d[1].download((level - 1) * n), w[1]), ("in place", level)
+
+
+@pytest.mark.parametrize("f64", [0, 1])
+@pytest.mark.parametrize("n,L,dnum", [(1 << 13, 24, 2), (1 << 14, 14, 2), (1 << 15, 10, 1), (1 << 16, 8, 1), (1 << 17, 9, 1)])
+def test_wide_digits(G, n, L, dnum, f64):
+    """Digits of 7 to 12 towers and 6 to 11 special primes: the fused forms'
+    widest sums, with levels whose digits hold few, six, seven and all towers."""
+    t = Setup(G, n, L, dnum, modup_f64=f64)
+    P, ctx, s = t.P, t.ctx, t.s
+    alpha = -(-L // dnum)
+    av, bv = t.hk[0]
+    ws = ctx.workspace()
+    levels = sorted({2, 6, 7, alpha, L} if n < 1 << 16 else {7, L})
+    for level in levels:
+        c = [t.ct(level) for _ in range(4)]
+        d = [G.Dev.of(x) for x in c]
+        o = [G.Dev(level * n) for _ in range(2)]
+        G.check(G.lib.gf_keyswitch(ctx.h, t.keys[0].h, level, d[0].ptr, o[0].ptr, o[1].ptr, ws.ptr, s.s))
+        s.sync()
+        w = P.keyswitch(level, c[0], av, bv)
+        assert np.array_equal(o[0].download(), w[0]) and np.array_equal(o[1].download(), w[1]), ("ks", level)
+        G.check(G.lib.gf_evalmult_rescale(ctx.h, t.keys[0].h, level, *[x.ptr for x in d], o[0].ptr, o[1].ptr, ws.ptr, s.s))
+        s.sync()
+        w = P.evalmult_rescale(level, *c, av, bv)
+        m = (level - 1) * n
+        assert np.array_equal(o[0].download(m), w[0]) and np.array_equal(o[1].download(m), w[1]), ("mult", level)
+    if n < 1 << 16:   # every level in one plan: narrow and wide digits in one stage
+        lv = list(range(2, L + 1))
+        c = [[t.ct(x) for _ in range(4)] for x in lv]
+        d = [[G.Dev.of(x) for x in v] for v in c]
+        o = [[G.Dev((x - 1) * n) for _ in range(2)] for x in lv]
+        wss = [ctx.workspace() for _ in lv]
+        plan = G.plan_evalmult_rescale(ctx, t.keys[0], lv, *[[x[j].ptr for x in d] for j in range(4)], [x[0].ptr for x in o],
+                                       [x[1].ptr for x in o], [w.ptr for w in wss])
+        plan.run(s)
+        s.sync()
+        for i in (0, 4, 5, alpha - 2, len(lv) - 1):
+            w = P.evalmult_rescale(lv[i], *c[i], av, bv)
+            assert np.array_equal(o[i][0].download(), w[0]) and np.array_equal(o[i][1].download(), w[1]), ("batch", lv[i])
