@@ -942,7 +942,7 @@ void Plan::run_jobs(size_t i, hipStream_t s, uint32_t which, uint32_t first, uin
         case Step::PTACC: launch_ptacc(GF_J(PtAccJob), cnt, n, s); break;
         case Step::NTT_FA: launch_ntt(GF_J(NttJob), cnt, geom, true, s, 1); break;
         case Step::KSI:
-            launch_ksi(GF_J(KsiJob), cnt, geom, st.arg & 0xFF, st.arg >> 8 & 0xFF, st.arg >> 16, s);
+            launch_ksi(GF_J(KsiJob), cnt, geom, st.arg & 0xFF, st.arg >> 8 & 0xFF, st.arg >> 16 & 3, st.arg >> 18, s);
             break;
         case Step::NTT_IB: launch_ntt(GF_J(NttJob), cnt, geom, false, s, 1); break;
         case Step::MODUP: launch_modup(GF_J(ModupJob), cnt, geom, st.arg, s); break;
@@ -2147,7 +2147,9 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
             const KsiJob* first = v.data() + steps[k].first;
             const uint32_t x = ksi_regions(*first), waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
             stage(Step::KSI, first, steps[k].second - steps[k].first, sizeof(KsiJob));
-            P->steps.back().arg = x | waves << 8 | ksi_form(*first) << 16;
+            uint32_t wide = 0;
+            for (size_t i = steps[k].first; i < steps[k].second; ++i) wide |= v[i].np == 5 || v[i].np == 6;
+            P->steps.back().arg = x | waves << 8 | ksi_form(*first) << 16 | wide << 18;
         }
     };
     stage_ksi(ksi_);

@@ -234,7 +234,8 @@ struct Step {
     size_t off;     // byte offset of the first job in the plan's device buffer
     uint32_t count;
     // KSI: the jobs' largest LDS region count (bits 0-7), waves per workgroup
-    // (bits 8-15), the jobs' form (bits 16-17: KSI_PLAIN, ..)
+    // (bits 8-15), the jobs' form (bits 16-17: KSI_PLAIN, ..), 1 << 18
+    // where some have 5 or 6 parts
     uint32_t arg = 0;
 };
 

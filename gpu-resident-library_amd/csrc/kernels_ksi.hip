@@ -1,57 +1,16 @@
-// The fused row pass of the keyswitch digits' forward transform and the key
-// inner product (ksi.hpp), with its launch.
-#include "ksi.hpp"
-#include "ntt_kernels.hpp"
+// The fused row pass of the keyswitch digits and the key inner product
+// (ksi_kernel.hpp), with its launch.
+#include "ksi_kernel.hpp"
 
 namespace gf {
 
-// ------------------------------------------- fused digit row pass + inner --
-// One wave's LDS region is private to it during the row passes.
-struct WaveSync {
-    __device__ void operator()() const { DevSync{}.wave(); }
-    __device__ void wave() const { DevSync{}.wave(); }
-};
-
-// At most 96 VGPRs (5 waves per SIMD, 20 per CU): every phase waits on memory
-// (row passes for twiddles, inner products for digits and keys), so the waves
-// in flight set the time.  Four parts with their last step take 5 waves of
-// 107 VGPRs uncapped: 64 EvalMult+Rescale at n = 2^16, L = 24 ran 8300 us with 4
-// waves per SIMD, 7570 with 5, 8280 with 6 (spills).
-// FIN: KSI_PLAIN, KSI_FIN, KSI_FIN_TENSOR.
-template <uint32_t S2, uint32_t RM, int FIN>
-__global__ __launch_bounds__(KSI_THREADS) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_ksi(const KsiJob* __restrict__ jobs, uint32_t off, uint32_t N1) {
-    extern __shared__ uint64_t lds[];
-    const KsiJob& j = jobs[off + blockIdx.y];
-    const uint32_t tid = threadIdx.x, nthr = blockDim.x;
-    auto go = [&](auto L) {
-        ksi_body<S2, RM, decltype(L)::value, WaveSync, DevSync, FIN>(j, N1, blockIdx.x, lds, tid >> 6, nthr >> 6,
-                                                                     tid & 63, 64, tid, nthr, WaveSync{}, DevSync{});
-    };
-    if (j.red) go(std::true_type{});
-    else go(std::false_type{});
-}
-
-void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, uint32_t fin, hipStream_t s) {
+void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, uint32_t fin, bool wide,
+                hipStream_t s) {
     if (g.single || g.n % KSI_TILE) throw std::runtime_error("gpufhe: fused inner product needs a two-phase ring");
     if (regions > KSI_MAXP || waves < 1 || waves > KSI_WAVES)
         throw std::runtime_error("gpufhe: fused inner product launch shape out of range");
-    const size_t shm = (size_t)regions * KSI_PART_WORDS * 8;
-    bool ok = with_radix(g.rmax, [&](auto Rc) {
-        constexpr uint32_t RM = decltype(Rc)::value;
-        const bool geom_ok = with_split(g.logN1, g.logN2, [&](auto, auto B) {
-            constexpr uint32_t S2 = decltype(B)::value;
-            for (uint32_t off = 0; off < nj; off += MAXY) {
-                const uint32_t cnt = nj - off < MAXY ? nj - off : MAXY;
-                const dim3 grid(g.n / KSI_TILE, cnt);
-                if (fin == KSI_FIN_TENSOR) k_ksi<S2, RM, KSI_FIN_TENSOR><<<grid, 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
-                else if (fin) k_ksi<S2, RM, KSI_FIN><<<grid, 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
-                else k_ksi<S2, RM, KSI_PLAIN><<<grid, 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
-            }
-        });
-        if (!geom_ok) throw std::runtime_error("gpufhe: unsupported ring dimension for the NTT");
-    });
-    if (!ok) throw std::runtime_error("gpufhe: unsupported NTT radix");
+    if (wide) launch_ksi_wide(d, nj, g, regions, waves, fin, s);
+    else run_ksi<4>(d, nj, g, regions, waves, fin, s);
 }
-
 
 }  // namespace gf

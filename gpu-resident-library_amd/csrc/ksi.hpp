@@ -10,7 +10,7 @@
 // block barrier every thread (including an optional extra wave that runs no
 // row pass) takes KSI_TILE / nthr positions and accumulates
 // sum_p digit_p * key_p for both key components (30-bit column sums where
-// every value is below 2^60 and there are at most 4 parts, else 128-bit sums).  A launch
+// every value is below 2^60 and there are at most 6 parts, else 128-bit sums).  A launch
 // gives its jobs one wave per transformed part (up to KSI_WAVES), so no wave
 // idles through the row passes.  The transformed digits therefore never
 // travel through HBM.  Parts whose tower i is the input's own (no transform)
@@ -166,7 +166,7 @@ enum { KSI_PLAIN = 0, KSI_FIN = 1, KSI_FIN_TENSOR = 2 };
 
 // the jobs whose last step may form the tensor products itself: the column
 // sums' form of the inner product with two positions per access
-inline bool ksi_tensor_here(const KsiJob& j) { return j.fin.v[0] && j.d30 && j.np <= 4 && j.pairs; }
+inline bool ksi_tensor_here(const KsiJob& j) { return j.fin.v[0] && j.d30 && j.np <= 6 && j.pairs; }
 
 // The tensor products of one position: t0, t1 for the lazy Shoup products and
 // t2 as a digit below 2^60.  fp64 rows: exact products in (-q, q) each, shifted
@@ -349,7 +349,7 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
 }
 
 // ksi_inner_cols for the job's part count, when it has an instantiation
-template <uint32_t V, bool LZ, int FIN>
+template <uint32_t V, bool LZ, int FIN, int NPMAX>
 GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t tid, uint32_t nthr,
                              const NttJob& t) {
     switch (j.np) {
@@ -357,6 +357,21 @@ GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint3
         case 2: ksi_inner_cols<2, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
         case 3: ksi_inner_cols<3, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
         case 4: ksi_inner_cols<4, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
+        // 5 and 6 parts take one position per access (two need more registers
+        // than 5 waves per SIMD leave), in kernels of their own (NPMAX = 6):
+        // beside the others their operands' scalar loads spill 180 SGPRs more
+        case 5:
+            if constexpr (NPMAX >= 5) {
+                ksi_inner_cols<5, 1, LZ, FIN>(j, lds, off, tid, nthr, t);
+                return true;
+            }
+            return false;
+        case 6:
+            if constexpr (NPMAX >= 6) {
+                ksi_inner_cols<6, 1, LZ, FIN>(j, lds, off, tid, nthr, t);
+                return true;
+            }
+            return false;
         default: return false;
     }
 }
@@ -364,7 +379,7 @@ GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint3
 // LZ = (j.red != 0), FIN = KSI_FIN where j.fin.v[0] is set, KSI_FIN_TENSOR
 // where j.fin.in[0] is too, else KSI_PLAIN.  The wave-level sync wsync separates the row passes of
 // one wave's region; bsync is the workgroup barrier before the inner product.
-template <uint32_t S2, uint32_t RM, bool LZ, class WSync, class BSync, int FIN = KSI_PLAIN>
+template <uint32_t S2, uint32_t RM, bool LZ, class WSync, class BSync, int FIN = KSI_PLAIN, int NPMAX = 4>
 GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, uint32_t wave, uint32_t nwaves,
                     uint32_t lane, uint32_t wlanes, uint32_t tid, uint32_t nthr, WSync wsync, BSync bsync) {
     constexpr uint32_t ROWS = KSI_TILE >> S2, LOGR = KSI_LOG_TILE - S2;
@@ -405,11 +420,11 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
         t.c1p = j.fin.cep;
     }
     bsync();
-    // up to 4 parts with every value below 2^60: column sums, loads first
+    // up to 6 parts with every value below 2^60: column sums, loads first
     bool done = false;
     if (j.d30)
-        done = FIN == KSI_FIN_TENSOR || j.pairs ? ksi_inner_cols_np<2, LZ, FIN>(j, lds, off, tid, nthr, t)
-                                                : ksi_inner_cols_np<1, LZ, FIN>(j, lds, off, tid, nthr, t);
+        done = FIN == KSI_FIN_TENSOR || j.pairs ? ksi_inner_cols_np<2, LZ, FIN, NPMAX>(j, lds, off, tid, nthr, t)
+                                                : ksi_inner_cols_np<1, LZ, FIN, NPMAX>(j, lds, off, tid, nthr, t);
     // positions idx .. idx + V - 1 per step (V = 2: one 16-byte access per operand)
     auto inner = [&](auto Vc) {
         constexpr uint32_t V = decltype(Vc)::value;
