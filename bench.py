@@ -233,7 +233,7 @@ def cpu_baseline(q, p, roots, av, bv, seconds=12.0, threads=1):
 def host_threads():
     """CPU threads for the multi-core baseline: the cores this process may run
     on (its affinity mask), limited by the job's thread allowance
-    OMP_NUM_THREADS when that is set (the GPU box sets it to its CPU share)."""
+    OMP_NUM_THREADS when that is set (a machine that is shared sets it to the CPU share)."""
     n = len(os.sched_getaffinity(0))
     env = os.environ.get("OMP_NUM_THREADS")
     if env and env.isdigit() and int(env) > 0:

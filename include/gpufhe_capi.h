@@ -283,8 +283,8 @@ int gf_plan_run_step_kernel(gf_plan* p, uint32_t i, uint32_t which, hipStream_t 
 
 /* ---- tuning ----
  * NTT register radix log2 (2, 3 or 4) used by plans built afterwards; the
- * autotuner times each on a synthetic 256 MiB tower batch (forward and
- * inverse, in place) and keeps the fastest; ms_out is per 96 towers. */
+ * autotuner times 2 and 3 on a synthetic 256 MiB tower batch (forward and
+ * inverse, in place) and keeps the faster; ms_out is per 96 towers. */
 int gf_ctx_set_ntt_radix(gf_ctx* c, uint32_t rmax);
 uint32_t gf_ctx_get_ntt_radix(const gf_ctx* c);
 int gf_ctx_autotune(gf_ctx* c, hipStream_t s, uint32_t* rmax_out, float* ms_out);
@@ -301,12 +301,16 @@ int gf_ctx_autotune(gf_ctx* c, hipStream_t s, uint32_t* rmax_out, float* ms_out)
  * prologue and surviving towers' forward column pass as one kernel, 0/1),
  * "tensor_ib" (with modup_fused, the tensor product and the inverse row pass
  * of its t2 as one kernel per row tile, 0/1), "ksi_rowpass" (with
- * moddown_fused, the P part's inverse row pass inside the P rows' inner
- * product launch, from its LDS, 0/1).
+ * moddown_fused, the P part's and the dropped tower's inverse row passes
+ * inside the inner product launch, from its LDS, 0/1).
  * The report is JSON with every candidate's time, the radix search of
  * gf_ctx_autotune included; valid until the next tuning call.  Knobs (and
- * "ntt_radix", "rechunk_wgs", "modup_min_wgs") can be set by name; plans built
- * afterwards use them, and results are identical for every setting. */
+ * "ntt_radix", "rechunk_wgs", "modup_min_wgs", "modup_split_wgs" (workgroups a
+ * fused ModUp or ModDown stage splits its targets for), "ksi_fin" (the Q rows'
+ * inner products in the launch of the outputs' row passes, 0/1), "ksi_tensor"
+ * (with it, the tensor products formed there too, 0/1)) can be set by name;
+ * plans built afterwards use them, and results are identical for every
+ * setting. */
 int gf_ctx_autotune_plan(gf_ctx* c, uint32_t batch, hipStream_t s);
 const char* gf_ctx_tuning_report(const gf_ctx* c);
 int gf_ctx_set_knob(gf_ctx* c, const char* name, uint32_t value);
