@@ -162,7 +162,9 @@ inline uint32_t ksi_d30(uint64_t q, uint64_t red) {
 // positions, whose digits it has already read
 // the forms of the kernel: inner products stored (or through rp), with the
 // rows' last step, and with the tensor products formed there
-enum { KSI_PLAIN = 0, KSI_FIN = 1, KSI_FIN_TENSOR = 2 };
+// KSI_FIN_TENSOR_IN: KSI_FIN_TENSOR with the input towers' tile through LDS
+// (ksi_request_inputs), a launch's choice (run_ksi)
+enum { KSI_PLAIN = 0, KSI_FIN = 1, KSI_FIN_TENSOR = 2, KSI_FIN_TENSOR_IN = 3 };
 
 // the jobs whose last step may form the tensor products itself: the column
 // sums' form of the inner product with two positions per access
@@ -186,6 +188,34 @@ GF_HD void ksi_tensor(const KsiJob& j, const uint64_t* x, uint64_t& t0, uint64_t
     t.qneg = j.qneg;
     t.r2 = j.fin.r2;
     tensor_one(t, x[0], x[1], x[2], x[3], t0, t1, t2);
+}
+
+// The four input towers' tile of a last step that forms the tensor products
+// goes to LDS behind the job's regions, straight from HBM, requested before the
+// row passes: one round trip to HBM less behind the barrier, and no registers
+// held for it.
+enum { KSI_IN_WORDS = 4 * KSI_TILE, KSI_IN_CHUNK = 128 };   // a chunk: one 16-byte access per lane
+GF_HD uint32_t ksi_in_off(const KsiJob& j) { return ((uint32_t)__builtin_popcount(j.xf) + 2) * KSI_PART_WORDS; }
+GF_HD void ksi_request_inputs(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t wave, uint32_t nwaves,
+                              uint32_t lane) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    for (uint32_t c = __builtin_amdgcn_readfirstlane(wave); c < KSI_IN_WORDS / KSI_IN_CHUNK; c += nwaves) {
+        const uint32_t k = c / (KSI_TILE / KSI_IN_CHUNK), o = c % (KSI_TILE / KSI_IN_CHUNK) * KSI_IN_CHUNK;
+        const GF_GLOBAL uint64_t* src = gcast(j.fin.in[k]) + off + o + 2 * lane;
+        __builtin_amdgcn_global_load_lds((const GF_GLOBAL void*)src,
+                                         (__attribute__((address_space(3))) void*)(lds + ksi_in_off(j) + c * KSI_IN_CHUNK),
+                                         16, 0, 0);
+    }
+#else
+    for (uint32_t i = wave * 64 + lane; i < KSI_IN_WORDS; i += nwaves * 64)
+        lds[ksi_in_off(j) + i] = j.fin.in[i / KSI_TILE][off + i % KSI_TILE];
+#endif
+}
+// this wave's requests have arrived (the workgroup barrier follows)
+GF_HD void ksi_wait_inputs() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
 }
 
 template <uint32_t V>
@@ -212,7 +242,7 @@ GF_HD void ksi_store(const KsiJob& j, uint64_t* lds, uint32_t idx, uint32_t gi, 
         const uint32_t k0 = (uint32_t)__builtin_popcount(j.xf) * KSI_PART_WORDS;
         auto comp = [&](uint32_t c, const uint64_t* r, const uint64_t* e) {
             uint64_t y[V];
-            const int ep = FIN == KSI_FIN_TENSOR || !j.fin.e_plain ? 0 : j.fin.e[c] ? 1 : 2;
+            const int ep = FIN >= KSI_FIN_TENSOR || !j.fin.e_plain ? 0 : j.fin.e[c] ? 1 : 2;
 #pragma unroll
             for (uint32_t v = 0; v < V; ++v) {
                 const uint64_t z = lds[k0 + c * KSI_PART_WORDS + padded(idx + v)];
@@ -289,7 +319,7 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
             if (xf[p]) {
 #pragma unroll
                 for (uint32_t v = 0; v < V; ++v) dv[p][v] = lds[reg[p] + padded(idx + v)];
-            } else if constexpr (FIN != KSI_FIN_TENSOR) {
+            } else if constexpr (FIN < KSI_FIN_TENSOR) {
                 load_words_any<V>(src[p], gi, j, dv[p]);
             }
             load_words<V>(kb[p], gi, bv[p]);
@@ -297,10 +327,17 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
         }
         KsiEps<V> ep;
         ksi_load_eps<FIN, V>(j, gi, ep);
-        if constexpr (FIN == KSI_FIN_TENSOR) {
+        if constexpr (FIN >= KSI_FIN_TENSOR) {
             uint64_t x[4][V];
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) load_words<V>(gcast(j.fin.in[k]), gi, x[k]);
+            for (uint32_t k = 0; k < 4; ++k) {
+                if constexpr (FIN == KSI_FIN_TENSOR_IN) {
+#pragma unroll
+                    for (uint32_t v = 0; v < V; ++v) x[k][v] = lds[ksi_in_off(j) + k * KSI_TILE + idx + v];
+                } else {
+                    load_words<V>(gcast(j.fin.in[k]), gi, x[k]);
+                }
+            }
 #pragma unroll
             for (uint32_t v = 0; v < V; ++v) {
                 const uint64_t y[4] = {x[0][v], x[1][v], x[2][v], x[3][v]};
@@ -405,6 +442,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
         ++k;
     };
     const uint32_t np = j.np, rows = FIN ? np + 2 : np;
+    if constexpr (FIN == KSI_FIN_TENSOR_IN) ksi_request_inputs(j, lds, off, wave, nwaves, lane);
     for (uint32_t p = 0; p < rows; ++p) {
         if (p < np) {
             if ((j.xf >> p) & 1) row_pass(j.src[p]);
@@ -419,11 +457,12 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
         t.c1 = j.fin.ce;
         t.c1p = j.fin.cep;
     }
+    if constexpr (FIN == KSI_FIN_TENSOR_IN) ksi_wait_inputs();
     bsync();
     // up to 6 parts with every value below 2^60: column sums, loads first
     bool done = false;
     if (j.d30)
-        done = FIN == KSI_FIN_TENSOR || j.pairs ? ksi_inner_cols_np<2, LZ, FIN, NPMAX>(j, lds, off, tid, nthr, t)
+        done = FIN >= KSI_FIN_TENSOR || j.pairs ? ksi_inner_cols_np<2, LZ, FIN, NPMAX>(j, lds, off, tid, nthr, t)
                                                 : ksi_inner_cols_np<1, LZ, FIN, NPMAX>(j, lds, off, tid, nthr, t);
     // positions idx .. idx + V - 1 per step (V = 2: one 16-byte access per operand)
     auto inner = [&](auto Vc) {
@@ -470,7 +509,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
             ksi_store<FIN, LZ, V>(j, lds, idx, gi, r0, r1, ep, t);
         }
     };
-    if (FIN != KSI_FIN_TENSOR && !done) {   // (those jobs have the column sums' form)
+    if (FIN < KSI_FIN_TENSOR && !done) {   // (those jobs have the column sums' form)
         if (j.pairs) inner(std::integral_constant<uint32_t, 2>{});
         else inner(std::integral_constant<uint32_t, 1>{});
     }
