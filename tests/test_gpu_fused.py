@@ -287,3 +287,25 @@ def test_wide_digits(G, n, L, dnum, f64):
         for i in (0, 4, 5, alpha - 2, len(lv) - 1):
             w = P.evalmult_rescale(lv[i], *c[i], av, bv)
             assert np.array_equal(o[i][0].download(), w[0]) and np.array_equal(o[i][1].download(), w[1]), ("batch", lv[i])
+
+
+@pytest.mark.parametrize("f64", [0, 1])
+@pytest.mark.parametrize("n,L,dnum,count", [(1 << 13, 8, 4, 24), (1 << 14, 5, 5, 12), (1 << 17, 4, 4, 4)])
+def test_last_step_inputs_through_lds(G, n, L, dnum, count, f64):
+    """Products of 4 and 5 parts, whose last step brings the input towers into
+    LDS, beside products of fewer parts (levels below), which may share the
+    launch: tiles at both ends of the ring, each output against the oracle's."""
+    t = Setup(G, n, L, dnum, modup_f64=f64)
+    lv = [L - 2 * (i % 2) for i in range(count)]
+    c = [[t.ct(x) for _ in range(4)] for x in lv]
+    d = [[G.Dev.of(x) for x in v] for v in c]
+    o = [[G.Dev((x - 1) * n) for _ in range(2)] for x in lv]
+    ws = [t.ctx.workspace() for _ in range(count)]
+    plan = G.plan_evalmult_rescale(t.ctx, t.keys[0], lv, *[[x[j].ptr for x in d] for j in range(4)],
+                                   [x[0].ptr for x in o], [x[1].ptr for x in o], [w.ptr for w in ws])
+    assert plan.steps()[-1][0] == "ksi", plan.steps()
+    plan.run(t.s)
+    t.s.sync()
+    for i in sorted({0, 1, count - 2, count - 1}):
+        w = t.P.evalmult_rescale(lv[i], *c[i], *t.hk[0])
+        assert np.array_equal(o[i][0].download(), w[0]) and np.array_equal(o[i][1].download(), w[1]), i
