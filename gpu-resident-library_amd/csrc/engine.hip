@@ -322,12 +322,18 @@ size_t Ctx::rescale_ws_words() const { return (size_t)L * n; }
 void Ctx::set_radix(uint32_t r) {
     if (r < 2 || r > 4) throw std::runtime_error("gpufhe: NTT radix log2 must be 2, 3 or 4");
     std::vector<RowTables> t(L + K);
-    for (uint32_t i = 0; i < L + K; ++i) t[i] = row_tables(n, mods[i], roots[i], r);
+    for (uint32_t i = 0; i < L + K; ++i) t[i] = row_tables(n, mods[i], roots[i], row_radix(r));
     geom = make_geom(n, r);
     rtr = std::move(t);
     row_of_.clear();
+    big_row_of_.clear();
     f64_of_.clear();
     for (uint32_t i = 0; i < L + K; ++i) {
+        if (r == 4 && !geom.single) {
+            const RowTables b = row_tables(n, mods[i], roots[i], r);
+            big_row_of_[rt[i].fw2] = b.fwd;
+            big_row_of_[rt[i].iv2] = b.inv;
+        }
         row_of_[rt[i].fw2] = rtr[i].fwd;
         row_of_[rt[i].iv2] = rtr[i].inv;
         if (!rt[i].fw2d) continue;
@@ -342,6 +348,19 @@ const uint64_t* Ctx::row_table_of(const uint64_t* paired) const {
     const auto it = row_of_.find(paired);
     return it == row_of_.end() ? nullptr : it->second;
 }
+const uint64_t* Ctx::big_row_table_of(const uint64_t* paired) const {
+    const auto it = big_row_of_.find(paired);
+    return it == big_row_of_.end() ? nullptr : it->second;
+}
+// A row pass at radix 2^4 on 4096-element tiles, from this many workgroups on, else
+// at 2^3 on 1024-element tiles.  Both sides, 4096 / 1024: 640 workgroups forward
+// 13.6 / 13.1 us at n = 2^13, 14.8 / 14.2 at 2^16; 768 13.8 / 14.4 and 15.1 / 16.2; 1536
+// 24.1 / 25.6 and 26.4 / 28.2; inverse 384 10.2 / 9.7 and 11.0 / 10.3; 768 15.1 / 16.9 and
+// 16.6 / 17.4.
+enum { NTT_ROWS_WGS = 768 };
+bool Ctx::big_row_tiles(size_t towers) const {
+    return geom.rmax == 4 && !geom.single && towers * (n >> NTT_LOG_TILE_BIG) >= NTT_ROWS_WGS;
+}
 const uint64_t* Ctx::f64_table_of(const uint64_t* paired) const {
     const auto it = f64_of_.find(paired);
     return it == f64_of_.end() ? nullptr : it->second;
@@ -351,15 +370,12 @@ uint32_t Ctx::autotune(hipStream_t s, float* best_ms) {
     // 256 MiB of towers (enough workgroups to fill the chip several times
     // over, as the batched stages do) cycling through every modulus, forward
     // then inverse, in place; each radix is timed twice, interleaved, and
-    // keeps its faster round.  Radix 2^4 is not a candidate: its 16-element
-    // units leave three quarters of a 1024-element row tile's lanes idle (64
-    // EvalMult+Rescale at n = 2^16, L = 24: 9156 us, 7519 at 2^3, 7549 at 2^2),
-    // which whole transforms alone, bound by memory here, do not show.
+    // keeps its faster round.
     const uint32_t towers = std::max<uint32_t>(96, (1u << 25) / n);
     DevBuf buf((size_t)towers * n * 8);
     // job arrays per radix (the row tables differ): [r - 2][fwd towers, inv towers]
     std::vector<NttJob> jobs;
-    for (uint32_t r = 2; r <= 3; ++r)
+    for (uint32_t r = 2; r <= 4; ++r)
         for (int inv = 0; inv < 2; ++inv)
             for (uint32_t t = 0; t < towers; ++t) {
                 const uint32_t m = t % (L + K);
@@ -381,16 +397,17 @@ uint32_t Ctx::autotune(hipStream_t s, float* best_ms) {
     float bms = 1e30f;
     float per[5] = {1e30f, 1e30f, 1e30f, 1e30f, 1e30f};
     for (int round = 0; round < 2; ++round)
-        for (uint32_t r = 2; r <= 3; ++r) {
+        for (uint32_t r = 2; r <= 4; ++r) {
             NttGeom g = make_geom(n, r);
+            const bool big = r == 4;   // (towers is above big_row_tiles' line at every n)
             const NttJob* fw = dj.as<NttJob>() + (size_t)(r - 2) * 2 * towers;
             const NttJob* iv = fw + towers;
-            launch_ntt(fw, towers, g, true, s);   // warm
-            launch_ntt(iv, towers, g, false, s);
+            launch_ntt(fw, towers, g, true, s, 3, big);   // warm
+            launch_ntt(iv, towers, g, false, s, 3, big);
             hip_check(hipEventRecord(e0, s), "event");
             for (int rep = 0; rep < 3; ++rep) {
-                launch_ntt(fw, towers, g, true, s);
-                launch_ntt(iv, towers, g, false, s);
+                launch_ntt(fw, towers, g, true, s, 3, big);
+                launch_ntt(iv, towers, g, false, s, 3, big);
             }
             hip_check(hipEventRecord(e1, s), "event");
             hip_check(hipEventSynchronize(e1), "event sync");
@@ -405,7 +422,7 @@ uint32_t Ctx::autotune(hipStream_t s, float* best_ms) {
     {
         std::ostringstream o;
         o << "{\"workload_towers\": " << towers << ", \"ms_per_fwd_inv_pass\": {";
-        for (uint32_t r = 2; r <= 3; ++r) o << (r > 2 ? ", " : "") << "\"" << r << "\": " << per[r] / 3;
+        for (uint32_t r = 2; r <= 4; ++r) o << (r > 2 ? ", " : "") << "\"" << r << "\": " << per[r] / 3;
         o << "}, \"chosen\": " << best << "}";
         radix_report = o.str();
     }
@@ -926,8 +943,8 @@ void Plan::run_jobs(size_t i, hipStream_t s, uint32_t which, uint32_t first, uin
     if (st.kind != Step::NTT_F && st.kind != Step::NTT_I && !(which & 1)) return;
 #define GF_J(T) ((const T*)p + first)
     switch (st.kind) {
-        case Step::NTT_F: launch_ntt(GF_J(NttJob), cnt, geom, true, s, which); break;
-        case Step::NTT_I: launch_ntt(GF_J(NttJob), cnt, geom, false, s, which); break;
+        case Step::NTT_F: launch_ntt(GF_J(NttJob), cnt, geom, true, s, which, st.arg & 1); break;
+        case Step::NTT_I: launch_ntt(GF_J(NttJob), cnt, geom, false, s, which, st.arg & 1); break;
         case Step::TENSOR: launch_tensor(GF_J(TensorJob), cnt, n, s); break;
         case Step::TENSOR_IB: launch_tensor_ib(GF_J(TensorIbJob), cnt, geom, s); break;
         case Step::CONV: launch_conv(GF_J(ConvJob), cnt, n, s); break;
@@ -1974,6 +1991,11 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
             if (!j.twr && !C_.geom.single) throw std::runtime_error("gpufhe: transform table of another context");
         }
     }
+    // whole transforms of large launches: their row pass on big tiles (ntt_v_'s,
+    // with their epilogue, stay on small ones: Ctx::big_row_tiles)
+    for (auto* v : {&intt_up_, &intt_p_, &intt_drop_, &ntt_dig_, &ntt_conv_, &ntt_sw_})
+        if (C_.big_row_tiles(v->size()))
+            for (NttJob& j : *v) j.twr = C_.big_row_table_of(j.tw);
     // forward transforms over moduli below 2^57 skip the butterflies'
     // conditional subtractions; the digits stay unreduced for the inner product
     for (auto* v : {&ntt_dig_, &ntt_diga_, &ntt_digb_, &ntt_conv_, &ntt_sw_, &ntt_v_, &ntt_vb_, &ntt_rsb_})
@@ -2048,6 +2070,11 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         P->steps.push_back(Step{kind, off, (uint32_t)cnt});
     };
 #define GF_STAGE(k, v) stage(Step::k, v.data(), v.size(), sizeof(v[0]))
+    auto stage_whole = [&](Step::Kind kind, const std::vector<NttJob>& v) {
+        if (v.empty()) return;
+        stage(kind, v.data(), v.size(), sizeof(NttJob));
+        P->steps.back().arg = C_.big_row_tiles(v.size());
+    };
     // one launch for every source count (per conversion reduction, and 7 or
     // more sources apart), the longest jobs first
     auto stage_modup = [&](Step::Kind kind, std::vector<ModupJob>& v) {
@@ -2109,10 +2136,10 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
     GF_STAGE(TENSOR, tensor_);
     GF_STAGE(PERM, perm_);
     GF_STAGE(NTT_IB, intt_upb_);
-    GF_STAGE(NTT_I, intt_up_);
+    stage_whole(Step::NTT_I, intt_up_);
     stage_modup(Step::MODUP, modup_);
     GF_STAGE(CONV, conv_up_);
-    GF_STAGE(NTT_F, ntt_dig_);
+    stage_whole(Step::NTT_F, ntt_dig_);
     GF_STAGE(NTT_FA, ntt_diga_);
     GF_STAGE(NTT_FB, ntt_digb_);
     GF_STAGE(INNER, inner_);
@@ -2153,18 +2180,18 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         }
     };
     stage_ksi(ksi_);
-    GF_STAGE(NTT_I, intt_p_);
+    stage_whole(Step::NTT_I, intt_p_);
     GF_STAGE(NTT_IB, intt_pb_);
     stage_modup(Step::MODDOWN, moddown_);
     stage_modup(Step::KSDOWN, ksdown_);
     GF_STAGE(CONV, conv_dn_);
-    GF_STAGE(NTT_F, ntt_conv_);
+    stage_whole(Step::NTT_F, ntt_conv_);
     GF_STAGE(COMBINE, combine_);
     GF_STAGE(ADD, add_rot_);
     GF_STAGE(COPY, copy_rot_);
-    GF_STAGE(NTT_I, intt_drop_);
+    stage_whole(Step::NTT_I, intt_drop_);
     GF_STAGE(SWITCH, switch_);
-    GF_STAGE(NTT_F, ntt_sw_);
+    stage_whole(Step::NTT_F, ntt_sw_);
     GF_STAGE(FUSE, fuse_);
     GF_STAGE(NTT_IB, intt_dropb_);
     stage_modup(Step::MODDOWN, rsdown_);

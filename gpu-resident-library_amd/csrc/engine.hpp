@@ -117,16 +117,24 @@ public:
     // digit row pass feeds the key inner product directly (KSI)
     bool fused = true;
     uint32_t wide = 0;                        // 1: a modulus is 2^60 or more (generic conversion sums)
-    std::vector<RowTables> rtr;               // per row: phase-B row tables for geom.rmax
+    std::vector<RowTables> rtr;               // per row: phase-B row tables for row_radix(geom.rmax)
     // register radix of transforms in plans built from now on (2..4)
     void set_radix(uint32_t r);
     // the row table matching a paired table of this context (fw2, iv2, or
     // their fp64 pairs fw2d, iv2d), else null
     const uint64_t* row_table_of(const uint64_t* paired) const;
+    // Whether the row pass of a launch of this many whole transforms takes
+    // 4096-element tiles and radix 2^4 (over big_row_table_of their tables): at
+    // radix 2^4, from NTT_ROWS_WGS such workgroups on.  A forward transform
+    // with an epilogue does not: its row pass waits for the epilogue's operands,
+    // with more workgroups per CU on 1024-element tiles (176 towers at n = 2^16:
+    // 70.5 us on 4096, 67.2 on 1024).
+    bool big_row_tiles(size_t towers) const;
+    const uint64_t* big_row_table_of(const uint64_t* paired) const;
     // the fp64 pairs of the same twiddles as a paired table (fw2 -> fw2d,
     // iv2 -> iv2d), null for moduli of 2^50 and above
     const uint64_t* f64_table_of(const uint64_t* paired) const;
-    std::unordered_map<const uint64_t*, const uint64_t*> row_of_, f64_of_;   // what those two look up (set_radix)
+    std::unordered_map<const uint64_t*, const uint64_t*> row_of_, big_row_of_, f64_of_;   // what those look up (set_radix)
     uint32_t row_q(uint32_t i) const { return i; }
     uint32_t row_p(uint32_t k) const { return L + k; }
     uint32_t num_parts(uint32_t l) const { return (l + alpha - 1) / alpha; }
@@ -235,7 +243,8 @@ struct Step {
     uint32_t count;
     // KSI: the jobs' largest LDS region count (bits 0-7), waves per workgroup
     // (bits 8-15), the jobs' form (bits 16-17: KSI_PLAIN, ..), 1 << 18
-    // where some have 5 or 6 parts
+    // where some have 5 or 6 parts.  NTT_I: 1: row passes on big tiles
+    // (Ctx::big_row_tiles)
     uint32_t arg = 0;
 };
 

@@ -204,8 +204,9 @@ inline void hip_check(hipError_t e, const char* what) {
 // batched launches (jobs in device memory)
 // which: 3 = the whole transform; 1 / 2 = only its first / second kernel
 // (two-phase rings; a single-phase ring has one kernel, run when bit 0 is set)
+// big_rows: see Ctx::big_row_tiles
 void launch_ntt(const NttJob* d_jobs, uint32_t njobs, const NttGeom& g, bool fwd, hipStream_t s,
-                uint32_t which = 3);
+                uint32_t which = 3, bool big_rows = false);
 void launch_ntt_one(const NttJob& job, const NttGeom& g, bool fwd, hipStream_t s);
 void launch_tensor(const TensorJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 void launch_conv(const ConvJob* d, uint32_t nj, uint32_t n, hipStream_t s);

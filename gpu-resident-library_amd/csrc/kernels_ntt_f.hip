@@ -3,10 +3,10 @@
 
 namespace gf {
 
-void launch_ntt_fwd(const NttJob* d_jobs, uint32_t njobs, const NttGeom& g, hipStream_t s, uint32_t which) {
+void launch_ntt_fwd(const NttJob* d_jobs, uint32_t njobs, const NttGeom& g, hipStream_t s, uint32_t which, bool big_rows) {
     for (uint32_t off = 0; off < njobs; off += MAXY) {
         const uint32_t cnt = njobs - off < MAXY ? njobs - off : MAXY;
-        ntt_dispatch_dir<true, true>(JobsDev{d_jobs, off}, cnt, g, s, which);
+        ntt_dispatch_dir<true, true>(JobsDev{d_jobs, off}, cnt, g, s, which, big_rows);
     }
 }
 

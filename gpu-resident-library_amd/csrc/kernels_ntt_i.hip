@@ -24,7 +24,7 @@ __global__ __launch_bounds__(NTT_THREADS) __attribute__((amdgpu_waves_per_eu(4, 
 void launch_tensor_ib(const TensorIbJob* d, uint32_t nj, const NttGeom& g, hipStream_t s) {
     if (g.single || g.R * (1u << g.logN2) != NTT_TILE)
         throw std::runtime_error("gpufhe: the fused tensor + row pass needs a two-phase ring");
-    bool ok = with_radix(g.rmax, [&](auto Rc) {
+    bool ok = with_row_radix(g.rmax, [&](auto Rc) {
         constexpr uint32_t RM = decltype(Rc)::value;
         const bool geom_ok = with_split(g.logN1, g.logN2, [&](auto, auto B) {
             constexpr uint32_t S2 = decltype(B)::value;
@@ -38,10 +38,10 @@ void launch_tensor_ib(const TensorIbJob* d, uint32_t nj, const NttGeom& g, hipSt
     if (!ok) throw std::runtime_error("gpufhe: unsupported NTT radix");
 }
 
-void launch_ntt_inv(const NttJob* d_jobs, uint32_t njobs, const NttGeom& g, hipStream_t s, uint32_t which) {
+void launch_ntt_inv(const NttJob* d_jobs, uint32_t njobs, const NttGeom& g, hipStream_t s, uint32_t which, bool big_rows) {
     for (uint32_t off = 0; off < njobs; off += MAXY) {
         const uint32_t cnt = njobs - off < MAXY ? njobs - off : MAXY;
-        ntt_dispatch_dir<false, true>(JobsDev{d_jobs, off}, cnt, g, s, which);
+        ntt_dispatch_dir<false, true>(JobsDev{d_jobs, off}, cnt, g, s, which, big_rows);
     }
 }
 

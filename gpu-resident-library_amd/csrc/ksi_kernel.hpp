@@ -43,7 +43,7 @@ inline void run_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t reg
     // no faster (chains of three parts 2797 -> 2814 us, two parts 157.3 -> 159.7).
     const bool in = fin == KSI_FIN_TENSOR && (NPMAX > 4 || regions >= 5);
     const size_t shm = ((size_t)regions * KSI_PART_WORDS + (in ? KSI_IN_WORDS : 0)) * 8;
-    bool ok = with_radix(g.rmax, [&](auto Rc) {
+    bool ok = with_row_radix(g.rmax, [&](auto Rc) {
         constexpr uint32_t RM = decltype(Rc)::value;
         const bool geom_ok = with_split(g.logN1, g.logN2, [&](auto, auto B) {
             constexpr uint32_t S2 = decltype(B)::value;

@@ -132,25 +132,34 @@ struct NttGeom {
     uint32_t C;             // columns per phase-A tile of NTT_TILE
     uint32_t R;             // rows per phase-B tile
     uint32_t single;        // 1: whole tower in one tile
-    uint32_t rmax;          // largest register radix log2 (tuning knob, 2..4)
+    uint32_t rmax;          // largest register radix log2 (tuning knob, 2..4; row_radix)
 };
 
-// Tiles of 1024 elements.  A row pass needs nothing larger (its rows are
-// contiguous): the smaller tile keeps 8.5 KiB of LDS and short register
+// Tiles of 1024 elements.  A row pass up to radix 2^3 needs nothing larger (its
+// rows are contiguous): the smaller tile keeps 8.5 KiB of LDS and short register
 // passes, so more workgroups share a CU and a single operation's few towers
-// spread over 4 times as many CUs as with 4096 (the epilogue row pass of 4
-// towers at n = 2^14: 12.2 -> 7.9 us; of 2944 towers at n = 2^16: unchanged, at
-// the copy rate).  A column pass of a launch that fills the chip takes
-// 4096-element tiles (NTT_LOG_TILE_COLS): their rows of 2^(12 - S1) words are
-// whole L2 lines at n = 2^16 (column passes of 8 operations at L = 24, dnum = 2:
-// 1390 us a pass with them, 1677 with 1024).
+// spread over 4 times as many CUs as with 4096 (n = 2^16, radix 2^3: 20 towers
+// forward with their epilogue 17.1 -> 10.7 us, 170 towers 72.0 -> 64.5, 1290 towers
+// 546 -> 512; 136 towers inverse 40.8 -> 37.9).  Two kinds of pass take 4096-element tiles
+// (NTT_LOG_TILE_BIG) where their launch fills the chip:
+// - column passes: their rows of 2^(12 - S1) words are whole L2 lines at
+//   n = 2^16 (170 towers forward, radix 2^3: 82.0 us with 1024, 36.8 with 4096);
+// - whole transforms' row passes at radix 2^4, whose 16-element units occupy 64
+//   of 256 lanes of the small tile (1032 towers inverse at n = 2^16: 337 us with
+//   1024, 251 with 4096; at radix 2^3 285 with either).
 enum {
     NTT_LOG_TILE = 10,
     NTT_TILE = 1 << NTT_LOG_TILE,
-    NTT_LOG_TILE_COLS = 12,
+    NTT_LOG_TILE_BIG = 12,
     NTT_SINGLE_MAX = 4096,
     NTT_THREADS = 256
 };
+
+// Register radix of the passes that work on 1024-element tiles or smaller:
+// 2^3 at most (a radix 2^4 unit per lane would leave three quarters of the lanes
+// idle; 64 EvalMult+Rescale at n = 2^16, L = 24: 9156 us with 2^4 in every kernel,
+// 7519 with 2^3, 7549 with 2^2)
+GF_HD constexpr uint32_t row_radix(uint32_t rmax) { return rmax < 3 ? rmax : 3; }
 
 // row-tile padding: one spare word every 16, so strided radix units hit distinct LDS banks
 GF_HD constexpr uint32_t padded(uint32_t k) { return k + (k >> 4); }
@@ -689,12 +698,13 @@ GF_HD void row_tile(const NttJob& j, const TileDesc& d, const GF_GLOBAL uint64_t
     }
 }
 
-// Phase B: tile = rows [a0, a0+R), each a contiguous run of N2 = 2^S2.
+// Phase B: tile = rows [a0, a0+R), each a contiguous run of N2 = 2^S2 (2^LOGT elements).
 // IN_LDS (inverse): the tile's input is already in LDS (row_tile).
-template <bool FWD, bool LZ, bool PAIRED, uint32_t S2, uint32_t RM, class Sync, bool IN_LDS = false>
+template <bool FWD, bool LZ, bool PAIRED, uint32_t S2, uint32_t RM, class Sync, bool IN_LDS = false,
+          uint32_t LOGT = NTT_LOG_TILE>
 GF_HD void phaseB_body(const NttJob& j, const NttGeom& g, uint32_t tile, uint64_t* lds,
                        uint32_t tid, uint32_t nthr, Sync sync) {
-    constexpr uint32_t N2 = 1u << S2, logR = NTT_LOG_TILE - S2, R = 1u << logR;
+    constexpr uint32_t N2 = 1u << S2, logR = LOGT - S2, R = 1u << logR;
     const uint32_t N1 = 1u << g.logN1;
     const uint32_t a0 = tile * R;
     const TileDesc d{logR, 1, padded(N2), N1 + a0, 1, false, true};
@@ -726,6 +736,14 @@ inline bool with_radix(uint32_t r, F&& f) {
     if (r == 3) { f(std::integral_constant<uint32_t, 3>{}); return true; }
     if (r == 4) { f(std::integral_constant<uint32_t, 4>{}); return true; }
     return false;
+}
+// the radices of row_radix
+template <class F>
+inline bool with_row_radix(uint32_t r, F&& f) {
+    if (r < 2 || r > 4) return false;
+    if (row_radix(r) == 2) f(std::integral_constant<uint32_t, 2>{});
+    else f(std::integral_constant<uint32_t, 3>{});
+    return true;
 }
 template <class F>
 inline bool with_single(uint32_t logn, F&& f) {

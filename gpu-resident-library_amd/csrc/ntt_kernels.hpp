@@ -51,11 +51,11 @@ __global__ __launch_bounds__(NTT_THREADS) void k_ntt_A(J jobs, NttGeom g) {
                                                                             blockDim.x, DevSync{});
     });
 }
-template <bool FWD, bool PAIRED, uint32_t S2, uint32_t RM, class J>
+template <bool FWD, bool PAIRED, uint32_t S2, uint32_t RM, uint32_t LOGT, class J>
 __global__ __launch_bounds__(NTT_THREADS) void k_ntt_B(J jobs, NttGeom g) {
     extern __shared__ uint64_t lds[];
     const NttJob j = jobs.get(blockIdx.y);
-    if constexpr (!FWD && PAIRED) {
+    if constexpr (!FWD && PAIRED && LOGT == NTT_LOG_TILE) {
         // inverse jobs that carry fp64 tables (moduli below 2^50)
         if (j.twd) {
             phaseB_inv_f64<S2, RM>(j, g, blockIdx.x, lds, threadIdx.x, blockDim.x, DevSync{});
@@ -63,8 +63,8 @@ __global__ __launch_bounds__(NTT_THREADS) void k_ntt_B(J jobs, NttGeom g) {
         }
     }
     with_lz<FWD>(j, [&](auto L) {
-        phaseB_body<FWD, decltype(L)::value, PAIRED, S2, RM>(j, g, blockIdx.x, lds, threadIdx.x, blockDim.x,
-                                                             DevSync{});
+        phaseB_body<FWD, decltype(L)::value, PAIRED, S2, RM, DevSync, false, LOGT>(j, g, blockIdx.x, lds, threadIdx.x,
+                                                                                   blockDim.x, DevSync{});
     });
 }
 template <bool FWD, bool PAIRED, uint32_t S, uint32_t RM, class J>
@@ -85,12 +85,15 @@ enum { NTT_COLS_WGS = 128 };
 
 // PAIRED: library plans use interleaved (w, Shoup precon) tables; the
 // reference ABI launchers take the two arrays separately.  g.rmax selects the
-// register radix (the tuning knob the autotuner sets).
+// register radix (the tuning knob the autotuner sets), row_radix(g.rmax) on
+// 1024-element tiles.  big_rows: row passes on 4096-element tiles, over row
+// tables of g.rmax = 4 (Ctx::big_row_tiles).
 template <bool FWD, bool PAIRED, class J>
-inline void ntt_dispatch_dir(J jobs, uint32_t njobs, const NttGeom& g, hipStream_t s, uint32_t which) {
+inline void ntt_dispatch_dir(J jobs, uint32_t njobs, const NttGeom& g, hipStream_t s, uint32_t which,
+                             bool big_rows = false) {
     const dim3 thr(NTT_THREADS);
     bool ok = with_radix(g.rmax, [&](auto Rc) {
-        constexpr uint32_t RM = decltype(Rc)::value;
+        constexpr uint32_t RM = decltype(Rc)::value, RR = row_radix(RM);
         bool geom_ok;
         if (g.single) {
             geom_ok = with_single(g.logn, [&](auto Sc) {
@@ -101,26 +104,43 @@ inline void ntt_dispatch_dir(J jobs, uint32_t njobs, const NttGeom& g, hipStream
         } else {
             geom_ok = with_split(g.logN1, g.logN2, [&](auto A, auto B) {
                 constexpr uint32_t S1 = decltype(A)::value, S2 = decltype(B)::value;
-                const dim3 gB((1u << S1) / g.R, njobs);
-                const size_t shB = (size_t)padded(NTT_TILE) * 8;
-                // the column pass takes large tiles where they fill the chip
+                using Small = std::integral_constant<uint32_t, NTT_LOG_TILE>;
+                using Big = std::integral_constant<uint32_t, NTT_LOG_TILE_BIG>;
                 auto run_A = [&] {
                     auto go = [&](auto T) {
                         constexpr uint32_t LOGT = decltype(T)::value;
-                        k_ntt_A<FWD, PAIRED, S1, RM, LOGT>
+                        k_ntt_A<FWD, PAIRED, S1, LOGT == NTT_LOG_TILE ? RR : RM, LOGT>
                             <<<dim3(g.n >> LOGT, njobs), thr, (size_t)8 << LOGT, s>>>(jobs, g);
                     };
-                    if ((uint64_t)njobs * (g.n >> NTT_LOG_TILE_COLS) >= NTT_COLS_WGS)
-                        go(std::integral_constant<uint32_t, NTT_LOG_TILE_COLS>{});
-                    else
-                        go(std::integral_constant<uint32_t, NTT_LOG_TILE>{});
+                    // (one tower never has that many)
+                    if constexpr (PAIRED) {
+                        if ((uint64_t)njobs * (g.n >> NTT_LOG_TILE_BIG) >= NTT_COLS_WGS) {
+                            go(Big{});
+                            return;
+                        }
+                    }
+                    go(Small{});
+                };
+                auto run_B = [&] {
+                    auto go = [&](auto T) {
+                        constexpr uint32_t LOGT = decltype(T)::value;
+                        k_ntt_B<FWD, PAIRED, S2, LOGT == NTT_LOG_TILE ? RR : RM, LOGT>
+                            <<<dim3(g.n >> LOGT, njobs), thr, (size_t)padded(1u << LOGT) * 8, s>>>(jobs, g);
+                    };
+                    if constexpr (PAIRED && RM == 4) {
+                        if (big_rows) {
+                            go(Big{});
+                            return;
+                        }
+                    }
+                    go(Small{});
                 };
                 // which: bit 0 = first kernel of the transform, bit 1 = second
                 if (FWD) {
                     if (which & 1) run_A();
-                    if (which & 2) k_ntt_B<FWD, PAIRED, S2, RM><<<gB, thr, shB, s>>>(jobs, g);
+                    if (which & 2) run_B();
                 } else {
-                    if (which & 1) k_ntt_B<FWD, PAIRED, S2, RM><<<gB, thr, shB, s>>>(jobs, g);
+                    if (which & 1) run_B();
                     if (which & 2) run_A();
                 }
             });
