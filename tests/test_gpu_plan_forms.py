@@ -79,3 +79,91 @@ def test_whole_transforms_at_every_radix(G, n, L, counts):
             for i in range(count):
                 for k in range(2):
                     assert np.array_equal(o[i][k].download(), w[i % 3][k]), (radix, count, i, k)
+
+
+@pytest.mark.parametrize("f64", [0, 1])
+@pytest.mark.parametrize("dnum,down", [(1, "both"), (1, "modup"), (3, "both"), (3, "moddown")])
+def test_stages_below_modup_min_wgs_run_apart(G, dnum, down, f64):
+    """Fused ModUp and ModDown stages of fewer workgroups than modup_min_wgs run
+    as transforms and conversions of their own: both stages, or only the one
+    with fewer jobs (one part per operation against two components, or three
+    parts against two).  Products, rotations (apart and over their inputs),
+    hoisted rotations, keyswitches and linear transforms."""
+    n, L, count = 1 << 14, 6, 8
+    t = Setup(G, n, L, dnum, nkeys=2, knobs=dict(modup_f64=f64))
+    P, ctx, s = t.P, t.ctx, t.s
+    ks = [pow(5, 9, 2 * n), 2 * n - 1]
+    c = [[t.ct(L) for _ in range(4)] for _ in range(count)]
+    ws = [ctx.workspace() for _ in range(3 * count)]
+    wp = [w.ptr for w in ws]
+    some = (0, 1, count - 1)
+
+    def fresh():
+        return [[G.Dev.of(x) for x in v] for v in c]
+
+    def col(d, j):
+        return [x[j].ptr for x in d]
+
+    def line(ups, downs):
+        """the knob between the two stages' workgroups (ups parts, downs components)"""
+        if down == "both":
+            ctx.set_knob("modup_min_wgs", 1 << 30)
+        else:
+            lo, hi = (ups, downs) if down == "modup" else (downs, ups)
+            if lo >= hi:
+                return False
+            ctx.set_knob("modup_min_wgs", lo * n // 1024 + 1)
+        return True
+
+    def run(plan, fused_down):
+        kinds = [k for k, _ in plan.steps()]
+        assert ("modup" in kinds) == (down == "moddown"), kinds
+        assert (fused_down in kinds) == (down == "modup"), kinds
+        plan.run(s)
+        s.sync()
+
+    def check(dev, want, what):
+        assert np.array_equal(dev[0].download(want[0].size), want[0]), what
+        assert np.array_equal(dev[1].download(want[1].size), want[1]), what
+
+    assert line(count * dnum, 2 * count)
+    for over in (False, True):
+        d = fresh()
+        o = [x[:2] for x in d] if over else [[G.Dev((L - 1) * n) for _ in range(2)] for _ in range(count)]
+        run(G.plan_evalmult_rescale(ctx, t.keys[0], [L] * count, *[col(d, j) for j in range(4)], col(o, 0), col(o, 1), wp[:count]),
+            "moddown")
+        for i in some:
+            check(o[i], P.evalmult_rescale(L, *c[i], *t.hk[0]), ("mult", over, i))
+        d = fresh()
+        o = [x[:2] for x in d] if over else [[G.Dev(L * n) for _ in range(2)] for _ in range(count)]
+        kk, kh = [ks[i % 2] for i in range(count)], [t.keys[i % 2] for i in range(count)]
+        run(G.plan_rotate(ctx, kh, [L] * count, kk, col(d, 0), col(d, 1), col(o, 0), col(o, 1), wp[:count]), "ksdown")
+        for i in some:
+            check(o[i], P.rotate(L, c[i][0], c[i][1], kk[i], *t.hk[i % 2]), ("rot", over, i))
+        if line(count * dnum, 4 * count):
+            d = fresh()
+            h = [[G.Dev(L * n) for _ in range(2)] for _ in range(2 * count)]
+            if over:   # the first rotation of each over its input
+                for i in range(count):
+                    h[2 * i] = d[i][:2]
+            run(G.plan_rotate_hoisted(ctx, [L] * count, col(d, 0), col(d, 1), t.keys, ks, col(h, 0), col(h, 1), wp[:count], wp[count:]),
+                "ksdown")
+            for i in some:
+                for j, w in enumerate(P.rotate_hoisted(L, c[i][0], c[i][1], ks, t.hk)):
+                    check(h[2 * i + j], w, ("hoist", over, i, j))
+        line(count * dnum, 2 * count)
+    assert line(dnum, 2)
+    d = fresh()
+    o = [G.Dev(L * n) for _ in range(2)]
+    G.check(G.lib.gf_keyswitch(ctx.h, t.keys[0].h, L, d[0][0].ptr, o[0].ptr, o[1].ptr, wp[0], s.s))
+    s.sync()
+    check(o, P.keyswitch(L, c[0][0], *t.hk[0]), "ks")
+    G.check(G.lib.gf_evalmult(ctx.h, t.keys[0].h, L, *[x.ptr for x in d[0]], o[0].ptr, o[1].ptr, wp[0], s.s))
+    s.sync()
+    check(o, P.evalmult(L, *c[0], *t.hk[0]), "evalmult")
+    pts = [t.ct(L) for _ in range(3)]
+    dp = [G.Dev.of(x) for x in pts]
+    G.linear_transform(ctx, L, d[0][0].ptr, d[0][1].ptr, [None] + t.keys, [1] + ks, [x.ptr for x in dp], o[0].ptr, o[1].ptr,
+                       wp[0], wp[1:4], s)
+    s.sync()
+    check(o, P.linear_transform(L, c[0][0], c[0][1], [1] + ks, [None] + t.hk, pts), "linear")
