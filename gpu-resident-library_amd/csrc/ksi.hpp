@@ -197,7 +197,7 @@ GF_HD void ksi_tensor(const KsiJob& j, const uint64_t* x, uint64_t& t0, uint64_t
 enum { KSI_IN_WORDS = 4 * KSI_TILE, KSI_IN_CHUNK = 128 };   // a chunk: one 16-byte access per lane
 GF_HD uint32_t ksi_in_off(const KsiJob& j) { return ((uint32_t)__builtin_popcount(j.xf) + 2) * KSI_PART_WORDS; }
 GF_HD void ksi_request_inputs(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t wave, uint32_t nwaves,
-                              uint32_t lane) {
+                              uint32_t lane, uint32_t wlanes) {
 #if defined(__HIP_DEVICE_COMPILE__)
     for (uint32_t c = __builtin_amdgcn_readfirstlane(wave); c < KSI_IN_WORDS / KSI_IN_CHUNK; c += nwaves) {
         const uint32_t k = c / (KSI_TILE / KSI_IN_CHUNK), o = c % (KSI_TILE / KSI_IN_CHUNK) * KSI_IN_CHUNK;
@@ -207,7 +207,7 @@ GF_HD void ksi_request_inputs(const KsiJob& j, uint64_t* lds, uint32_t off, uint
                                          16, 0, 0);
     }
 #else
-    for (uint32_t i = wave * 64 + lane; i < KSI_IN_WORDS; i += nwaves * 64)
+    for (uint32_t i = wave * wlanes + lane; i < KSI_IN_WORDS; i += nwaves * wlanes)
         lds[ksi_in_off(j) + i] = j.fin.in[i / KSI_TILE][off + i % KSI_TILE];
 #endif
 }
@@ -442,7 +442,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
         ++k;
     };
     const uint32_t np = j.np, rows = FIN ? np + 2 : np;
-    if constexpr (FIN == KSI_FIN_TENSOR_IN) ksi_request_inputs(j, lds, off, wave, nwaves, lane);
+    if constexpr (FIN == KSI_FIN_TENSOR_IN) ksi_request_inputs(j, lds, off, wave, nwaves, lane, wlanes);
     for (uint32_t p = 0; p < rows; ++p) {
         if (p < np) {
             if ((j.xf >> p) & 1) row_pass(j.src[p]);
