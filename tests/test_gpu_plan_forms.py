@@ -167,3 +167,67 @@ def test_stages_below_modup_min_wgs_run_apart(G, dnum, down, f64):
                        wp[0], wp[1:4], s)
     s.sync()
     check(o, P.linear_transform(L, c[0][0], c[0][1], [1] + ks, [None] + t.hk, pts), "linear")
+
+
+# knobs that differ from the defaults; radix 0: the default
+LAST_STEP = [dict(), dict(ntt_radix=2), dict(ntt_radix=4), dict(ksi_fin=0), dict(ksi_tensor=0), dict(ksi_tensor=0, ntt_radix=2),
+             dict(modup_f64=0), dict(modup_f64=0, ntt_radix=2), dict(ksi_f64=0, ksi_extra=1), dict(ksi_rowpass=0),
+             dict(ksi_rowpass=0, ntt_radix=2, ksi_f64=0), dict(tensor_ib=0), dict(ksi_extra=1, ntt_radix=2), dict(ksi_fin=0, ksi_extra=1),
+             dict(moddown_fused=0), dict(modup_fused=0, ntt_radix=2)]
+DEFAULTS = dict(ntt_radix=3, ksi_fin=1, ksi_tensor=1, modup_f64=1, ksi_f64=1, ksi_extra=0, ksi_rowpass=1, tensor_ib=1,
+                moddown_fused=1, modup_fused=1)
+
+
+@pytest.mark.parametrize("n,L,dnum,count", [(1 << 13, 6, 3, 24), (1 << 13, 8, 4, 16), (1 << 14, 6, 6, 8), (1 << 15, 5, 5, 5)])
+def test_last_step_at_every_knob(G, n, L, dnum, count):
+    """Batches above the line from which the Q rows' inner products take the
+    outputs' row passes with them (and form the tensor products there): every
+    knob and radix that changes those launches, levels mixed, products,
+    rotations and hoisted rotations, buffers at 16-byte and at 8-byte addresses."""
+    t = Setup(G, n, L, dnum, nkeys=2)
+    P, ctx, s = t.P, t.ctx, t.s
+    lv = [L - i % 2 for i in range(max(count, 6))]
+    c = [[t.ct(lv[i]) for _ in range(4)] for i in range(6)]   # taken in turn
+    ks = [pow(5, 13, 2 * n), 2 * n - 1]
+    wm = [P.evalmult_rescale(lv[i], *c[i], *t.hk[0]) for i in range(6)]
+    wr = [P.rotate(lv[i], c[i][0], c[i][1], ks[i % 2], *t.hk[i % 2]) for i in range(6)]
+    wh = P.rotate_hoisted(lv[0], c[0][0], c[0][1], ks, t.hk)
+    lv = lv[:count]
+    ws = [ctx.workspace() for _ in range(count)]
+    wp = [w.ptr for w in ws]
+    hc = count // 4   # ciphertexts of the hoisted rotations, two rotations each
+
+    def place(x, odd):
+        d = G.Dev(x.size + 2)
+        d.upload(x, odd)
+        return d
+
+    for odd in (0, 1):
+        d = [[place(x, odd) for x in v] for v in c]
+        at = [[x.at(odd) for x in d[i % 6]] for i in range(count)]
+        o = [[G.Dev(L * n + 2) for _ in range(2)] for _ in range(count)]
+        oat = [[x.at(odd) for x in v] for v in o]
+        for knobs in LAST_STEP if not odd else LAST_STEP[:2] + [dict(modup_f64=0)]:
+            for k, v in {**DEFAULTS, **knobs}.items():
+                ctx.set_knob(k, v)
+            fused = knobs.get("moddown_fused", 1)
+
+            def run(plan, last, want, what):
+                kinds = [k for k, _ in plan.steps()]
+                assert not fused or kinds[-1] == ("ksi" if last else "ntt_fwd_b"), (knobs, odd, kinds)
+                plan.run(s)
+                s.sync()
+                for i, w in enumerate(want):
+                    for j in range(2):
+                        assert np.array_equal(o[i][j].download(w[j].size, odd), w[j]), (what, knobs, odd, i, j)
+
+            fin = knobs.get("ksi_fin", 1)
+            run(G.plan_evalmult_rescale(ctx, t.keys[0], lv, *[[x[j] for x in at] for j in range(4)],
+                                        [x[0] for x in oat], [x[1] for x in oat], wp),
+                fin and knobs.get("ksi_rowpass", 1), [wm[i % 6] for i in range(count)], "mult")
+            run(G.plan_rotate(ctx, [t.keys[i % 2] for i in range(count)], lv, [ks[i % 2] for i in range(count)],
+                              [x[0] for x in at], [x[1] for x in at], [x[0] for x in oat], [x[1] for x in oat], wp),
+                fin, [wr[i % 6] for i in range(count)], "rot")
+            run(G.plan_rotate_hoisted(ctx, [L] * hc, [at[0][0]] * hc, [at[0][1]] * hc, t.keys, ks,
+                                      [x[0] for x in oat[:2 * hc]], [x[1] for x in oat[:2 * hc]], wp[:hc], wp[hc:3 * hc]),
+                fin and 2 * hc * L * (n // 512) >= 1024, [wh[i % 2] for i in range(2 * hc)], "hoist")
