@@ -70,29 +70,38 @@ def kernel_bytes(name, kind, nkern, total, epilogue):
     return [tr // 2, tr - tr // 2 + epilogue]
 
 
-def step_bytes(n, L, K, alpha, np_parts, kinds, batch):
+def step_bytes(n, L, K, alpha, np_parts, kinds, batch, ksi_tensor=True):
     """Algorithmic HBM bytes per operation of each plan step, in plan order:
     each transform reads and writes its tower once (16 n B), pointwise steps
     move their operands once, conversions read sources once and write
     targets once, the key inner product reads every digit once and every key
     row once per launch: the batch's ops share one key, so a key row counts
-    1 / batch per op (B_key = batch).  Entries are (stage, bytes, bytes read
-    by a fused transform epilogue)."""
+    1 / batch per op (B_key = batch).  ksi_tensor: the knob of that name (the
+    last step forms the tensor products where the tensor step has the row pass
+    fused).  Entries are (stage, bytes, bytes read by a fused transform
+    epilogue)."""
     T = 8 * n
     key = 2 * np_parts / batch   # key rows read per tower row, per op
     # the Q rows' inner products in the launch that runs the outputs' row
-    # passes: the digits, keys, ModDown column passes and tensor towers in, the
-    # outputs out, no accumulators; the P rows (and the dropped tower's, with
-    # t's two towers in) store their inverse transforms' row passes
+    # passes: the transformed digits, keys, ModDown column passes, the own digit
+    # and two tensor towers in, the outputs out, no accumulators; the P rows (and
+    # the dropped tower's, with t's two towers in) store their inverse transforms'
+    # row passes.  Where that launch forms the tensor products itself, it reads
+    # the four input towers in their place, and the tensor step reads two and
+    # writes the row pass of t2 (the dropped tower's: four in, four out)
     if kinds[-1] == "ksi":
         up, dn = kinds.index("modup"), kinds.index("moddown")
         assert list(kinds[up + 1:]) == ["ksi", "moddown", "ksi"], kinds
         full = {name: (b, e) for name, b, e in
                 step_bytes(n, L, K, alpha, np_parts, list(kinds[:up + 1]) + ["ksi", "ksi", "moddown", "ntt_fwd_b"], batch)}
         head = [(k, *v) for k, v in full.items() if k in ("tensor", "intt_modup_rowpass", "tensor_intt_rowpass", "modup_fused")]
+        own = 1 + 2
+        if ksi_tensor and head[0][0] == "tensor_intt_rowpass":
+            own = 4
+            head[0] = (head[0][0], T * (3 * (L - 1) + 8), 0)
         return head + [("rowpass_inner_p_drop", T * K * (np_parts + key + 2) + T * (np_parts + key + 2 + 2), 0),
                        ("moddown_fused", *full["moddown_fused"]),
-                       ("rowpass_inner_q_final", T * (L - 1) * (np_parts + key + 2 + 2 + 2), 0)]
+                       ("rowpass_inner_q_final", T * (L - 1) * ((np_parts - 1) + key + own + 2 + 2), 0)]
     # the dropped tower's inverse transform inside the other steps: one per
     # component, of t + res / P, its row pass in the Q rows' inner product (t's
     # two towers in, two out; the accumulators' stay on chip) and its column
@@ -765,7 +774,7 @@ def main():
 
     stages = time_steps(G, res["plan"], stream)
     np_parts = -(-L // alpha)
-    sb = step_bytes(N, L, K, alpha, np_parts, [s[0] for s in stages], B)
+    sb = step_bytes(N, L, K, alpha, np_parts, [s[0] for s in stages], B, bool(ctx.knob("ksi_tensor")))
     stage_report, kernels = [], []
     for (kind, jobs, ms, kms), (name, bytes_per_op, epi) in zip(stages, sb):
         gbs = bytes_per_op * B / (ms / 1e3) / 1e9
