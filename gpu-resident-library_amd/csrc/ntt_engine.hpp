@@ -65,7 +65,10 @@ struct NttJob {
     const uint64_t* in;   // tower read by the first phase
     uint64_t* out;        // tower written by every phase (may equal in)
     const uint64_t* tw;   // twiddles: paired table (w, Shoup precon) or w alone
-    const uint64_t* twp;  // Shoup precons when tw is not paired, else unused
+    union {
+        const uint64_t* twp;  // Shoup precons when tw is not paired
+        const uint64_t* mid;  // paired, forward row pass alone: the column-pass output it reads (null: out)
+    };
     uint64_t q;
     uint64_t post, postp; // inverse only: final multiplier (n^-1 * c) and precon
     // forward only, optional epilogue: out = NTT(in) + e0*c0 + e1*c1 (mod q)
@@ -82,22 +85,24 @@ struct NttJob {
     uint64_t red;
     // with red: store those unreduced values, for a consumer that reduces them
     // itself (the key inner product); ignored with an epilogue
-    uint32_t lazy_out;
+    uint32_t lazy_out : 1;
+    // forward epilogue: 1: e1 is added as it is (residues in [0, q), or null
+    // for none; c1 unused), out = NTT(in) + e0*c0 + e1
+    uint32_t e1_plain : 1;
+    // inverse row pass, and e1_plain operands: the tower is read through the
+    // evaluation-domain automorphism of index gk (0: as it is), n = 2^glog
+    uint32_t glog : 8;
+    uint32_t gk;
     // inverse phase B of a modulus below 2^50 with inputs below 4q: its fp64
     // pairs and their row table (ntt_f64.hpp; null: the integer passes), q
     // and fl(1/q).  Its output is then in [0, 2q).
     const uint64_t* twd;
     const uint64_t* twrd;
     double fq, fqinv;
-    // forward epilogue: 1: e1 is added as it is (residues in [0, q), or null
-    // for none; c1 unused), out = NTT(in) + e0*c0 + e1
-    uint32_t e1_plain;
-    // inverse row pass, and e1_plain operands: the tower is read through the
-    // evaluation-domain automorphism of index gk (0: as it is), n = 2^glog
-    uint32_t gk, glog;
-    // forward row pass alone: the column-pass output it reads (null: out)
-    const uint64_t* mid;
 };
+// a plan's transforms are most of its job arrays, and those of the allocation-free
+// EvalMult+Rescale have a fixed area (256 towers in 16 digits take 4862)
+static_assert(sizeof(NttJob) == 160, "job arrays sized by it");
 
 // Evaluation-domain automorphism sigma_k of a tower in bit-reversed order:
 // sigma_k(x)[i] = x[galois_index(i, k, log n)], k odd.  e = (2 brv(i) + 1) k mod
@@ -711,7 +716,7 @@ GF_HD void phaseB_body(const NttJob& j, const NttGeom& g, uint32_t tile, uint64_
     // forward: phase B is the second phase (reads out); inverse: the first.
     // Inverse phase B hands lazy values in [0,4q) to phase A.
     row_tile<FWD, LZ, PAIRED, S2, RM, R, FWD ? 2 : 0, PAIRED, Sync, false, IN_LDS>(
-        j, d, gcast(!FWD ? j.in : j.mid ? j.mid : j.out), gcast(j.out), a0 << S2, lds, tid, nthr, sync);
+        j, d, gcast(!FWD ? j.in : PAIRED && j.mid ? j.mid : j.out), gcast(j.out), a0 << S2, lds, tid, nthr, sync);
 }
 
 // Single phase: the whole tower (n = 2^S <= NTT_SINGLE_MAX) is one tile.

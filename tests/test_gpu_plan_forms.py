@@ -231,3 +231,19 @@ def test_last_step_at_every_knob(G, n, L, dnum, count):
             run(G.plan_rotate_hoisted(ctx, [L] * hc, [at[0][0]] * hc, [at[0][1]] * hc, t.keys, ks,
                                       [x[0] for x in oat[:2 * hc]], [x[1] for x in oat[:2 * hc]], wp[:hc], wp[hc:3 * hc]),
                 fin and 2 * hc * L * (n // 512) >= 1024, [wh[i % 2] for i in range(2 * hc)], "hoist")
+
+
+def test_largest_plan_in_the_static_job_area(G):
+    """The allocation-free EvalMult+Rescale at the most towers and digits that a
+    context takes (256 towers, 16 digits of 16, 14 special primes): its plan of
+    nearly 5000 transforms still fits the static job area."""
+    n, L, dnum = 1 << 10, 256, 16
+    t = Setup(G, n, L, dnum)
+    assert t.P.K == 14
+    c = [t.ct(L) for _ in range(4)]
+    d = [G.Dev.of(x) for x in c]
+    o = [G.Dev((L - 1) * n) for _ in range(2)]
+    G.check(G.lib.gf_evalmult_rescale_noalloc(t.ctx.h, t.keys[0].h, L, *[x.ptr for x in d], o[0].ptr, o[1].ptr, t.s.s))
+    t.s.sync()
+    for x, w in zip(o, t.P.evalmult_rescale(L, *c, *t.hk[0])):
+        assert np.array_equal(x.download(), w)
