@@ -187,16 +187,14 @@ def ptrs(arrays):
     return (u64p * len(arrays))(*[O.P(a) for a in arrays])
 
 
-@pytest.mark.parametrize("sp,wide", [(1, 1), (6, 1), (7, 1), (7, 7), (8, 2), (9, 9), (11, 3), (12, 12), (12, 1)])
-@pytest.mark.parametrize("logn", [13, 16])
+@pytest.mark.parametrize("logn,sp,wide", [(13, 1, 1), (13, 6, 1), (13, 7, 1), (13, 7, 7), (13, 8, 2), (13, 9, 9), (13, 11, 3),
+                                          (13, 12, 12), (13, 12, 1), (16, 7, 1), (16, 12, 12)])
 def test_modup_of_many_sources(emu, logn, sp, wide):
     """The fused ModUp over 1, 6 and 7 to 12 sources, `wide` of them of 60 bits
     (the largest sums), to targets of 60 and 50 bits in ranges of one and of
     all: sum_i INTT(x_i) f_i tab_i R^-1 mod t, transformed, with integer and
     with fp64 passes and, where it applies, the R = 2^60 reduction."""
     n = 1 << logn
-    if logn == 16 and (sp, wide) not in ((7, 1), (12, 12)):
-        pytest.skip("the larger ring at two counts")
     mods = moduli(n, wide + 1, sp - wide + 2)
     sm, tm = mods[:wide] + mods[wide + 1:wide + 1 + sp - wide], [mods[wide]] + mods[-2:]
     rng = np.random.default_rng(logn * 100 + sp + wide)
@@ -225,16 +223,13 @@ def test_modup_of_many_sources(emu, logn, sp, wide):
                     assert np.array_equal(dst[j * n:(j + 1) * n], want[j]), (f64, c60, ln, j)
 
 
-@pytest.mark.parametrize("K", [0, 1, 6, 7, 8, 11, 12])
-@pytest.mark.parametrize("logn", [13, 16])
+@pytest.mark.parametrize("logn,K", [(13, 0), (13, 1), (13, 6), (13, 7), (13, 8), (13, 11), (13, 12), (16, 0), (16, 12)])
 def test_moddown_with_the_dropped_tower_as_a_source(emu, logn, K):
     """The fused ModDown's rescale mode over K special primes of 60 bits, the
     dropped tower one more source, larger and smaller than the targets (K = 0:
     a plain rescale): with dv = INTT(x_d) - pinv sum_k INTT(x_k) f_k tabd_k R^-1,
     centred, the targets' sum_k INTT(x_k) f_k tab_k R^-1 + s2 dv, transformed."""
     n = 1 << logn
-    if logn == 16 and K not in (0, 12):
-        pytest.skip("the larger ring at two counts")
     mods = moduli(n, K + 2, 4)
     pm, rest = mods[:K], mods[K:]
     for old in (rest[0], rest[2]):   # of 60 bits; of 50 bits, between the targets
