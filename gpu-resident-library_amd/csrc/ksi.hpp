@@ -395,8 +395,12 @@ GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint3
         case 3: ksi_inner_cols<3, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
         case 4: ksi_inner_cols<4, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
         // 5 and 6 parts take one position per access (two need more registers
-        // than 5 waves per SIMD leave), in kernels of their own (NPMAX = 6):
-        // beside the others their operands' scalar loads spill 180 SGPRs more
+        // than 5 waves per SIMD leave).  Beside the other counts their operands'
+        // scalar loads spill SGPRs (42 to 49 in the plain form, 213 to 255 with the
+        // last step, 49 to 68 with the tensor products), so only launches that have
+        // such jobs take a kernel with all six (NPMAX = 6; 59 EvalMult+Rescale of
+        // 19 towers in 5 parts at n = 2^14: 1580 us by 128-bit sums, 1503 by these);
+        // the other launches' kernels spill none, 33 to 41, and up to 6.
         case 5:
             if constexpr (NPMAX >= 5) {
                 ksi_inner_cols<5, 1, LZ, FIN>(j, lds, off, tid, nthr, t);

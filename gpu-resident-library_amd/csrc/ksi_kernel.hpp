@@ -17,7 +17,10 @@ struct WaveSync {
 // (row passes for twiddles, inner products for digits and keys), so the waves
 // in flight set the time.  Four parts with their last step take 5 waves of
 // 107 VGPRs uncapped: 64 EvalMult+Rescale at n = 2^16, L = 24 ran 8300 us with 4
-// waves per SIMD, 7570 with 5, 8280 with 6 (spills).
+// waves per SIMD, 7570 with 5, 8280 with 6 (spills).  The last step's kernels
+// (NPMAX = 4) spill scalar registers into vector lanes, 33 to 41 in KSI_FIN, none
+// to 6 with the tensor products, and there 1 to 5 VGPRs to scratch; the stored
+// form spills nothing.
 // FIN: KSI_PLAIN, KSI_FIN, KSI_FIN_TENSOR(_IN); NPMAX: the largest part count with
 // column sums (4, or 6 in kernels_ksi_w.hip).
 template <uint32_t S2, uint32_t RM, int FIN, int NPMAX>

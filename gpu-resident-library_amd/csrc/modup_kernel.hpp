@@ -88,9 +88,10 @@ __device__ __forceinline__ void modup_run(const ModupJob& j, const NttGeom& g, u
 // ciphertexts at levels 8..20, n = 2^16: five launches of 63, 68, 81, 89 and
 // 744 us became one of 898).  SPMAX keeps the registers of small
 // contexts down (8 per source); jobs of 7 to 12 sources (SPMAX = 12) have 168
-// registers and 3 waves per SIMD, in launches of their own: 8 EvalMult+Rescale at
-// n = 2^16, L = 24, dnum = 2 run 963 us with them, 1367 unfused; one of 17 towers
-// at n = 2^14, dnum = 2 103 us, 171 unfused.
+// registers and 3 waves per SIMD, in launches of their own, and at 12 sources
+// still spill some (ModUp 14 to 54 registers by ring split, 54 at n = 2^16; ModDown
+// 2 to 19): 8 EvalMult+Rescale at n = 2^16, L = 24, dnum = 2 run 963 us with them,
+// 1367 unfused; one of 17 towers at n = 2^14, dnum = 2 103 us, 171 unfused.
 template <uint32_t S1, uint32_t SPMAX, bool RS, bool C60>
 __global__ __launch_bounds__(MODUP_THREADS) __attribute__((amdgpu_waves_per_eu(SPMAX > 6 ? 3 : 4, 8))) void k_modup(const ModupJob* __restrict__ jobs, uint32_t off, NttGeom g) {
     __shared__ uint64_t lds[2 * MODUP_TILE];   // phases alternate between the two tiles

@@ -70,7 +70,7 @@ private:
 // The draws of std::mt19937_64 (MT19937-64, Nishimura and Matsumoto), a block
 // of 312 at a time: both loops of the recurrence and the tempering are free of
 // dependences within a vector, so the compiler runs them several words at
-// once (2.4 -> 0.9 ns a draw).
+// once (1.07 -> 0.69 ns a draw on the measuring machine's host).
 class Mt64Block {
 public:
     enum { N = 312, M = 156 };
@@ -106,8 +106,8 @@ private:
 //
 // The draws come from blocks and the next draw's place depends on the last
 // one only through whether it took a sign: no branch on a drawn value but the
-// rare steps of index(), so nothing is mispredicted (2^15
-// coefficients: 1350 -> 445 us on one host core).
+// rare steps of index(), so nothing is mispredicted (2^15 coefficients: 639 ->
+// 215 us on one core of the measuring machine's host).
 template <class V>
 inline void sample_switch_key(size_t cnt, double sigma, uint64_t seed, V* u, V* e0, V* e1) {
     Mt64Block g(seed);
