@@ -361,6 +361,23 @@ enum { NTT_ROWS_WGS = 768 };
 bool Ctx::big_row_tiles(size_t towers) const {
     return geom.rmax == 4 && !geom.single && towers * (n >> NTT_LOG_TILE_BIG) >= NTT_ROWS_WGS;
 }
+// Workgroups from which a stored inner product over integer rows takes them.
+// 1024-element tiles at radix 2^4 / 512-element ones at 2^3, rows below 2^57:
+// n = 2^15, 2 parts 3072 workgroups 29.8 / 32.1 us, 3 parts 4608 55.0 / 57.2, 6 parts 6144
+// 192 / 214; n = 2^16, 3 parts 2304 32.0 / 33.5, 4 parts 2048 40.7 / 38.5, 6 parts 3072
+// 102 / 114.  Rows of 128 words (n <= 2^14) and rows above 2^57, whose butterflies
+// hold more registers, are faster on the small ones at every size (n = 2^14, 3
+// parts, 9216: 131 / 118; the special primes' rows at n = 2^16, 2 parts, 3072: 42.1 / 37.6).
+enum { KSI_BIG_WGS = 3072 };
+bool Ctx::big_ksi_tiles(const KsiJob* j, size_t jobs) const {
+    if (geom.rmax != 4 || geom.single || geom.logN2 != 8 || jobs * (n >> KSI_LOG_TILE_BIG) < KSI_BIG_WGS) return false;
+    size_t lazy = 0;
+    for (size_t i = 0; i < jobs; ++i) {
+        if (j[i].fin.v[0] || j[i].rp_on || j[i].twd || !j[i].xf) return false;
+        lazy += j[i].red != 0;
+    }
+    return 2 * lazy >= jobs;
+}
 const uint64_t* Ctx::f64_table_of(const uint64_t* paired) const {
     const auto it = f64_of_.find(paired);
     return it == f64_of_.end() ? nullptr : it->second;
@@ -959,7 +976,7 @@ void Plan::run_jobs(size_t i, hipStream_t s, uint32_t which, uint32_t first, uin
         case Step::PTACC: launch_ptacc(GF_J(PtAccJob), cnt, n, s); break;
         case Step::NTT_FA: launch_ntt(GF_J(NttJob), cnt, geom, true, s, 1); break;
         case Step::KSI:
-            launch_ksi(GF_J(KsiJob), cnt, geom, st.arg & 0xFF, st.arg >> 8 & 0xFF, st.arg >> 16 & 3, st.arg >> 18, s);
+            launch_ksi(GF_J(KsiJob), cnt, geom, st.arg & 0xFF, st.arg >> 8 & 0xFF, st.arg >> 16 & 3, st.arg >> 18 & 1, st.arg >> 19 & 1, s);
             break;
         case Step::NTT_IB: launch_ntt(GF_J(NttJob), cnt, geom, false, s, 1); break;
         case Step::MODUP: launch_modup(GF_J(ModupJob), cnt, geom, st.arg, s); break;
@@ -2171,12 +2188,15 @@ std::unique_ptr<Plan> PlanBuilder::layout(std::vector<char>& blob) {
         }
         // launched the fewest regions first
         for (size_t k = steps.size(); k-- > 0;) {
-            const KsiJob* first = v.data() + steps[k].first;
+            KsiJob* first = v.data() + steps[k].first;
+            const bool big = C_.big_ksi_tiles(first, steps[k].second - steps[k].first);
+            if (big)
+                for (size_t i = steps[k].first; i < steps[k].second; ++i) v[i].twr = C_.big_row_table_of(v[i].tw);
             const uint32_t x = ksi_regions(*first), waves = std::max(1u, std::min<uint32_t>(x + C_.ksi_extra, KSI_WAVES));
             stage(Step::KSI, first, steps[k].second - steps[k].first, sizeof(KsiJob));
             uint32_t wide = 0;
             for (size_t i = steps[k].first; i < steps[k].second; ++i) wide |= v[i].np == 5 || v[i].np == 6;
-            P->steps.back().arg = x | waves << 8 | ksi_form(*first) << 16 | wide << 18;
+            P->steps.back().arg = x | waves << 8 | ksi_form(*first) << 16 | wide << 18 | (uint32_t)big << 19;
         }
     };
     stage_ksi(ksi_);

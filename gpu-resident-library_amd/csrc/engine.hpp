@@ -131,6 +131,9 @@ public:
     // 70.5 us on 4096, 67.2 on 1024).
     bool big_row_tiles(size_t towers) const;
     const uint64_t* big_row_table_of(const uint64_t* paired) const;
+    // whether a launch of these inner products takes 1024-element tiles, with radix
+    // 2^4 in its integer row passes (over big_row_table_of their tables)
+    bool big_ksi_tiles(const KsiJob* jobs, size_t count) const;
     // the fp64 pairs of the same twiddles as a paired table (fw2 -> fw2d,
     // iv2 -> iv2d), null for moduli of 2^50 and above
     const uint64_t* f64_table_of(const uint64_t* paired) const;
@@ -243,7 +246,7 @@ struct Step {
     uint32_t count;
     // KSI: the jobs' largest LDS region count (bits 0-7), waves per workgroup
     // (bits 8-15), the jobs' form (bits 16-17: KSI_PLAIN, ..), 1 << 18
-    // where some have 5 or 6 parts.  NTT_I: 1: row passes on big tiles
+    // where some have 5 or 6 parts, 1 << 19 on 1024-element tiles.  NTT_I: 1: row passes on big tiles
     // (Ctx::big_row_tiles)
     uint32_t arg = 0;
 };

@@ -233,9 +233,10 @@ void launch_center(uint64_t* x, uint64_t q, uint32_t n, hipStream_t s);
 void launch_ptacc(const PtAccJob* d, uint32_t nj, uint32_t n, hipStream_t s);
 // fused digit row pass + key inner product: regions = LDS regions (at least every
 // job's ksi_regions), waves = workgroup size in waves (1..KSI_WAVES), fin: the
-// jobs' one form (KSI_PLAIN, ..), wide: some have 5 or 6 parts
+// jobs' one form (KSI_PLAIN, ..), wide: some have 5 or 6 parts, big: 1024-element tiles
+// over row tables of radix 2^4 (Ctx::big_ksi_tiles)
 void launch_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, uint32_t fin, bool wide,
-                hipStream_t s);
+                bool big, hipStream_t s);
 void launch_tensor_ib(const TensorIbJob* d, uint32_t nj, const NttGeom& g, hipStream_t s);
 // the fused ModUp over jobs of at most arg & 0xff sources each and of one c60
 // (arg >> 8)

@@ -28,15 +28,20 @@ namespace gf {
 // workgroups a CU holds and how evenly they interleave (64 EvalMult+Rescale at
 // n = 2^16, L = 24: 7690 -> 7590 us; a 10-deep chain of 16 at n = 2^15: 3418 ->
 // 3231; one rotation at n = 2^15: 115 -> 98).  256 positions leave half the
-// lanes of a pass idle (8490 us).
+// lanes of a pass idle (8490 us).  Large launches over integer rows of 256 words
+// take 1024 where the tuner chose radix 2^4: a unit of 16 per lane, and two passes
+// instead of three (Ctx::big_ksi_tiles).
 enum {
     KSI_MAXP = 7,                                    // parts per job (KSI_MAXP regions fit 64 KiB of LDS)
     KSI_LOG_TILE = 9,
     KSI_TILE = 1 << KSI_LOG_TILE,                    // positions per workgroup
     KSI_PART_WORDS = KSI_TILE + KSI_TILE / 16,       // one part's padded LDS region
+    KSI_LOG_TILE_BIG = 10,                           // (Ctx::big_ksi_tiles)
     KSI_WAVES = 7,                                   // largest workgroup, in waves
     KSI_THREADS = 64 * KSI_WAVES
 };
+
+GF_HD constexpr uint32_t ksi_part_words(uint32_t logt) { return (1u << logt) + (1u << logt) / 16; }
 
 // The last step of an output row of both components c, in the launch that
 // forms its inner products r_c: v[c] is the column-pass output of the ModDown's
@@ -235,17 +240,17 @@ GF_HD void ksi_load_eps(const KsiJob& j, uint32_t gi, KsiEps<V>& x) {
         }
     }
 }
-template <int FIN, bool LZ, uint32_t V>
+template <int FIN, bool LZ, uint32_t V, uint32_t PART>
 GF_HD void ksi_store(const KsiJob& j, uint64_t* lds, uint32_t idx, uint32_t gi, const uint64_t* r0,
                      const uint64_t* r1, const KsiEps<V>& x, const NttJob& t) {
     if constexpr (FIN) {
-        const uint32_t k0 = (uint32_t)__builtin_popcount(j.xf) * KSI_PART_WORDS;
+        const uint32_t k0 = (uint32_t)__builtin_popcount(j.xf) * PART;
         auto comp = [&](uint32_t c, const uint64_t* r, const uint64_t* e) {
             uint64_t y[V];
             const int ep = FIN >= KSI_FIN_TENSOR || !j.fin.e_plain ? 0 : j.fin.e[c] ? 1 : 2;
 #pragma unroll
             for (uint32_t v = 0; v < V; ++v) {
-                const uint64_t z = lds[k0 + c * KSI_PART_WORDS + padded(idx + v)];
+                const uint64_t z = lds[k0 + c * PART + padded(idx + v)];
                 y[v] = ep == 0   ? ntt_ep_value<LZ, 0>(z, t, r[v], e[v])
                        : ep == 1 ? ntt_ep_value<LZ, 1>(z, t, r[v], e[v])
                                  : ntt_ep_value<LZ, 2>(z, t, r[v], 0);
@@ -270,7 +275,7 @@ GF_HD void ksi_store(const KsiJob& j, uint64_t* lds, uint32_t idx, uint32_t gi, 
                 b = addmod(t1[v], shoup(b, j.dpinv, j.dpinvp, j.q), j.q);
             }
             lds[padded(idx + v)] = a;
-            lds[KSI_PART_WORDS + padded(idx + v)] = b;
+            lds[PART + padded(idx + v)] = b;
         }
         return;
     }
@@ -296,7 +301,7 @@ GF_HD U128 cols_to_u128(uint64_t lo, uint64_t mid, uint64_t hi) {
 // sums are 30-bit column sums (j.d30): per part and component four 32 x 32
 // multiply-adds with no carries.  NP <= 7 keeps every column below 2^64
 // (lo, hi < 7 2^60; mid < 14 2^60).
-template <uint32_t NP, uint32_t V, bool LZ, int FIN>
+template <uint32_t NP, uint32_t V, bool LZ, int FIN, uint32_t LOGT>
 GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t tid, uint32_t nthr,
                           const NttJob& t) {
     const GF_GLOBAL uint64_t *src[NP], *kb[NP], *ka[NP];
@@ -308,10 +313,10 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
         kb[p] = gcast(j.kb[p]);
         ka[p] = gcast(j.ka[p]);
         xf[p] = (j.xf >> p) & 1;
-        reg[p] = (uint32_t)__builtin_popcount(j.xf & ((1u << p) - 1)) * KSI_PART_WORDS;
+        reg[p] = (uint32_t)__builtin_popcount(j.xf & ((1u << p) - 1)) * ksi_part_words(LOGT);
     }
     const uint64_t q = j.q, qneg = j.qneg;
-    for (uint32_t idx = tid * V; idx < KSI_TILE; idx += nthr * V) {
+    for (uint32_t idx = tid * V; idx < 1u << LOGT; idx += nthr * V) {
         const uint32_t gi = off + idx;
         uint64_t dv[NP][V], bv[NP][V], av[NP][V];
 #pragma unroll
@@ -381,19 +386,19 @@ GF_HD void ksi_inner_cols(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t
                 r1[v] = redc(s1, q, qneg);
             }
         }
-        ksi_store<FIN, LZ, V>(j, lds, idx, gi, r0, r1, ep, t);
+        ksi_store<FIN, LZ, V, ksi_part_words(LOGT)>(j, lds, idx, gi, r0, r1, ep, t);
     }
 }
 
 // ksi_inner_cols for the job's part count, when it has an instantiation
-template <uint32_t V, bool LZ, int FIN, int NPMAX>
+template <uint32_t V, bool LZ, int FIN, int NPMAX, uint32_t LOGT>
 GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint32_t tid, uint32_t nthr,
                              const NttJob& t) {
     switch (j.np) {
-        case 1: ksi_inner_cols<1, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
-        case 2: ksi_inner_cols<2, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
-        case 3: ksi_inner_cols<3, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
-        case 4: ksi_inner_cols<4, V, LZ, FIN>(j, lds, off, tid, nthr, t); return true;
+        case 1: ksi_inner_cols<1, V, LZ, FIN, LOGT>(j, lds, off, tid, nthr, t); return true;
+        case 2: ksi_inner_cols<2, V, LZ, FIN, LOGT>(j, lds, off, tid, nthr, t); return true;
+        case 3: ksi_inner_cols<3, V, LZ, FIN, LOGT>(j, lds, off, tid, nthr, t); return true;
+        case 4: ksi_inner_cols<4, V, LZ, FIN, LOGT>(j, lds, off, tid, nthr, t); return true;
         // 5 and 6 parts take one position per access (two need more registers
         // than 5 waves per SIMD leave).  Beside the other counts their operands'
         // scalar loads spill SGPRs (42 to 49 in the plain form, 213 to 255 with the
@@ -403,13 +408,13 @@ GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint3
         // the other launches' kernels spill none, 33 to 41, and up to 6.
         case 5:
             if constexpr (NPMAX >= 5) {
-                ksi_inner_cols<5, 1, LZ, FIN>(j, lds, off, tid, nthr, t);
+                ksi_inner_cols<5, 1, LZ, FIN, LOGT>(j, lds, off, tid, nthr, t);
                 return true;
             }
             return false;
         case 6:
             if constexpr (NPMAX >= 6) {
-                ksi_inner_cols<6, 1, LZ, FIN>(j, lds, off, tid, nthr, t);
+                ksi_inner_cols<6, 1, LZ, FIN, LOGT>(j, lds, off, tid, nthr, t);
                 return true;
             }
             return false;
@@ -420,10 +425,11 @@ GF_HD bool ksi_inner_cols_np(const KsiJob& j, uint64_t* lds, uint32_t off, uint3
 // LZ = (j.red != 0), FIN = KSI_FIN where j.fin.v[0] is set, KSI_FIN_TENSOR
 // where j.fin.in[0] is too, else KSI_PLAIN.  The wave-level sync wsync separates the row passes of
 // one wave's region; bsync is the workgroup barrier before the inner product.
-template <uint32_t S2, uint32_t RM, bool LZ, class WSync, class BSync, int FIN = KSI_PLAIN, int NPMAX = 4>
+template <uint32_t S2, uint32_t RM, bool LZ, class WSync, class BSync, int FIN = KSI_PLAIN, int NPMAX = 4,
+          uint32_t LOGT = KSI_LOG_TILE>
 GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, uint32_t wave, uint32_t nwaves,
                     uint32_t lane, uint32_t wlanes, uint32_t tid, uint32_t nthr, WSync wsync, BSync bsync) {
-    constexpr uint32_t ROWS = KSI_TILE >> S2, LOGR = KSI_LOG_TILE - S2;
+    constexpr uint32_t ROWS = (1u << LOGT) >> S2, LOGR = LOGT - S2, PART = ksi_part_words(LOGT);
     const uint32_t a0 = tile * ROWS, off = a0 << S2;
     NttJob t{};
     t.tw = j.tw;
@@ -438,10 +444,10 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
         if (k % nwaves == wave) {
             if (j.twd)
                 row_tile_f64<true, S2, RM, ROWS, true>(j.twd, j.twrd, j.fq, j.fqinv, d, gcast(src), nullptr, off,
-                                                       lds + k * KSI_PART_WORDS, lane, wlanes, wsync);
+                                                       lds + k * PART, lane, wlanes, wsync);
             else
                 row_tile<true, LZ, true, S2, RM, ROWS, 2, true, WSync, true>(
-                    t, d, gcast(src), nullptr, off, lds + k * KSI_PART_WORDS, lane, wlanes, wsync);
+                    t, d, gcast(src), nullptr, off, lds + k * PART, lane, wlanes, wsync);
         }
         ++k;
     };
@@ -466,13 +472,13 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
     // up to 6 parts with every value below 2^60: column sums, loads first
     bool done = false;
     if (j.d30)
-        done = FIN >= KSI_FIN_TENSOR || j.pairs ? ksi_inner_cols_np<2, LZ, FIN, NPMAX>(j, lds, off, tid, nthr, t)
-                                                : ksi_inner_cols_np<1, LZ, FIN, NPMAX>(j, lds, off, tid, nthr, t);
+        done = FIN >= KSI_FIN_TENSOR || j.pairs ? ksi_inner_cols_np<2, LZ, FIN, NPMAX, LOGT>(j, lds, off, tid, nthr, t)
+                                                : ksi_inner_cols_np<1, LZ, FIN, NPMAX, LOGT>(j, lds, off, tid, nthr, t);
     // positions idx .. idx + V - 1 per step (V = 2: one 16-byte access per operand)
     auto inner = [&](auto Vc) {
         constexpr uint32_t V = decltype(Vc)::value;
         const uint64_t q = j.q, qneg = j.qneg;
-        for (uint32_t idx = tid * V; idx < KSI_TILE; idx += nthr * V) {
+        for (uint32_t idx = tid * V; idx < 1u << LOGT; idx += nthr * V) {
             const uint32_t gi = off + idx;
             U128 s0[V], s1[V];
             for (uint32_t v = 0; v < V; ++v) s0[v] = s1[v] = U128{0, 0};
@@ -481,7 +487,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
                 if ((j.xf >> p) & 1) {
                     const uint32_t k = __builtin_popcount(j.xf & ((1u << p) - 1));
                     for (uint32_t v = 0; v < V; ++v) {
-                        dv[v] = lds[k * KSI_PART_WORDS + padded(idx + v)];
+                        dv[v] = lds[k * PART + padded(idx + v)];
                         // LZ: below 72q (the sums stay below 2^125); else [0, 8q) -> [0, q)
                         if constexpr (!LZ) dv[v] = ntt_final<true>(dv[v], t);
                     }
@@ -510,7 +516,7 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
             }
             KsiEps<V> ep;
             ksi_load_eps<FIN, V>(j, gi, ep);
-            ksi_store<FIN, LZ, V>(j, lds, idx, gi, r0, r1, ep, t);
+            ksi_store<FIN, LZ, V, PART>(j, lds, idx, gi, r0, r1, ep, t);
         }
     };
     if (FIN < KSI_FIN_TENSOR && !done) {   // (those jobs have the column sums' form)
@@ -526,11 +532,11 @@ GF_HD void ksi_body(const KsiJob& j, uint32_t N1, uint32_t tile, uint64_t* lds, 
             const NttJob& r = j.rp[c];
             if (r.twd)
                 row_tile_f64<false, S2, RM, ROWS, false, WSync, true>(r.twd, r.twrd, r.fq, r.fqinv, d, nullptr,
-                                                                      gcast(r.out), off, lds + c * KSI_PART_WORDS, lane,
+                                                                      gcast(r.out), off, lds + c * PART, lane,
                                                                       wlanes, wsync);
             else
                 row_tile<false, false, true, S2, RM, ROWS, 0, true, WSync, false, true>(
-                    r, d, nullptr, gcast(r.out), off, lds + c * KSI_PART_WORDS, lane, wlanes, wsync);
+                    r, d, nullptr, gcast(r.out), off, lds + c * PART, lane, wlanes, wsync);
         }
     }
 }

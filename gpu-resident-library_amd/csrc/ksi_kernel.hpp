@@ -23,14 +23,14 @@ struct WaveSync {
 // form spills nothing.
 // FIN: KSI_PLAIN, KSI_FIN, KSI_FIN_TENSOR(_IN); NPMAX: the largest part count with
 // column sums (4, or 6 in kernels_ksi_w.hip).
-template <uint32_t S2, uint32_t RM, int FIN, int NPMAX>
+template <uint32_t S2, uint32_t RM, int FIN, int NPMAX, uint32_t LOGT = KSI_LOG_TILE>
 __global__ __launch_bounds__(KSI_THREADS) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_ksi(const KsiJob* __restrict__ jobs, uint32_t off, uint32_t N1) {
     extern __shared__ __align__(16) uint64_t lds[];
     const KsiJob& j = jobs[off + blockIdx.y];
     const uint32_t tid = threadIdx.x, nthr = blockDim.x;
     auto go = [&](auto L) {
-        ksi_body<S2, RM, decltype(L)::value, WaveSync, DevSync, FIN, NPMAX>(j, N1, blockIdx.x, lds, tid >> 6, nthr >> 6,
-                                                                     tid & 63, 64, tid, nthr, WaveSync{}, DevSync{});
+        ksi_body<S2, RM, decltype(L)::value, WaveSync, DevSync, FIN, NPMAX, LOGT>(
+            j, N1, blockIdx.x, lds, tid >> 6, nthr >> 6, tid & 63, 64, tid, nthr, WaveSync{}, DevSync{});
     };
     if (j.red) go(std::true_type{});
     else go(std::false_type{});
@@ -38,7 +38,17 @@ __global__ __launch_bounds__(KSI_THREADS) __attribute__((amdgpu_waves_per_eu(5, 
 
 template <int NPMAX>
 inline void run_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, uint32_t fin,
-                    hipStream_t s) {
+                    bool big, hipStream_t s) {
+    if (big) {
+        const size_t shm = (size_t)regions * ksi_part_words(KSI_LOG_TILE_BIG) * 8;
+        const bool ok = with_split(g.logN1, g.logN2, [&](auto, auto B) {
+            for (uint32_t off = 0; off < nj; off += MAXY)
+                k_ksi<decltype(B)::value, 4, KSI_PLAIN, NPMAX, KSI_LOG_TILE_BIG>
+                    <<<dim3(g.n >> KSI_LOG_TILE_BIG, nj - off < MAXY ? nj - off : MAXY), 64 * waves, shm, s>>>(d, off, 1u << g.logN1);
+        });
+        if (!ok) throw std::runtime_error("gpufhe: unsupported ring dimension for the NTT");
+        return;
+    }
     // The input towers through LDS: 64 EvalMult+Rescale at n = 2^16, L = 24 6970 ->
     // 6780 us, one 196 -> 192; as a run-time branch of one kernel 6906 (spills).
     // The inputs' 16 KiB take no workgroup per CU from launches of 5 regions (4 of
@@ -66,7 +76,7 @@ inline void run_ksi(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t reg
     if (!ok) throw std::runtime_error("gpufhe: unsupported NTT radix");
 }
 // launches with jobs of 5 or 6 parts
-void launch_ksi_wide(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, uint32_t fin,
+void launch_ksi_wide(const KsiJob* d, uint32_t nj, const NttGeom& g, uint32_t regions, uint32_t waves, uint32_t fin, bool big,
                      hipStream_t s);
 
 }  // namespace gf

@@ -89,7 +89,7 @@ struct KsiArgs {
     uint64_t dpinv, post;
 };
 
-template <uint32_t RM, bool LZ, int FORM>
+template <uint32_t RM, bool LZ, int FORM, uint32_t LOGT = KSI_LOG_TILE>
 static void ksi_row(const KsiArgs& a) {
     const uint32_t n = (uint32_t)a.n;
     const uint64_t q = a.q;
@@ -183,10 +183,10 @@ static void ksi_row(const KsiArgs& a) {
             column_pass(v0.p());
             column_pass(v1.p());
         }
-        Guarded lds((size_t)ksi_regions(J) * KSI_PART_WORDS + (FORM == KSI_FIN_TENSOR_IN ? KSI_IN_WORDS : 0));
-        for (uint32_t tile = 0; tile < n / KSI_TILE; ++tile) {
+        Guarded lds((size_t)ksi_regions(J) * ksi_part_words(LOGT) + (FORM == KSI_FIN_TENSOR_IN ? KSI_IN_WORDS : 0));
+        for (uint32_t tile = 0; tile < n >> LOGT; ++tile) {
             std::fill(lds.p(), lds.p() + lds.n, ~0ull);   // a tile sees only what it wrote itself
-            ksi_body<S2, RM, LZ, NoSync, NoSync, FORM, 6>(J, 1u << S1, tile, lds.p(), 0, 1, 0, 1, 0, 1, NoSync{}, NoSync{});
+            ksi_body<S2, RM, LZ, NoSync, NoSync, FORM, 6, LOGT>(J, 1u << S1, tile, lds.p(), 0, 1, 0, 1, 0, 1, NoSync{}, NoSync{});
         }
         if (rp)
             for (int c = 0; c < 2; ++c) {
@@ -199,7 +199,14 @@ static void ksi_row(const KsiArgs& a) {
     std::memcpy(a.o1, o1.p(), n * 8);
 }
 
+// rmax 4: the stored form on 1024-element tiles
 extern "C" void emu_ksi_form(const KsiArgs* a) {
+    if (a->rmax == 4) {
+        if (a->form != KSI_PLAIN) std::abort();
+        if (lazy_red_of(a->q)) ksi_row<4, true, KSI_PLAIN, KSI_LOG_TILE_BIG>(*a);
+        else ksi_row<4, false, KSI_PLAIN, KSI_LOG_TILE_BIG>(*a);
+        return;
+    }
     with_row_radix((uint32_t)a->rmax, [&](auto Rc) {
         constexpr uint32_t RM = decltype(Rc)::value;
         auto form = [&](auto F) {

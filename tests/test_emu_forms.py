@@ -97,7 +97,7 @@ PARTS = [(1, 0b0), (1, 0b1), (2, 0b01), (3, 0b101), (4, 0b1110), (5, 0b11011), (
 def test_inner_product_forms(emu, logn, np_, xf):
     """sum_p digit_p key_p through every form of the fused step: stored; with the
     untransformed digits read through an automorphism; as the inverse transforms
-    of the dropped tower t + sum P^-1; with the last step's NTT(v) + sum ci + e
+    of the dropped tower t + sum P^-1; on tiles of 1024; with the last step's NTT(v) + sum ci + e
     (e times ce, as it is through the automorphism, or absent); and with e and
     the untransformed digit formed from two ciphertexts' rows, read or brought
     through LDS."""
@@ -145,6 +145,9 @@ def test_inner_product_forms(emu, logn, np_, xf):
             emu.emu_ksi_form(C.byref(a))
             return o
 
+        for pairs in (0, 1):   # 1024-element tiles at radix 2^4
+            o = run(KSI_PLAIN, 4, pairs, 0)
+            assert np.array_equal(o[0], sums[0][0]) and np.array_equal(o[1], sums[0][1]), (bits, pairs)
         for rmax in (2, 3):
             for f64 in (0, 1) if bits == 50 else (0,):
                 for pairs in (0, 1):

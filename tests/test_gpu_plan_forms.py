@@ -169,7 +169,36 @@ def test_stages_below_modup_min_wgs_run_apart(G, dnum, down, f64):
     check(o, P.linear_transform(L, c[0][0], c[0][1], [1] + ks, [None] + t.hk, pts), "linear")
 
 
-# knobs that differ from the defaults; radix 0: the default
+@pytest.mark.parametrize("n,L,dnum,count", [(1 << 15, 6, 3, 17), (1 << 15, 7, 7, 14), (1 << 16, 5, 5, 11)])
+def test_inner_products_on_large_tiles(G, n, L, dnum, count):
+    """With a 61-bit modulus (inner products stored, integer rows) at radix 2^4,
+    launches on both sides of the inner product's tile line: products and
+    rotations of 3, 5 and 7 parts."""
+    t = Setup(G, n, L, dnum, nkeys=1, q0bits=61)
+    t.ctx.set_ntt_radix(4)
+    c = [[t.ct(L) for _ in range(4)] for _ in range(2)]
+    d = [[G.Dev.of(x) for x in v] for v in c]
+    wm = [t.P.evalmult_rescale(L, *v, *t.hk[0]) for v in c]
+    k = pow(5, 17, 2 * n)
+    wr = [t.P.rotate(L, v[0], v[1], k, *t.hk[0]) for v in c]
+    o = [[G.Dev(L * n) for _ in range(2)] for _ in range(count)]
+    keep = [t.ctx.workspace() for _ in range(count)]
+    ws = [w.ptr for w in keep]
+    for cnt in (1, count):
+        assert (cnt * L * n // 1024 >= 3072) == (cnt > 1)   # the Q rows' workgroups
+        col = [[d[i % 2][j].ptr for i in range(cnt)] for j in range(4)]
+        out = [[x[j].ptr for x in o[:cnt]] for j in range(2)]
+        for plan, want in ((G.plan_evalmult_rescale(t.ctx, t.keys[0], [L] * cnt, *col, *out, ws[:cnt]), wm),
+                           (G.plan_rotate(t.ctx, [t.keys[0]] * cnt, [L] * cnt, [k] * cnt, col[0], col[1], *out, ws[:cnt]), wr)):
+            assert "ksi" in {x for x, _ in plan.steps()}, plan.steps()
+            plan.run(t.s)
+            t.s.sync()
+            for i in range(cnt):
+                for j in range(2):
+                    assert np.array_equal(o[i][j].download(want[i % 2][j].size), want[i % 2][j]), (cnt, i, j)
+
+
+# knobs that differ from the defaults
 LAST_STEP = [dict(), dict(ntt_radix=2), dict(ntt_radix=4), dict(ksi_fin=0), dict(ksi_tensor=0), dict(ksi_tensor=0, ntt_radix=2),
              dict(modup_f64=0), dict(modup_f64=0, ntt_radix=2), dict(ksi_f64=0, ksi_extra=1), dict(ksi_rowpass=0),
              dict(ksi_rowpass=0, ntt_radix=2, ksi_f64=0), dict(tensor_ib=0), dict(ksi_extra=1, ntt_radix=2), dict(ksi_fin=0, ksi_extra=1),
